@@ -1110,8 +1110,10 @@ int tao_prefill(const tao_state_dev* st, const tao_tokens* tok, const tao_fusion
       return fail(TAO_E_CAPACITY, "epoch range exceeds the pools or the state");
   }
   // ---- turns
+  bool turns_ascend = true;
   for (int64_t i = 0; i < n_turns; ++i) {
     const int64_t* t = plan + off_turns + 8 * i;
+    if (i && t[1] < t[1 - 8]) turns_ascend = false;
     const int64_t epoch = first_epoch + t[1];
     const int64_t eligible = t[4] * G + t[3];
     if (t[0] < 0 || t[0] >= T || t[1] < 0 || t[1] >= n_epochs ||
@@ -1141,7 +1143,8 @@ int tao_prefill(const tao_state_dev* st, const tao_tokens* tok, const tao_fusion
         // t[2] = coarse pages, t[3] = selected of the tile's epoch
         const int64_t K = epoch / G, eligible = t[2] * G + epoch % G;
         if (t[2] < 0 || t[2] > K || t[3] < 1 || t[3] > eligible ||
-            eligible > tao::kQueryRouteMaxKeys || K > tao::kQueryRouteMaxKeys || epoch > 1024 ||
+            eligible > tao::kQueryRouteMaxKeys || K > tao::kQueryRouteMaxKeys ||
+            epoch > tao::kQueryRouteMaxEpoch ||
             (epoch + 31) / 32 > pools->qsel_words)
           return fail(TAO_E_ARGUMENT, "invalid per-query read tile in the plan");
       } else if (t[2] < 0 || t[2] >= pools->sel_slots || t[3] < 1 || t[3] > 128 ||
@@ -1313,6 +1316,7 @@ int tao_prefill(const tao_state_dev* st, const tao_tokens* tok, const tao_fusion
     rp.chosen_cap = st->chosen_cap;
     rp.group = G;
     rp.max_epoch = (int)(first_epoch + n_epochs - 1);
+    rp.n_epochs = turns_ascend ? (int)n_epochs : 0;
     e = tao::launch_route(rp, D, s);
     if (e != hipSuccess) return check_hip(e, "tao_prefill routes");
   }

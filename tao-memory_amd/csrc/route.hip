@@ -563,177 +563,33 @@ __global__ __launch_bounds__(kRefreshThreads) void refresh_fold_kernel(RoutePara
 }
 
 // ---------------------------------------------------------------------------
-// Per-query routes of the full-sequence read (route_interval = 1 in
-// _read_training_group, tao_stream.py:596-665, with candidate_scores,
-// routing_scores.py:7-47): every history query of a read tile routes itself
-// against its tile's epoch with route_kernel's arithmetic and reduction
-// order (same candidates, masses and stable top-k), and its selection is
-// written as a bitmask over fine ids; the read needs the set, not the order.
-// One 256-thread workgroup per (read tile, batch, head); wave w routes
-// queries w, w + 4, ... on its own LDS arrays, so waves only synchronise
-// with themselves. This is the general path (any number of visible fines up
-// to the read's limit); route_tile_kernel below serves tiles whose rows fit
-// in LDS.
+// Routes of many queries at once: the per-query routes of the full-sequence
+// read (route_interval = 1 in _read_training_group, tao_stream.py:596-665,
+// with candidate_scores, routing_scores.py:7-47) and the turn routes of a
+// prefill. The same candidates, masses, reduction order and stable top-k as
+// route_kernel.
+//
+// What bounds them is VALU: every (query, row, channel) takes a product, its
+// bf16 rounding and an fp32 add in the fold order. So a lane owns a query and
+// keeps the rounded h * pw of one page in registers for the page's eight
+// fines, and a row's weights are the same for the whole wave: they come
+// through scalar loads and are widened on the scalar unit, which leaves 3.5
+// vector instructions per channel (a lane per (query, row) pair with both
+// rows in LDS needed about 9, and a wave per query 10 and a cross-lane fold
+// per row). Masses of every visible fine are formed, also those of pages a
+// query did not choose: the lanes of a wave choose different pages.
+// A workgroup's four waves take pages p = w, w + 4, ....
+// Measured (B1 T16384 H8 D128): 463 us with a wave per query, 103 us now, of
+// which the masses' VALU is about 56; (B2 T8192 H12 D64): 116 us with a lane
+// per (query, row) pair, 59 us now.
 constexpr int kQThreads = 256;
 constexpr int kQWaves = kQThreads / 64;
-constexpr int kQMaxWords = 512;          // bitmask words per query (16384 fines)
-
-template <int D>
-struct QueryRouteSmem {
-  float h[kQWaves][D];
-  unsigned long long keys[kQWaves][kQueryRouteMaxKeys];
-  int chosen[kQWaves][kQueryRouteMaxKeys / 8];
-  uint32_t bits[kQWaves][kQMaxWords];
-  bf16_t qrows[32][D];                  // raw_q rows of the tile's queries
-};
 
 // Orders one wave's LDS accesses across its lanes (arrays private to a wave).
 TAO_DEV void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-template <int D>
-__global__ __launch_bounds__(kQThreads) void route_queries_kernel(QueryRouteParams p) {
-  __shared__ QueryRouteSmem<D> sm;
-  const int BH = p.B * p.H;
-  const int bh = blockIdx.x % BH;
-  const int b = bh / p.H, h = bh % p.H;
-  const int64_t* desc = p.tiles + 8 * (blockIdx.x / BH);
-  if (!desc[6]) return;                          // no history: workgroup-uniform
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int q_first = (int)desc[0], nq = (int)desc[1];
-  const int coarse = (int)desc[2], M = (int)desc[3], erel = (int)desc[4];
-  constexpr int G = 8;                           // coarse_group (checked at launch)
-  const int epoch = p.first_epoch + erel;
-  const int K = epoch / G, pending = epoch % G;
-  const int E = G * coarse + pending;
-  const int words = (epoch + 31) >> 5;
-  const bf16_t* pw_g = p.pw_pool + ((size_t)erel * BH + bh) * p.pool_pcap * D;
-  const SwRows sw_g{p.sw + (size_t)bh * p.fine_cap * D,
-                    p.psw_pool + ((size_t)erel * BH + bh) * 8 * D, K * G};
-  for (int i = threadIdx.x; i < nq * (D / 8); i += kQThreads) {
-    const int r = i / (D / 8), c = i % (D / 8);
-    *(uint4*)&sm.qrows[r][c * 8] =
-        *(const uint4*)(p.rq + b * p.rq_sb + (int64_t)(q_first + r) * p.rq_st + h * p.rq_sh + c * 8);
-  }
-  __syncthreads();
-  const bf16_t* pw = pw_g;
-  const SwRows swr = sw_g;
-  float* hw = sm.h[w];
-  unsigned long long* keys = sm.keys[w];
-  int* chosen = sm.chosen[w];
-  uint32_t* bits = sm.bits[w];
-  auto cand = [&](int j, int& page, int& id) __attribute__((always_inline)) {
-    if (j < G * coarse) {
-      page = chosen[j / G];
-      id = page * G + j % G;
-    } else {
-      page = K;
-      id = K * G + (j - G * coarse);
-    }
-  };
-  for (int qi = w; qi < nq; qi += kQWaves) {
-    const int t = q_first + qi;
-    query_weights<D>(sm.qrows[qi], lane, hw);
-    for (int i = lane; i < words; i += 64) bits[i] = 0u;
-    wave_sync();
-    // ---- page masses of the completed pages, stable top-`coarse`, ascending
-    if (coarse > 0) {
-      for (int base = 0; base < K; base += kBatch) {
-        int pages[kBatch];
-        float mass[kBatch];
-        const int count = min(kBatch, K - base);
-#pragma unroll
-        for (int i = 0; i < kBatch; ++i) pages[i] = base + min(i, count - 1);
-        wave_masses<D>(hw, pw, nullptr, pages, pages, count, lane, mass);
-        if (lane < count) {
-          float mine = mass[0];
-#pragma unroll
-          for (int i = 1; i < kBatch; ++i) if (lane == i) mine = mass[i];
-          keys[base + lane] = score_key(mine, base + lane);
-        }
-      }
-      wave_sync();
-      int placed = 0;
-      for (int c0 = 0; c0 < K; c0 += 64) {
-        const int i = c0 + lane;
-        const bool pick = i < K && key_rank(keys, K, keys[i]) < coarse;
-        const unsigned long long ball = __ballot(pick);
-        if (pick) chosen[placed + __popcll(ball & ((1ull << lane) - 1ull))] = i;
-        placed += __popcll(ball);
-      }
-      wave_sync();
-    }
-    // ---- candidate masses: 8 fines of each chosen page, then the pending fines
-    for (int base = 0; base < E; base += kBatch) {
-      int pages[kBatch], ids[kBatch];
-      float mass[kBatch];
-      const int count = min(kBatch, E - base);
-#pragma unroll
-      for (int i = 0; i < kBatch; ++i) cand(base + min(i, count - 1), pages[i], ids[i]);
-      wave_masses<D>(hw, pw, &swr, pages, ids, count, lane, mass);
-      if (lane < count) {
-        float mine = mass[0];
-#pragma unroll
-        for (int i = 1; i < kBatch; ++i) if (lane == i) mine = mass[i];
-        keys[base + lane] = score_key(mine, base + lane);
-      }
-    }
-    wave_sync();
-    // ---- stable top-M candidates -> bitmask
-    for (int j = lane; j < E; j += 64)
-      if (key_rank(keys, E, keys[j]) < M) {
-        int page, id;
-        cand(j, page, id);
-        atomicOr(&bits[id >> 5], 1u << (id & 31));
-      }
-    wave_sync();
-    uint32_t* dst = p.qsel + ((size_t)(b * p.T + t) * p.H + h) * p.qsel_words;
-    for (int i = lane; i < words; i += 64) dst[i] = bits[i];
-    wave_sync();                                 // h, keys and bits are reused
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Per-query routes, lane per (query, row) pair: the same arithmetic as
-// route_queries_kernel with the channel sum of one mass done by one lane in
-// registers, in the fold order (pairs (e, e + 64) for D = 128, then
-// (e, e + 32), (e, e + 16), ..., (e, e + 1)), so no cross-lane reduction is
-// needed. One 256-thread workgroup per (read tile of <= 32 queries, batch,
-// head); the tile's h rows, page-weight rows and the segment-weight rows of
-// its visible fines sit in LDS, and the (query, page) and (query, candidate)
-// pairs are spread over all lanes. Keys are 32-bit: monotone bf16 score in
-// the high half, 0xFFFF - index in the low half (same order as score_key).
-constexpr int kTileQ = 32;
-
-template <int D, int ROWS_ = (D == 64 ? 128 : 64)>
-struct RouteTileGeo {
-  static constexpr int PAD = D + 8;                  // padded LDS row (bf16)
-  static constexpr int ROWS = ROWS_;                 // staged pw + sw rows
-  static constexpr int KEYS = ROWS;                  // >= pages, >= candidates
-  static constexpr int WORDS = ROWS / 32;
-};
-// Staged rows of the turn-route kernel (prefill turns reach further epochs).
-template <int D>
-constexpr int kTurnRows = D == 64 ? 256 : 160;
-
-template <int D, int ROWS_ = (D == 64 ? 128 : 64)>
-struct RouteTileSmem {
-  using G = RouteTileGeo<D, ROWS_>;
-  bf16_t h[kTileQ][G::PAD];
-  bf16_t rows[G::ROWS][G::PAD];
-  uint32_t keys[kTileQ][G::KEYS];
-  uint8_t chosen[kTileQ][G::KEYS / 8];
-  uint32_t bits[kTileQ][G::WORDS];
-  float hf[4][D];                                    // one query's h per wave (fp32)
-};
-
-TAO_DEV uint32_t score_key32(float score_bf, int index) {
-  bf16_t bits = f2bf(score_bf);
-  if (bits == 0x8000) bits = 0;                      // -0 ties with +0, as in torch's sort
-  return (bf16_order_key(bits) << 16) | (uint32_t)(0xFFFF - index);
 }
 
 TAO_DEV void unpack8(const uint4& u, float out[8]) {
@@ -745,218 +601,555 @@ TAO_DEV void unpack8(const uint4& u, float out[8]) {
   }
 }
 
-// r(fold_e r(r(h[e] * pw[e]) * sw[e])) (WITH_SW) or r(fold_e r(h[e] * pw[e])).
-template <int D, bool WITH_SW>
-TAO_DEV float lane_mass(const bf16_t* hrow, const bf16_t* pwrow, const bf16_t* swrow) {
-  float s1[32];
+// Wave-uniform read-only rows: the constant address space makes the loads
+// scalar.
+typedef const __attribute__((address_space(4))) uint32_t* const_words;
+TAO_DEV const_words uniform_row(const bf16_t* p) { return (const_words)(uint64_t)p; }
+TAO_DEV float word_bf(uint32_t w, int k) {
+  return __uint_as_float(k ? (w & 0xFFFF0000u) : (w << 16));
+}
+
+// Sum over D channels in the fold order, the channels' values made as the
+// tree reaches them: T(e, n) = T(e, 2n) + T(e + n, 2n), and pair(e) =
+// y_e + y_(e + D/2) is a leaf.
+template <int D, int E, int N, class Pair>
+TAO_DEV float fold_tree(const Pair& pair) {
+  if constexpr (N == D / 2) {
+    return pair(E);
+  } else {
+    const float lo = fold_tree<D, E, 2 * N>(pair);
+    const float hi = fold_tree<D, E + N, 2 * N>(pair);
+    // Subtrees of 16 channels in turn: together they would not fit the registers.
+    if constexpr (N == D / 16) __builtin_amdgcn_sched_barrier(0);
+    return lo + hi;
+  }
+}
+
+// 16-bit order key of a mass, never 0 (0 marks a fine that is no candidate).
+TAO_DEV uint16_t mass_key(float mass) {
+  bf16_t bits = f2bf(mass);
+  if (bits == 0x8000) bits = 0;                      // -0 ties with +0, as in torch's sort
+  const uint32_t key = bf16_order_key(bits);
+  return (uint16_t)(key ? key : 1u);
+}
+
+// Page and fine keys of one query per lane, pages w, w + 4, ... of the wave.
+template <int D>
+TAO_DEV void lane_masses(const bf16_t* hrow, int w, bool write, bool pages, int K, int epoch,
+                         const bf16_t* pw, const SwRows& sw, uint16_t* pkey, uint16_t* fkey) {
+  constexpr int G = 8, HALF = D / 2;
+  const int P = (epoch + G - 1) / G;
+  for (int p = w; p < P; p += kQWaves) {
+    const const_words pwr = uniform_row(pw + (size_t)p * D);
+    float x[D];
 #pragma unroll
-  for (int c = 0; c < 4; ++c) {            // s1[8c + k], k < 8
-    float part[D / 32][8];
-#pragma unroll
-    for (int b = 0; b < D / 32; ++b) {     // channels 8c + k + 32 b
-      const int e0 = 8 * c + 32 * b;
-      float hv[8], pv[8];
-      unpack8(*(const uint4*)(hrow + e0), hv);
-      unpack8(*(const uint4*)(pwrow + e0), pv);
-      float sv[8];
-      if constexpr (WITH_SW) unpack8(*(const uint4*)(swrow + e0), sv);
+    for (int c = 0; c < HALF; c += 8) {
+      float lo[8], hi[8];
+      unpack8(*(const uint4*)(hrow + c), lo);
+      unpack8(*(const uint4*)(hrow + HALF + c), hi);
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        const float x = rbf(hv[k] * pv[k]);
-        part[b][k] = WITH_SW ? rbf(x * sv[k]) : x;
+        const uint32_t u = pack_bf16x2(lo[k] * word_bf(pwr[(c + k) / 2], k & 1),
+                                       hi[k] * word_bf(pwr[(HALF + c + k) / 2], k & 1));
+        x[c + k] = word_bf(u, 0);
+        x[HALF + c + k] = word_bf(u, 1);
       }
     }
-#pragma unroll
-    for (int k = 0; k < 8; ++k) {
-      if constexpr (D == 64)
-        s1[8 * c + k] = part[0][k] + part[1][k];
-      else
-        s1[8 * c + k] = (part[0][k] + part[2][k]) + (part[1][k] + part[3][k]);
+    if (pages && p < K) {
+      const float m = fold_tree<D, 0, 1>([&](int e) __attribute__((always_inline)) {
+        return x[e] + x[e + HALF];
+      });
+      if (write) pkey[p] = mass_key(rbf(m));
+    }
+    const int n = min(G, epoch - G * p);
+    for (int j = 0; j < n; ++j) {
+      const const_words s = uniform_row(sw.row(G * p + j, D));
+      const float m = fold_tree<D, 0, 1>([&](int e) __attribute__((always_inline)) {
+        const uint32_t u = pack_bf16x2(x[e] * word_bf(s[e / 2], e & 1),
+                                       x[e + HALF] * word_bf(s[(e + HALF) / 2], e & 1));
+        return word_bf(u, 0) + word_bf(u, 1);
+      });
+      if (write) fkey[G * p + j] = mass_key(rbf(m));
     }
   }
-#pragma unroll
-  for (int w = 16; w >= 1; w >>= 1)
-#pragma unroll
-    for (int i = 0; i < w; ++i) s1[i] += s1[i + w];
-  return rbf(s1[0]);
 }
 
-// Lane-per-pair routing of nq queries whose h rows (sm.h) and page-weight /
-// segment-weight rows (sm.rows: P page rows, then one row per fine id) are
-// staged: coarse pages by page mass (stable top-`coarse`, then ascending, in
-// sm.chosen), candidate masses, stable top-M; emit(q, rank, id) for every
-// selected candidate (rank = position in score order). All threads call it.
-template <int D, class SM, class Emit>
-TAO_DEV void route_core(SM& sm, int nq, int K, int coarse, int E, int M, int P, int tid,
-                        Emit emit) {
-  constexpr int G = 8;
-  // ---- coarse pages: stable top-`coarse` by page mass, listed ascending
-  if (coarse >= K) {
-    for (int i = tid; i < nq * K; i += kQThreads) sm.chosen[i / K][i % K] = (uint8_t)(i % K);
-  } else {
-    for (int i = tid; i < nq * K; i += kQThreads) {
-      const int q = i / K, pg = i % K;
-      const float m = lane_mass<D, false>(sm.h[q], sm.rows[pg], nullptr);
-      sm.keys[q][pg] = score_key32(m, pg);
-    }
-    __syncthreads();
-    // chosen flag in the low byte of the key slot's spare: rank < coarse
-    for (int i = tid; i < nq * K; i += kQThreads) {
-      const int q = i / K, pg = i % K;
-      const uint32_t mine = sm.keys[q][pg];
-      int rank = 0;
-      for (int j = 0; j < K; ++j) rank += sm.keys[q][j] > mine;
-      if (rank < coarse) {
-        // ascending position = chosen pages with a smaller index
-        int pos = 0;
-        for (int j = 0; j < pg; ++j) {
-          const uint32_t other = sm.keys[q][j];
-          int r2 = 0;
-          for (int l = 0; l < K; ++l) r2 += sm.keys[q][l] > other;
-          pos += r2 < coarse;
-        }
-        sm.chosen[q][pos] = (uint8_t)pg;
-      }
-    }
-  }
-  __syncthreads();
-  // ---- candidate masses: 8 fines of each chosen page, then the pending fines
-  auto cand = [&](int q, int j, int& page, int& id) __attribute__((always_inline)) {
-    if (j < G * coarse) {
-      page = sm.chosen[q][j / G];
-      id = page * G + j % G;
-    } else {
-      page = K;
-      id = K * G + (j - G * coarse);
+// N masses of one query and one page per lane, in the lane's own rows:
+// r(fold(r(r(h * pw) * sw_i))), or with PAGE r(fold(r(h * pw))). h * pw is
+// rounded once for the N fines. The fold as eight partial sums of the
+// channels 8c + k: chunks c and c + 2, then c and c + 1, then k by halves.
+template <int D, int N, bool PAGE>
+TAO_DEV void item_masses(const bf16_t* hrow, const bf16_t* pwrow, const bf16_t* const (&sw)[N],
+                         float (&mass)[N]) {
+  // Step n takes the channel blocks e and e + D / 2 of chunk c (D = 128: of
+  // e = 8 c, then of 8 c + 32); the next step's rows are in flight meanwhile.
+  constexpr int STEPS = D / 16;
+  uint4 pr[2][2], sr[2][N][2];
+  auto first = [](int n) __attribute__((always_inline)) {
+    const int c = D == 128 ? n / 2 : n;            // chunks 0, 2, 1, 3
+    return 8 * ((c & 1) * 2 + (c >> 1)) + (D == 128 ? 32 * (n & 1) : 0);
+  };
+  auto fetch = [&](int n) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int e0 = first(n) + (D / 2) * b;
+      pr[n & 1][b] = *(const uint4*)(pwrow + e0);
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        if constexpr (!PAGE) sr[n & 1][i][b] = *(const uint4*)(sw[i] + e0);
     }
   };
-  for (int i = tid; i < nq * E; i += kQThreads) {
-    const int q = i / E, j = i % E;
-    int page, id;
-    cand(q, j, page, id);
-    const float m = lane_mass<D, true>(sm.h[q], sm.rows[page], sm.rows[P + id]);
-    sm.keys[q][j] = score_key32(m, j);
-  }
-  __syncthreads();
-  // ---- stable top-M per query -> bitmask
-  for (int i = tid; i < nq * E; i += kQThreads) {
-    const int q = i / E, j = i % E;
-    const uint32_t mine = sm.keys[q][j];
-    int rank = 0;
-    for (int l = 0; l < E; ++l) rank += sm.keys[q][l] > mine;
-    if (rank < M) {
-      int page, id;
-      cand(q, j, page, id);
-      emit(q, rank, id);
+  float a[N][8], s[N][8], u[N][8];
+  fetch(0);
+#pragma unroll
+  for (int n = 0; n < STEPS; ++n) {
+    if (n + 1 < STEPS) fetch(n + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    float t[N][8];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      float hv[8], pv[8];
+      unpack8(*(const uint4*)(hrow + first(n) + (D / 2) * b), hv);
+      unpack8(pr[n & 1][b], pv);
+      uint32_t x[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        x[k] = pack_bf16x2(hv[2 * k] * pv[2 * k], hv[2 * k + 1] * pv[2 * k + 1]);
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        float sv[8];
+        if constexpr (!PAGE) unpack8(sr[n & 1][i][b], sv);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          float y = word_bf(x[k / 2], k & 1);
+          if constexpr (!PAGE) y *= sv[k];
+          if (b == 0) {
+            t[i][k] = y;
+          } else if constexpr (PAGE) {
+            t[i][k] += y;
+          } else {
+            const uint32_t r = pack_bf16x2(t[i][k], y);
+            t[i][k] = word_bf(r, 0) + word_bf(r, 1);
+          }
+        }
+      }
     }
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        // Pinned: the compiler sinks the sums below every load otherwise.
+        asm volatile("" : "+v"(t[i][k]));
+        if (D == 128 && (n & 1) == 0) { u[i][k] = t[i][k]; continue; }
+        const float v = D == 128 ? u[i][k] + t[i][k] : t[i][k];
+        const int step = D == 128 ? n / 2 : n;
+        if (step == 0) a[i][k] = v;
+        if (step == 1) a[i][k] += v;
+        if (step == 2) s[i][k] = v;
+        if (step == 3) a[i][k] += s[i][k] + v;
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    mass[i] = rbf(((a[i][0] + a[i][4]) + (a[i][2] + a[i][6])) +
+                  ((a[i][1] + a[i][5]) + (a[i][3] + a[i][7])));
+}
+
+// h = r(softmax_D(raw_q)) of n <= 4 queries by one wave, as query_weights:
+// sixteen lanes a query, lane i of them holding the channels i + 16 k, so the
+// fold's first levels are in the lane and the last four are row rotations.
+// row(q): raw_q row; dst(q): the row to store (bf16).
+template <int CTRL>
+TAO_DEV float row_ror(float v) { return dpp_partner<0x120 + CTRL>(v); }
+
+template <int D, class Row, class Dst>
+TAO_DEV void query_rows(int n, int lane, const Row& row, const Dst& dst) {
+  constexpr int PER = D / 16;
+  const int q = lane >> 4, i = lane & 15;
+  const bf16_t* r = row(min(q, n - 1));
+  float x[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) x[k] = bf2f(r[i + 16 * k]);
+  float mx = x[0];
+#pragma unroll
+  for (int k = 1; k < PER; ++k) mx = fmaxf(mx, x[k]);
+  mx = fmaxf(mx, row_ror<8>(mx));
+  mx = fmaxf(mx, row_ror<4>(mx));
+  mx = fmaxf(mx, row_ror<2>(mx));
+  mx = fmaxf(mx, row_ror<1>(mx));
+  float s[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) s[k] = x[k] = exp_cr(x[k] - mx);
+#pragma unroll
+  for (int w = PER / 2; w >= 1; w >>= 1)
+#pragma unroll
+    for (int k = 0; k < w; ++k) s[k] += s[k + w];
+  float t = s[0];
+  t += row_ror<8>(t);
+  t += row_ror<4>(t);
+  t += row_ror<2>(t);
+  t += row_ror<1>(t);
+  // x / t rounded to bf16: the product with the reciprocal is within 2 ulps
+  // of the quotient, which alone decides near a bf16 rounding boundary.
+  const float inv = 1.0f / t;
+  bool near = false;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    s[k] = x[k] * inv;
+    near |= near_bf16_midpoint(s[k], 4);
+  }
+  if (near) {
+#pragma unroll
+    for (int k = 0; k < PER; ++k) s[k] = x[k] / t;
+  }
+  if (q < n) {
+    bf16_t* d = dst(q);
+#pragma unroll
+    for (int k = 0; k < PER; ++k) d[i + 16 * k] = f2bf(s[k]);
   }
 }
 
+TAO_DEV int quad_sum(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xF, 0xF, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xF, 0xF, false);
+  return v;
+}
+TAO_DEV uint32_t quad_max(uint32_t v) {
+  v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false));
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false));
+}
+
+// A quad's share of the keys: up to N in registers, or in LDS (N = 0).
+template <int N>
+struct QuadKeys {
+  uint32_t k[N];
+  TAO_DEV QuadKeys(const uint16_t* keys, int lo, int hi) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) k[i] = lo + i < hi ? keys[lo + i] : 0u;
+  }
+  template <class F> TAO_DEV void each(const F& f) const {
+#pragma unroll
+    for (int i = 0; i < N; ++i) f(k[i], i);
+  }
+};
+template <>
+struct QuadKeys<0> {
+  const uint16_t* p; int n;
+  TAO_DEV QuadKeys(const uint16_t* keys, int lo, int hi) : p(keys + lo), n(hi - lo) {}
+  template <class F> TAO_DEV void each(const F& f) const {
+    for (int i = 0; i < n; ++i) f((uint32_t)p[i], i);
+  }
+};
+
+template <int N, class Emit>
+TAO_DEV void quad_select_n(const uint16_t* keys, int n, int m, int lane, const Emit& emit) {
+  const int len = (n + 3) >> 2;
+  const int lo = min(n, (lane & 3) * len), hi = min(n, lo + len);
+  const QuadKeys<N> own(keys, lo, hi);
+  // The bits that the largest and the smallest candidate share are the
+  // threshold's too.
+  uint32_t top = 0, low = 0;                    // low: largest of 0xFFFF - key
+  own.each([&](uint32_t k, int) __attribute__((always_inline)) {
+    top = max(top, k);
+    low = max(low, k ? 0xFFFFu - k : 0u);
+  });
+  top = quad_max(top);
+  low = 0xFFFFu - quad_max(low);
+  const uint32_t differ = top ^ low;
+  int bit = differ ? 31 - __clz((int)differ) : -1;
+  uint32_t t = bit < 0 ? top : top & ~((2u << bit) - 1u);
+  for (; bit >= 0; --bit) {
+    const uint32_t c = t | (1u << bit);
+    int count = 0;
+    own.each([&](uint32_t k, int) __attribute__((always_inline)) { count += k >= c; });
+    if (quad_sum(count) >= m) t = c;
+  }
+  int above = 0, ties = 0;
+  own.each([&](uint32_t k, int) __attribute__((always_inline)) {
+    above += k > t;
+    ties += k == t;
+  });
+  int left = m - quad_sum(above);
+  for (int i = 0; i < 3; ++i) {
+    const int other = __shfl(ties, (lane & ~3) + i, 64);
+    if (i < (lane & 3)) left -= other;
+  }
+  own.each([&](uint32_t k, int i) __attribute__((always_inline)) {
+    if (k > t || (k == t && k && left-- > 0)) emit(lo + i);
+  });
+}
+
+// The top m of keys[0, n) by (key descending, index ascending), 1 <= m <= the
+// number of non-zero keys (the candidates): four lanes (a quad, sub = lane &
+// 3) share the query and own a quarter of the indices each. The m-th largest
+// key comes bit by bit from counts; ties at it are taken in index order.
+// emit(index) runs in the owning lane, indices ascending over the quad.
+template <class Emit>
+TAO_DEV void quad_select(const uint16_t* keys, int n, int m, int lane, const Emit& emit) {
+  if (n <= 32)
+    quad_select_n<8>(keys, n, m, lane, emit);
+  else if (n <= 64)
+    quad_select_n<16>(keys, n, m, lane, emit);
+  else
+    quad_select_n<0>(keys, n, m, lane, emit);
+}
+
+// LDS of a per-query routing workgroup: h rows, fine keys and page keys of its
+// query slots. A key row holds an odd number of words, so a column of them
+// over the lanes spreads over the banks. Once the masses are formed the open
+// pages (a bit each) and the selection lie where the h rows were.
+struct RouteLds {
+  int slots, fkeys, pkeys;           // slots; 16-bit keys of a row
+  __host__ __device__ size_t bytes(int D) const {
+    return (size_t)slots * (2 * (D + 8) + 2 * fkeys + 2 * pkeys);
+  }
+};
+static RouteLds route_lds(int slots, int max_epoch) {
+  auto odd = [](int keys) { return 2 * (((keys + 1) / 2) | 1); };
+  return RouteLds{slots, odd(max_epoch), odd(max_epoch / 8 + 1)};
+}
+constexpr size_t kLdsBytes = 160 * 1024;
+
+// Opens the pages a query reads (open: one bit a page, zeroed) and clears the
+// keys of the other pages' fines; four lanes a query.
+TAO_DEV void quad_open_pages(const uint16_t* pkey, uint16_t* fkey, uint32_t* open, int K,
+                             int coarse, int lane) {
+  if (coarse < K) {
+    if (coarse > 0)
+      quad_select(pkey, K, coarse, lane,
+                  [&](int pg) __attribute__((always_inline)) { atomicOr(&open[pg >> 5], 1u << (pg & 31)); });
+    wave_sync();
+    for (int f = lane & 3; f < 8 * K; f += 4)
+      if (!(open[f >> 8] >> ((f >> 3) & 31) & 1u)) fkey[f] = 0;
+  } else {
+    for (int pg = lane & 3; pg < K; pg += 4) atomicOr(&open[pg >> 5], 1u << (pg & 31));
+  }
+  wave_sync();
+}
+
+// Per-query routes: a workgroup takes the queries of slots / 32 consecutive
+// read tiles of one (batch, head). Selections are bitmasks over fine ids (the
+// read needs the set, not the order).
 template <int D>
-__global__ __launch_bounds__(kQThreads) void route_tile_kernel(QueryRouteParams p) {
-  using Geo = RouteTileGeo<D>;
-  __shared__ RouteTileSmem<D> sm;
-  constexpr int G = 8;                           // coarse_group (checked at launch)
+__global__ __launch_bounds__(kQThreads, 2) void route_queries_kernel(QueryRouteParams p,
+                                                                     RouteLds lds) {
+  extern __shared__ __align__(16) unsigned char route_smem[];
+  constexpr int G = 8, PAD = D + 8;                // coarse_group (checked at launch)
+  bf16_t* const hs = (bf16_t*)route_smem;
+  uint16_t* const fkeys = (uint16_t*)(hs + lds.slots * PAD);
+  uint16_t* const pkeys = fkeys + lds.slots * lds.fkeys;
   const int BH = p.B * p.H;
   const int bh = blockIdx.x % BH;
   const int b = bh / p.H, h = bh % p.H;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // Tiles in reverse order: the latest tiles score the most keys.
-  const int64_t* desc = p.tiles + 8 * ((int)gridDim.x / BH - 1 - (int)blockIdx.x / BH);
-  if (!desc[6]) return;                          // no history: workgroup-uniform
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int q_first = (int)desc[0], nq = (int)desc[1];
-  const int coarse = (int)desc[2], M = (int)desc[3], erel = (int)desc[4];
-  const int epoch = p.first_epoch + erel;
-  const int K = epoch / G, pending = epoch % G;
-  const int E = G * coarse + pending;
-  const int P = K + (pending > 0);
-  const int words = (epoch + 31) >> 5;
-  const bf16_t* pw_g = p.pw_pool + ((size_t)erel * BH + bh) * p.pool_pcap * D;
-  const SwRows sw_g{p.sw + (size_t)bh * p.fine_cap * D,
-                    p.psw_pool + ((size_t)erel * BH + bh) * 8 * D, K * G};
-  // ---- stage: rows [0, P) page weights, [P, P + epoch) segment weights
-  for (int i = tid; i < (P + epoch) * (D / 8); i += kQThreads) {
-    const int r = i / (D / 8), c = i % (D / 8);
-    const bf16_t* src = r < P ? pw_g + (size_t)r * D : sw_g.row(r - P, D);
-    *(uint4*)&sm.rows[r][c * 8] = *(const uint4*)(src + c * 8);
-  }
-  for (int i = tid; i < kTileQ * Geo::WORDS; i += kQThreads) (&sm.bits[0][0])[i] = 0u;
-  // ---- h of each query: wave w does queries w, w + 4, ...
-  for (int qi = w; qi < nq; qi += 4) {
-    query_weights<D>(p.rq + b * p.rq_sb + (int64_t)(q_first + qi) * p.rq_st + h * p.rq_sh,
-                     lane, sm.hf[w]);
-    wave_sync();
-    for (int e = lane; e < D; e += 64) sm.h[qi][e] = f2bf(sm.hf[w][e]);
-    wave_sync();
-  }
-  __syncthreads();
-  route_core<D>(sm, nq, K, coarse, E, M, P, tid,
-                [&](int q, int rank, int id) { atomicOr(&sm.bits[q][id >> 5], 1u << (id & 31)); });
-  __syncthreads();
-  for (int i = tid; i < nq * words; i += kQThreads) {
-    const int q = i / words, wd = i % words;
-    p.qsel[((size_t)(b * p.T + q_first + q) * p.H + h) * p.qsel_words + wd] = sm.bits[q][wd];
-  }
-}
-
-// Turn routes of a prefill (route_kernel's turn mode) with the lane-per-pair
-// core: one 256-thread workgroup per (16 consecutive turns, batch, head).
-// The turns are split into runs that share a seal epoch (a run holds at most
-// the turns of one epoch, within the tile's 32 queries); each run stages its
-// epoch's rows once and routes its anchors together. Outputs as route_kernel: ids in score order into the turn's
-// sel_pool slot; the publishing turn also writes the state's route, chosen
-// pages and route size.
-constexpr int kTurnGroup = 16;
-
-template <int D>
-__global__ __launch_bounds__(kQThreads) void route_turns_kernel(RouteParams p) {
-  constexpr int ROWS = kTurnRows<D>;
-  __shared__ RouteTileSmem<D, ROWS> sm;
-  constexpr int G = 8;
-  const int BH = p.B * p.H;
-  const int bh = blockIdx.x % BH;
-  const int b = bh / p.H, h = bh % p.H;
-  // Turn groups in reverse order: the latest turns score the most rows.
-  const int t0 = ((p.n_turns + kTurnGroup - 1) / kTurnGroup - 1 - (int)blockIdx.x / BH) * kTurnGroup;
-  const int t1 = min(p.n_turns, t0 + kTurnGroup);
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  for (int s0 = t0; s0 < t1;) {
-    const int64_t* d0 = p.turns + 8 * s0;
-    int s1 = s0 + 1;
-    while (s1 < t1 && p.turns[8 * s1 + 1] == d0[1]) ++s1;
-    const int erel = (int)d0[1], K = (int)d0[2], pending = (int)d0[3];
-    const int coarse = (int)d0[4], M = (int)d0[5];
-    const int epoch = K * G + pending, P = K + (pending > 0), E = G * coarse + pending;
-    const int nq = s1 - s0;
-    const bf16_t* pw_g = p.pw_pool + ((size_t)erel * BH + bh) * p.pool_pcap * D;
-    const SwRows sw_g{p.sw + (size_t)bh * p.fine_cap * D,
-                      p.psw_pool + ((size_t)erel * BH + bh) * 8 * D, K * G};
-    __syncthreads();                               // the previous run is done with sm
-    for (int i = tid; i < (P + epoch) * (D / 8); i += kQThreads) {
-      const int r = i / (D / 8), c = i % (D / 8);
-      const bf16_t* src = r < P ? pw_g + (size_t)r * D : sw_g.row(r - P, D);
-      *(uint4*)&sm.rows[r][c * 8] = *(const uint4*)(src + c * 8);
+  const int per = lds.slots / 32;
+  const int t0 = ((int)gridDim.x / BH - 1 - (int)blockIdx.x / BH) * per;
+  const int64_t* desc = p.tiles + 8 * (size_t)t0;
+  const int tiles = min(per, p.n_tiles - t0);
+  for (int a = 0; a < tiles;) {
+    const int64_t* d0 = desc + 8 * a;
+    int z = a + 1;                                 // tiles [a, z) share their route's shape
+    while (z < tiles && desc[8 * z + 2] == d0[2] && desc[8 * z + 3] == d0[3] &&
+           desc[8 * z + 4] == d0[4] && desc[8 * z + 6] == d0[6])
+      ++z;
+    if (!d0[6]) {                                  // no history: workgroup-uniform
+      a = z;
+      continue;
     }
-    for (int qi = w; qi < nq; qi += 4) {
-      const int64_t anchor = p.turns[8 * (s0 + qi)];
-      query_weights<D>(p.rq + b * p.rq_sb + anchor * p.rq_st + h * p.rq_sh, lane, sm.hf[w]);
-      wave_sync();
-      for (int e = lane; e < D; e += 64) sm.h[qi][e] = f2bf(sm.hf[w][e]);
-      wave_sync();
+    const int coarse = (int)d0[2], M = (int)d0[3], erel = (int)d0[4];
+    const int epoch = p.first_epoch + erel, K = epoch / G;
+    const int words = (epoch + 31) >> 5;
+    const bf16_t* pw = p.pw_pool + ((size_t)erel * BH + bh) * p.pool_pcap * D;
+    const SwRows sw{p.sw + (size_t)bh * p.fine_cap * D,
+                    p.psw_pool + ((size_t)erel * BH + bh) * 8 * D, K * G};
+    // ---- h of each query
+    for (int tl = a; tl < z; ++tl) {
+      const int first = (int)desc[8 * tl], nq = (int)desc[8 * tl + 1];
+      for (int q0 = 4 * w; q0 < nq; q0 += 4 * kQWaves)
+        query_rows<D>(
+            min(4, nq - q0), lane,
+            [&](int i) __attribute__((always_inline)) {
+              return p.rq + b * p.rq_sb + (int64_t)(first + q0 + i) * p.rq_st + h * p.rq_sh;
+            },
+            [&](int i) __attribute__((always_inline)) { return hs + (32 * tl + q0 + i) * PAD; });
     }
     __syncthreads();
-    route_core<D>(sm, nq, K, coarse, E, M, P, tid, [&](int q, int rank, int id) {
-      const int64_t* dq = p.turns + 8 * (s0 + q);
-      p.sel_pool[((size_t)dq[6] * BH + bh) * p.sel_cap + rank] = id;
-      if (dq[7]) p.sel[(size_t)bh * p.sel_cap + rank] = id;
-    });
-    for (int q = 0; q < nq; ++q) {
-      if (!p.turns[8 * (s0 + q) + 7]) continue;   // workgroup-uniform
-      for (int i = tid; i < coarse; i += kQThreads)
-        p.chosen[(size_t)bh * p.chosen_cap + i] = sm.chosen[q][i];
-      if (bh == 0 && tid == 0) p.header[1] = M;
+    // ---- masses: lane = query slot (slots of no query compute and drop)
+    {
+      const int slot = lane & (lds.slots - 1);
+      const bool write = lane >= 32 * a && lane < 32 * z;
+      lane_masses<D>(hs + slot * PAD, w, write, coarse < K, K, epoch, pw, sw,
+                     pkeys + slot * lds.pkeys, fkeys + slot * lds.fkeys);
     }
-    s0 = s1;
+    __syncthreads();
+    // ---- selection: four lanes a query; open pages and bitmasks where h was
+    uint32_t* const bits = (uint32_t*)hs;                    // [slot][words]
+    uint32_t* const opens = bits + lds.slots * words;        // [slot][4]
+    for (int i = threadIdx.x; i < lds.slots * (words + 4); i += kQThreads) bits[i] = 0u;
+    __syncthreads();
+    const int slot = 16 * w + (lane >> 2), tl = slot >> 5;
+    if (tl >= a && tl < z && (slot & 31) < (int)desc[8 * tl + 1]) {
+      uint16_t* fkey = fkeys + slot * lds.fkeys;
+      quad_open_pages(pkeys + slot * lds.pkeys, fkey, opens + 4 * slot, K, coarse, lane);
+      quad_select(fkey, epoch, M, lane, [&](int id) __attribute__((always_inline)) {
+        atomicOr(&bits[slot * words + (id >> 5)], 1u << (id & 31));
+      });
+    }
+    __syncthreads();
+    for (int i = threadIdx.x + 32 * a * words; i < 32 * z * words; i += kQThreads) {
+      const int s = i / words, wd = i - s * words;
+      const int64_t* d = desc + 8 * (s >> 5);
+      if ((s & 31) < (int)d[1])
+        p.qsel[((size_t)(b * p.T + (int)d[0] + (s & 31)) * p.H + h) * p.qsel_words + wd] = bits[i];
+    }
+    __syncthreads();                               // h rows and keys are reused
+    a = z;
+  }
+}
+
+// Turn routes of a prefill (route_kernel's turn mode): one workgroup per
+// (seal epoch, batch, head), sixteen of the epoch's turns at a time. A period
+// of 24 tokens gives an epoch at most 11, too few for a lane per query: the
+// lanes take (turn, page) items for the page masses, then (turn, chosen page,
+// pair of its fines) items, so only candidates are scored and no lane waits
+// for a turn that is not there. Outputs as route_kernel: ids in score order
+// into the turn's sel_pool slot; the publishing turn also writes the state's
+// route, chosen pages and route size. Measured at a 16K prompt (H32 D128):
+// 87 us with a lane per (turn, row) pair in groups of sixteen turns over two
+// or three epochs, 57 us now; one 16K call at 128K (rows beyond that form's
+// LDS, a workgroup per turn): 350 -> 150 us.
+constexpr int kTurnSlots = 16;
+constexpr int kTurnMaxEpoch = 2048;
+
+TAO_DEV uint32_t score_key32(float score_bf, int index) {
+  bf16_t bits = f2bf(score_bf);
+  if (bits == 0x8000) bits = 0;                      // -0 ties with +0, as in torch's sort
+  return (bf16_order_key(bits) << 16) | (uint32_t)(0xFFFF - index);
+}
+
+template <int D>
+__global__ __launch_bounds__(kQThreads, 2) void route_turns_kernel(RouteParams p, int cap) {
+  extern __shared__ __align__(16) unsigned char route_smem[];
+  constexpr int G = 8, PAD = D + 8;
+  bf16_t* const hs = (bf16_t*)route_smem;                      // [slot][PAD]
+  uint32_t* const keys = (uint32_t*)(hs + kTurnSlots * PAD);   // [slot][cap]
+  uint8_t* const chosen = (uint8_t*)(keys + kTurnSlots * cap); // [slot][cap]
+  __shared__ uint32_t opens[kTurnSlots][kTurnMaxEpoch / 8 / 32];
+  const int BH = p.B * p.H;
+  const int bh = blockIdx.x % BH;
+  const int b = bh / p.H, h = bh % p.H;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // Epochs in reverse order: the latest turns score the most rows.
+  const int erel = p.n_epochs - 1 - (int)blockIdx.x / BH;
+  // First turn of the epoch (turns ascend by epoch), 64 ways at a time: the
+  // groups of `step` turns whose last turn is below the epoch are skipped.
+  int s0 = 0, span = p.n_turns;
+  while (span > 0) {
+    const int step = (span + 63) / 64;
+    const int at = s0 + min((lane + 1) * step, span) - 1;
+    const int below = __popcll(__ballot(p.turns[8 * (size_t)at + 1] < erel));
+    const int skip = min(below * step, span);
+    s0 += skip;
+    span = min(step, span - skip);
+    if (step == 1) break;
+  }
+  s0 = __builtin_amdgcn_readfirstlane(s0);
+  while (s0 < p.n_turns && p.turns[8 * (size_t)s0 + 1] == erel) {
+    const int64_t* d0 = p.turns + 8 * (size_t)s0;
+    const int64_t* dl = d0 + 8 * min(lane, min(kTurnSlots, p.n_turns - s0) - 1);
+    const uint64_t same = __ballot(lane < min(kTurnSlots, p.n_turns - s0) && dl[1] == erel &&
+                                   dl[4] == d0[4]);
+    const int nq = __ffsll((unsigned long long)~same) - 1;
+    const int K = (int)d0[2], pending = (int)d0[3], coarse = (int)d0[4];
+    const int E = G * coarse + pending;
+    const bf16_t* pw = p.pw_pool + ((size_t)erel * BH + bh) * p.pool_pcap * D;
+    const SwRows sw{p.sw + (size_t)bh * p.fine_cap * D,
+                    p.psw_pool + ((size_t)erel * BH + bh) * 8 * D, K * G};
+    for (int i = tid; i < kTurnSlots * (kTurnMaxEpoch / 256); i += kQThreads) (&opens[0][0])[i] = 0u;
+    for (int q0 = 4 * w; q0 < nq; q0 += 4 * kQWaves)
+      query_rows<D>(
+          min(4, nq - q0), lane,
+          [&](int i) __attribute__((always_inline)) {
+            return p.rq + b * p.rq_sb + d0[8 * (q0 + i)] * p.rq_st + h * p.rq_sh;
+          },
+          [&](int i) __attribute__((always_inline)) { return hs + (q0 + i) * PAD; });
+    __syncthreads();
+    // ---- coarse pages: stable top-`coarse` by page mass, listed ascending
+    if (coarse < K) {
+      for (int i = tid; i < nq * K; i += kQThreads) {
+        const int pg = i / nq, q = i - pg * nq;
+        const bf16_t* const none[1] = {nullptr};
+        float m[1];
+        item_masses<D, 1, true>(hs + q * PAD, pw + (size_t)pg * D, none, m);
+        keys[q * cap + pg] = score_key32(m[0], pg);
+      }
+      __syncthreads();
+      for (int i = tid; i < nq * K; i += kQThreads) {
+        const int pg = i / nq, q = i - pg * nq;
+        const uint32_t* row = keys + q * cap;
+        const uint32_t mine = row[pg];
+        int rank = 0;
+        for (int j = 0; j < K; ++j) rank += row[j] > mine;
+        if (rank < coarse) atomicOr(&opens[q][pg >> 5], 1u << (pg & 31));
+      }
+      __syncthreads();
+      for (int i = tid; i < nq * K; i += kQThreads) {
+        const int pg = i / nq, q = i - pg * nq;
+        const uint32_t word = opens[q][pg >> 5], bit = 1u << (pg & 31);
+        if (!(word & bit)) continue;
+        int pos = __popc(word & (bit - 1));
+        for (int j = 0; j < (pg >> 5); ++j) pos += __popc(opens[q][j]);
+        chosen[q * cap + pos] = (uint8_t)pg;
+      }
+    } else {
+      for (int i = tid; i < nq * K; i += kQThreads) {
+        const int pg = i / nq, q = i - pg * nq;
+        chosen[q * cap + pg] = (uint8_t)pg;
+      }
+    }
+    __syncthreads();
+    // ---- candidate masses: 8 fines of each chosen page, then the pending
+    // fines, two a lane (candidates 2 i and 2 i + 1 share their page)
+    auto cand = [&](int q, int j) __attribute__((always_inline)) {
+      return j < G * coarse ? chosen[q * cap + j / G] * G + j % G : K * G + (j - G * coarse);
+    };
+    const int pairs = (E + 1) / 2;
+    for (int i = tid; i < nq * pairs; i += kQThreads) {
+      const int j = 2 * (i / nq), q = i - (j / 2) * nq;
+      const int id = cand(q, j);
+      const bf16_t* const rows[2] = {sw.row(id, D), sw.row(min(id + 1, K * G + pending - 1), D)};
+      float m[2];
+      item_masses<D, 2, false>(hs + q * PAD, pw + (size_t)(id / G) * D, rows, m);
+      keys[q * cap + j] = score_key32(m[0], j);
+      if (j + 1 < E) keys[q * cap + j + 1] = score_key32(m[1], j + 1);
+    }
+    __syncthreads();
+    // ---- stable top-M in score order
+    for (int i = tid; i < nq * E; i += kQThreads) {
+      const int j = i / nq, q = i - j * nq;
+      const int64_t* d = d0 + 8 * q;
+      const uint32_t* row = keys + q * cap;
+      const uint32_t mine = row[j];
+      int rank = 0;
+      for (int l = 0; l < E; ++l) rank += row[l] > mine;
+      if (rank < (int)d[5]) {
+        const int id = cand(q, j);
+        p.sel_pool[((size_t)d[6] * BH + bh) * p.sel_cap + rank] = id;
+        if (d[7]) p.sel[(size_t)bh * p.sel_cap + rank] = id;
+      }
+    }
+    for (int q = 0; q < nq; ++q) {
+      if (!d0[8 * q + 7]) continue;                // workgroup-uniform
+      for (int i = tid; i < coarse; i += kQThreads)
+        p.chosen[(size_t)bh * p.chosen_cap + i] = chosen[q * cap + i];
+      if (bh == 0 && tid == 0) p.header[1] = (int)d0[8 * q + 5];
+    }
+    __syncthreads();                               // h rows, keys and lists are reused
+    s0 += nq;
   }
 }
 
@@ -964,42 +1157,45 @@ __global__ __launch_bounds__(kQThreads) void route_turns_kernel(RouteParams p) {
 
 hipError_t launch_route_queries(const QueryRouteParams& p, int head_dim, hipStream_t s) {
   if (p.n_tiles <= 0) return hipSuccess;
-  if (p.qsel_words < 1 || p.qsel_words > kQMaxWords || p.group != 8 || p.max_epoch < 1)
+  if (p.qsel_words < 1 || p.group != 8 || p.max_epoch < 1 || p.max_epoch > kQueryRouteMaxEpoch)
     return hipErrorInvalidValue;
-  const dim3 grid((unsigned)(p.n_tiles * p.B * p.H));
-  // Lane-per-pair kernel when every tile's page and fine rows fit its LDS
-  // rows (and tiles hold <= 32 queries); else one wave per query.
-  const int rows = p.max_epoch / p.group + 1 + p.max_epoch;
-  if (head_dim == 128) {
-    if (rows <= RouteTileGeo<128>::ROWS)
-      hipLaunchKernelGGL(route_tile_kernel<128>, grid, dim3(kQThreads), 0, s, p);
-    else
-      hipLaunchKernelGGL(route_queries_kernel<128>, grid, dim3(kQThreads), 0, s, p);
-  } else if (head_dim == 64) {
-    if (rows <= RouteTileGeo<64>::ROWS)
-      hipLaunchKernelGGL(route_tile_kernel<64>, grid, dim3(kQThreads), 0, s, p);
-    else
-      hipLaunchKernelGGL(route_queries_kernel<64>, grid, dim3(kQThreads), 0, s, p);
-  } else {
-    return hipErrorInvalidValue;
+  if (head_dim != 64 && head_dim != 128) return hipErrorInvalidValue;
+  // Two read tiles a workgroup fill a wave's lanes; one where their keys
+  // would not fit the LDS (beyond about 900 visible fines at D128).
+  RouteLds lds = route_lds(64, p.max_epoch);
+  if (lds.bytes(head_dim) > kLdsBytes) lds = route_lds(32, p.max_epoch);
+  const size_t bytes = lds.bytes(head_dim);
+  const int per = lds.slots / 32;
+  const dim3 grid((unsigned)((p.n_tiles + per - 1) / per * p.B * p.H));
+  const auto kernel = head_dim == 128 ? route_queries_kernel<128> : route_queries_kernel<64>;
+  if (bytes > 64 * 1024) {
+    const hipError_t e = hipFuncSetAttribute(
+        (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return e;
   }
+  hipLaunchKernelGGL(kernel, grid, dim3(kQThreads), bytes, s, p, lds);
   return hipGetLastError();
 }
 
 hipError_t launch_route(const RouteParams& p, int head_dim, hipStream_t s) {
   if (p.completed > kMaxSort || p.group * p.coarse + p.pending > kMaxSort)
     return hipErrorInvalidValue;
-  // Turn mode: the lane-per-pair kernel when every turn's rows fit its LDS.
   if (p.turns && p.gate.header) return hipErrorInvalidValue;   // gates serve single turns
-  if (p.turns && p.n_turns > 0 && p.group == 8 && p.max_epoch >= 1 &&
-      p.max_epoch / 8 + 1 + p.max_epoch <= (head_dim == 64 ? kTurnRows<64> : kTurnRows<128>)) {
-    const dim3 tgrid((unsigned)(p.B * p.H * ((p.n_turns + kTurnGroup - 1) / kTurnGroup)));
-    if (head_dim == 128)
-      hipLaunchKernelGGL(route_turns_kernel<128>, tgrid, dim3(kQThreads), 0, s, p);
-    else if (head_dim == 64)
-      hipLaunchKernelGGL(route_turns_kernel<64>, tgrid, dim3(kQThreads), 0, s, p);
-    else
-      return hipErrorInvalidValue;
+  // Turn mode: a workgroup per epoch when the turns ascend by epoch and the
+  // keys of sixteen turns fit the LDS; a workgroup per turn otherwise.
+  if (p.turns && p.n_turns > 0 && p.n_epochs > 0 && p.group == 8 && p.max_epoch >= 1 &&
+      p.max_epoch <= kTurnMaxEpoch && (head_dim == 64 || head_dim == 128)) {
+    // A turn has at most its epoch's candidates and pages, p.max_epoch of both.
+    const int cap = 4 * ((p.max_epoch + 3) / 4) + 4;
+    const size_t bytes = (size_t)kTurnSlots * (2 * (head_dim + 8) + 5 * cap);
+    const dim3 tgrid((unsigned)(p.B * p.H * p.n_epochs));
+    const auto kernel = head_dim == 128 ? route_turns_kernel<128> : route_turns_kernel<64>;
+    if (bytes > 60 * 1024) {
+      const hipError_t e = hipFuncSetAttribute(
+          (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+      if (e != hipSuccess) return e;
+    }
+    hipLaunchKernelGGL(kernel, tgrid, dim3(kQThreads), bytes, s, p, cap);
     return hipGetLastError();
   }
   // Single turn (a stream's refresh): the LDS-staged kernel when its rows fit.

@@ -266,6 +266,7 @@ struct RouteParams {
   int B, H, fine_cap, page_cap, sel_cap, chosen_cap, group;
   int completed, pending, coarse, selected;
   int max_epoch;                 // turn mode: largest epoch of any turn (0: unknown)
+  int n_epochs;                  // turn mode: epochs of the turns, which ascend by epoch (0: unordered)
   TurnGate gate;                 // single-turn mode only
 };
 hipError_t launch_route(const RouteParams& p, int head_dim, hipStream_t s);
@@ -289,6 +290,7 @@ struct QueryRouteParams {
 };
 hipError_t launch_route_queries(const QueryRouteParams& p, int head_dim, hipStream_t s);
 constexpr int kQueryRouteMaxKeys = 512;   // pages or candidates of one query route
+constexpr int kQueryRouteMaxEpoch = 1024; // visible fines of one query route
 
 struct WriterParams {
   TokView rk, v;                 // token operands (positions >= new_base)
