@@ -21,8 +21,8 @@
 //  * the local attention, the value matrices, the coarse read and the
 //    selected read's numerator accumulate in fp32 in their own order, within
 //    the 1e-4 tolerance of exact arithmetic.
-// These kernels are VALU code: the fp32 path serves parity at the reference's
-// CPU-eager configuration, not throughput.
+// The contractions run on the fp32 matrix instructions (fp32 products and
+// sums); everything else is VALU code.
 #pragma clang fp contract(off)
 
 #include "schedule.h"
@@ -38,18 +38,33 @@ constexpr int kGroup = 8;           // coarse_group
 constexpr int kKeep = 512;          // local_keep
 constexpr int kRowsPerPage = 36;    // segment-weight rows of a page: prefixes n = 1..8
 constexpr int kChunk = 16;          // queries per read block
-constexpr int kKeyStage = 16;       // keys per local-attention LDS stage
-constexpr int kVChunk = 32;         // value rows per writer LDS stage
 constexpr float kLogTwoF32 = 0.693147180559945309f;   // fp32(log 2)
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// fp32 matrix instructions, accumulated in fp32. 32x32x2: lane l gives A row
+// l % 32 and B column l % 32 of k = l / 32, accumulator i is row
+// acc_row(i, l / 32) of column l % 32. 16x16x4: A row / B column l % 16 of
+// k = l / 16, accumulator i is row 4 (l / 16) + i of column l % 16.
+TAO_DEV f32x16 mfma32(float a, float b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+TAO_DEV f32x4 mfma16(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+TAO_DEV int acc_row(int i, int half) { return 8 * (i / 4) + 4 * half + i % 4; }
 
 TAO_DEV float ld(const F32View& v, int b, int64_t t, int h, int d) {
   return v.p[b * v.sb + t * v.st + h * v.sh + d];
 }
-
-TAO_DEV float wave_max(float x) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
-  return x;
+// Four channels; 16-byte loads where every row of the view allows them.
+TAO_DEV f32x4 ld4(const float* p, bool vec) {
+  if (vec) return *(const f32x4*)p;
+  return (f32x4){p[0], p[1], p[2], p[3]};
+}
+bool rows_aligned(const F32View& v) {
+  return ((uintptr_t)v.p & 15) == 0 && v.sb % 4 == 0 && v.st % 4 == 0 && v.sh % 4 == 0;
 }
 
 // Butterfly sum of the 64 lanes' values (fold halves: lane i adds lane
@@ -60,222 +75,283 @@ TAO_DEV float wave_fold(float x) {
   return __shfl(x, 0);
 }
 
-// Butterfly sum over the D channels held as lane + 64 r (R = D / 64).
-template <int R>
-TAO_DEV float channel_fold(const float (&x)[R]) {
-  float s = x[0];
-  if constexpr (R == 2) s = x[0] + x[1];
-  return wave_fold(s);
-}
-
-// Butterfly sum of n values held as lane + 64 k (k < K slots, n <= 64 K).
-template <int K>
-TAO_DEV float slot_fold(float (&x)[K], int n) {
-  int width = 1;
-  while (width < n) width <<= 1;
-  const int lane = threadIdx.x & 63;
-  float v[K];
+TAO_DEV float wave_top(float x) {
 #pragma unroll
-  for (int k = 0; k < K; ++k) v[k] = (lane + 64 * k) < n ? x[k] : 0.0f;
-  for (int half = width / 2; half >= 64; half >>= 1) {
-    const int step = half / 64;
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-      if (k < step) v[k] = v[k] + v[k + step < K ? k + step : k];
-  }
-  return wave_fold(v[0]);
+  for (int off = 32; off >= 1; off >>= 1) x = fmaxf(x, __shfl_xor(x, off));
+  return x;
 }
 
 // --------------------------------------------------------------- local tiles
 // Query t of tile j attends causally to keys [max(0, 256 j - 512), t]
 // (_local_training_corrected_4k and its ragged fallback); softmax scale
-// 1/sqrt(D) as SDPA's default. A workgroup takes 64 queries (lane t0 + i of
-// every wave holds query t0 + i) and splits their key range by 16-key stages
-// over its kLocalWaves(D) waves (stage s to wave s % waves), each wave with
-// its own LDS stage and online softmax (m, l, acc); the waves' partials are
-// merged in wave order: M = max m_w, l = sum l_w e^(m_w - M),
-// o = sum acc_w e^(m_w - M) / l.
-template <int D> constexpr int kLocalWaves = D == 64 ? 8 : 4;
-constexpr int kMergeCols = 16;       // channels per merge round
+// 1/sqrt(D) as SDPA's default. A workgroup takes 32 queries and deals their
+// 32-key blocks to eight waves, each with its own online softmax; the waves'
+// partials are merged in wave order: M = max m_w, l = sum l_w e^(m_w - M),
+// o = sum acc_w e^(m_w - M) / l. Scores are K Q^T on the fp32 matrix cores,
+// so a lane holds sixteen keys of one query: its probabilities are the
+// operand of V^T P^T as they stand, and only K passes through LDS. B1 T2048 H4
+// D64 fills the chip with 256 workgroups, about 10 us of matrix time each:
+// 124 us with a query per lane on the VALU and K, V through LDS; 29 us now,
+// the writer's blocks included (50 us before in a launch of their own).
+constexpr int kLocalWaves = 8;
+constexpr int kLocalRows = 65;       // padded lanes of a merge row
 
 template <int D>
-__global__ __launch_bounds__(64 * kLocalWaves<D>) void f32_local_kernel(F32Params p) {
-  constexpr int NW = kLocalWaves<D>;
+struct F32LocalSmem {
+  union {
+    float k[kLocalWaves][32][D + 4];             // a wave's block, padded rows
+    float red[kLocalWaves][16][kLocalRows];
+  };
+  float wm[kLocalWaves][32], wl[kLocalWaves][32];
+};
+
+// Orders one wave's LDS accesses across its lanes (scratch private to a wave).
+TAO_DEV void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int D>
+TAO_DEV void local_tile(const F32Params& p, bool vec, int t0, int b, int h, F32LocalSmem<D>& sm) {
+  constexpr int CT = D / 32;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int h = blockIdx.y, b = blockIdx.z;
-  const int t0 = blockIdx.x * 64;
-  const int t = t0 + lane;
-  const bool active = t < p.T;
+  const int half = lane >> 5, col = lane & 31;
+  const int t = t0 + col;
   const int k0 = max(0, (t0 / kFine) * kFine - kKeep);
-  const int k1 = min(p.T, t0 + 64);
-  __shared__ float ks[NW][kKeyStage][D], vs[NW][kKeyStage][D];
-  __shared__ float wm[NW][64], wl[NW][64];
+  auto& red = sm.red;
+  auto& wm = sm.wm;
+  auto& wl = sm.wl;
   const float scale = 1.0f / sqrtf((float)D);
-  float q[D], acc[D];
+  // Lane: channels half * D / 2 + i of its query (and of a block's key).
+  const int c0 = half * (D / 2);
+  f32x4 q[D / 8];
+  const float* qp = p.q.p + b * p.q.sb + (int64_t)min(t, p.T - 1) * p.q.st + h * p.q.sh + c0;
 #pragma unroll
-  for (int d = 0; d < D; ++d) {
-    q[d] = active ? ld(p.q, b, t, h, d) : 0.0f;
-    acc[d] = 0.0f;
-  }
+  for (int i = 0; i < D / 8; ++i) q[i] = ld4(qp + 4 * i, vec);
+  f32x16 acc[CT] = {};
   float m = -__builtin_inff(), l = 0.0f;
-  for (int kb = k0 + w * kKeyStage; kb < k1; kb += NW * kKeyStage) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    for (int i = lane; i < kKeyStage * D; i += 64) {
-      const int j = i / D, d = i % D, key = kb + j;
-      ks[w][j][d] = key < k1 ? ld(p.k, b, key, h, d) : 0.0f;
-      vs[w][j][d] = key < k1 ? ld(p.v, b, key, h, d) : 0.0f;
+  // Keys past the sequence (the last block's) repeat its last row; the causal
+  // mask drops them. K rows come whole (a row per 16 or 32 lanes) and turn to
+  // a row per lane in LDS: read a row per lane from memory, every load touches
+  // 64 cache lines, which the eight waves evict before their next piece.
+  f32x4 k[D / 8];
+  float v[CT][16];
+  auto load = [&](int kb) __attribute__((always_inline)) {
+    constexpr int ROWS = 256 / D;                // rows of one load
+    const int row0 = lane / (D / 4), c = 4 * (lane % (D / 4));
+    const float* kp = p.k.p + b * p.k.sb + h * p.k.sh + c;
+#pragma unroll
+    for (int i = 0; i < D / 8; ++i)
+      k[i] = ld4(kp + (int64_t)min(kb + ROWS * i + row0, p.T - 1) * p.k.st, vec);
+  };
+  auto load_v = [&](int kb) __attribute__((always_inline)) {
+    const float* vp = p.v.p + b * p.v.sb + h * p.v.sh + col;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const float* row = vp + (int64_t)min(kb + acc_row(i, half), p.T - 1) * p.v.st;
+#pragma unroll
+      for (int c2 = 0; c2 < CT; ++c2) v[c2][i] = row[32 * c2];
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    float s[kKeyStage];
-    float cm = -__builtin_inff();
+  };
+  for (int kb = k0 + 32 * w; kb <= t0; kb += 32 * kLocalWaves) {
+    load(kb);
+    if (D == 64) load_v(kb);                     // D = 128: once K's registers are free
+    wave_sync();                                 // the previous block's rows are read
+    {
+      constexpr int ROWS = 256 / D;
 #pragma unroll
-    for (int j = 0; j < kKeyStage; ++j) {
-      s[j] = -__builtin_inff();
-      if (active && kb + j <= t) {
-        float dot = 0.0f;
-#pragma unroll
-        for (int d = 0; d < D; ++d) dot = fmaf(q[d], ks[w][j][d], dot);
-        s[j] = dot * scale;
-        cm = fmaxf(cm, s[j]);
-      }
+      for (int i = 0; i < D / 8; ++i)
+        *(f32x4*)&sm.k[w][ROWS * i + lane / (D / 4)][4 * (lane % (D / 4))] = k[i];
     }
-    if (cm > -__builtin_inff()) {
-      const float mn = fmaxf(m, cm);
-      const float corr = expf(m - mn);
-      l *= corr;
+    wave_sync();
 #pragma unroll
-      for (int d = 0; d < D; ++d) acc[d] *= corr;
+    for (int i = 0; i < D / 8; ++i) k[i] = *(const f32x4*)&sm.k[w][col][c0 + 4 * i];
+    f32x16 s = {};
 #pragma unroll
-      for (int j = 0; j < kKeyStage; ++j) {
-        const float wgt = expf(s[j] - mn);
-        l += wgt;
+    for (int i = 0; i < D / 8; ++i)
 #pragma unroll
-        for (int d = 0; d < D; ++d) acc[d] = fmaf(wgt, vs[w][j][d], acc[d]);
-      }
-      m = mn;
+      for (int j = 0; j < 4; ++j) s = mfma32(k[i][j], q[i][j], s);
+    if (D == 128) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_v(kb);
     }
+    float top = -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = kb + acc_row(i, half) <= t ? s[i] * scale : -__builtin_inff();
+      top = fmaxf(top, s[i]);
+    }
+    top = fmaxf(top, __shfl_xor(top, 32));   // finite: key kb <= t0 is every query's
+    const float mn = fmaxf(m, top);
+    const float corr = expf(m - mn);
+    l *= corr;
+#pragma unroll
+    for (int c = 0; c < CT; ++c) acc[c] *= corr;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      s[i] = expf(s[i] - mn);
+      l += s[i];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+#pragma unroll
+      for (int c = 0; c < CT; ++c) acc[c] = mfma32(v[c][i], s[i], acc[c]);
+    m = mn;
   }
-  // Merge the waves' partials (a wave with no key of a query has m = -inf
-  // and weighs 0; every query sees its own key, so M is finite).
-  wm[w][lane] = m;
-  wl[w][lane] = l;
-  __syncthreads();
-  float top = wm[0][lane];
+  l += __shfl_xor(l, 32);
+  // Merge the waves' partials (a wave without a block has m = -inf and weighs
+  // 0; the block of the query's own key makes M finite).
+  if (half == 0) wm[w][col] = m;
+  __syncthreads();                               // also: the K blocks are read
+  float top = wm[0][col];
 #pragma unroll
-  for (int v = 1; v < NW; ++v) top = fmaxf(top, wm[v][lane]);
+  for (int v = 1; v < kLocalWaves; ++v) top = fmaxf(top, wm[v][col]);
   const float f = m > -__builtin_inff() ? expf(m - top) : 0.0f;
-  float lsum = 0.0f;
+  if (half == 0) wl[w][col] = l * f;
+  // 32 channels a round; thread -> (channel, query), rows of 128 bytes.
 #pragma unroll
-  for (int v = 0; v < NW; ++v)
-    lsum += wm[v][lane] > -__builtin_inff() ? wl[v][lane] * expf(wm[v][lane] - top) : 0.0f;
-  // Channel rounds through the (now free) key stages: wave w's scaled
-  // partials of kMergeCols channels, then lane i of wave w sums query i's
-  // channels w, w + NW, ... of the round over the waves in order.
-  float* red = &ks[0][0][0];                       // [NW][64][kMergeCols]
-  static_assert(NW * 64 * kMergeCols <= NW * kKeyStage * D, "merge buffer fits the stages");
-  float* o = p.local + (((size_t)b * p.T + (active ? t : 0)) * p.H + h) * D;
+  for (int c = 0; c < CT; ++c) {
+    if (c) __syncthreads();
 #pragma unroll
-  for (int c0 = 0; c0 < D; c0 += kMergeCols) {
+    for (int i = 0; i < 16; ++i) red[w][i][lane] = acc[c][i] * f;
     __syncthreads();
+    for (int i = threadIdx.x; i < 32 * 32; i += 64 * kLocalWaves) {
+      const int ch = i & 31, qi = i >> 5;
+      if (t0 + qi >= p.T) continue;
+      float sum = 0.0f, lsum = 0.0f;
 #pragma unroll
-    for (int c = 0; c < kMergeCols; ++c) red[(w * 64 + lane) * kMergeCols + c] = acc[c0 + c] * f;
-    __syncthreads();
-    for (int c = w; c < kMergeCols; c += NW) {
-      float sum = 0.0f;
-#pragma unroll
-      for (int v = 0; v < NW; ++v) sum += red[(v * 64 + lane) * kMergeCols + c];
-      if (active) o[c0 + c] = sum / lsum;
+      for (int v = 0; v < kLocalWaves; ++v) {
+        sum += red[v][(ch >> 3) * 4 + (ch & 3)][qi + 32 * ((ch >> 2) & 1)];
+        lsum += wl[v][qi];
+      }
+      p.local[(((size_t)b * p.T + t0 + qi) * p.H + h) * D + 32 * c + ch] = sum / lsum;
     }
   }
 }
 
 // ------------------------------------------------------------------- writer
-// One visible block (fine f) of one head: per channel d over its 256 tokens,
-// top = max k, e = exp(k - top), Z = quarter sums, P = e / Z,
-// z = top + log Z; then C[d][e] = sum_t P[t][d] v[t][e].
+// 32 channels d of one visible block (fine f) of one head: per channel over
+// its 256 tokens, top = max k, e = exp(k - top), Z = quarter sums, P = e / Z,
+// z = top + log Z; then C[d][e] = sum_t P[t][d] v[t][e] on the fp32 matrix
+// cores, the tokens dealt to the waves and their partials added in order.
+// Bound by the fp64 exps and the latency of its phases: sixteen tokens a
+// thread (50 us for the 20 blocks of B1 T2048 H4 D64 with a workgroup per
+// block, sixty-four tokens a thread and the product on the VALU; 14 us now,
+// alone).
+struct F32WriterSmem {
+  float prob[kFine][32];
+  float red[16][32];
+  float part_c[6][16][64];
+};
+
 template <int D>
-__global__ __launch_bounds__(4 * D) void f32_writer_kernel(F32Params p) {
-  const int f = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
-  const int tid = threadIdx.x;
-  const int d = tid % D, quarter = tid / D;
-  __shared__ float prob[kFine][D];
-  __shared__ float red[4][D];
-  __shared__ float vchunk[kVChunk][D];
+TAO_DEV void writer_slice(const F32Params& p, int f, int c0, int b, int h, F32WriterSmem& sm) {
+  constexpr int CT = D / 32, PARTS = 8 / CT, STEP = kFine / PARTS;
+  const int tid = threadIdx.x, d = tid & 31, seg = tid >> 5;
+  auto& prob = sm.prob;
+  auto& red = sm.red;
+  auto& part_c = sm.part_c;
   const int64_t base = (int64_t)f * kFine;
+  const size_t bh = (size_t)b * p.H + h;
+  float x[16];
   float top = -__builtin_inff();
-  for (int i = 0; i < 64; ++i) top = fmaxf(top, ld(p.rk, b, base + quarter * 64 + i, h, d));
-  red[quarter][d] = top;
-  __syncthreads();
-  top = fmaxf(fmaxf(red[0][d], red[1][d]), fmaxf(red[2][d], red[3][d]));
-  __syncthreads();
-  float acc = 0.0f;
-  for (int i = 0; i < 64; ++i) {
-    const int tok = quarter * 64 + i;
-    const float e = exp_cr(ld(p.rk, b, base + tok, h, d) - top);
-    prob[tok][d] = e;
-    acc = acc + e;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    x[i] = ld(p.rk, b, base + 16 * seg + i, h, c0 + d);
+    top = fmaxf(top, x[i]);
   }
-  red[quarter][d] = acc;
+  red[seg][d] = top;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 16; ++i) top = fmaxf(top, red[i][d]);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    x[i] = exp_cr(x[i] - top);
+    prob[16 * seg + i][d] = x[i];
+  }
+  __syncthreads();
+  if (seg < 4) {                       // the quarter's tokens in order
+    float acc = 0.0f;
+#pragma unroll 16
+    for (int i = 0; i < 64; ++i) acc = acc + prob[64 * seg + i][d];
+    red[seg][d] = acc;
+  }
   __syncthreads();
   const float total = (red[0][d] + red[1][d]) + (red[2][d] + red[3][d]);
-  for (int i = 0; i < 64; ++i) {
-    const int tok = quarter * 64 + i;
-    prob[tok][d] = prob[tok][d] / total;
-  }
-  const size_t bh = (size_t)b * p.H + h;
-  if (quarter == 0) p.fine_z[(bh * p.S + f) * D + d] = top + log_cr(total);
+#pragma unroll
+  for (int i = 0; i < 16; ++i) prob[16 * seg + i][d] = x[i] / total;
+  if (seg == 0) p.fine_z[(bh * p.S + f) * D + c0 + d] = top + log_cr(total);
   __syncthreads();
-  constexpr int E = D / 4;
-  const int row = tid / 4, part = tid % 4;
-  float c[E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) c[e] = 0.0f;
-  // v staged kVChunk tokens at a time (the token order of the sums is kept).
-  for (int c0 = 0; c0 < kFine; c0 += kVChunk) {
-    __syncthreads();
-    for (int i = tid; i < kVChunk * D; i += 4 * D) {
-      const int tt = i / D, e = i % D;
-      vchunk[tt][e] = ld(p.v, b, base + c0 + tt, h, e);
-    }
-    __syncthreads();
-    for (int tt = 0; tt < kVChunk; ++tt) {
-      const float pr = prob[c0 + tt][row];
-#pragma unroll
-      for (int e = 0; e < E; ++e) c[e] = fmaf(pr, vchunk[tt][part * E + e], c[e]);
-    }
+  const int lane = tid & 63, half = lane >> 5, col = lane & 31;
+  const int ct = (tid >> 6) % CT, part = (tid >> 6) / CT;
+  f32x16 acc = {};
+  const float* vp = p.v.p + b * p.v.sb + h * p.v.sh + 32 * ct + col;
+#pragma unroll 16
+  for (int i = 0; i < STEP / 2; ++i) {
+    const int tok = STEP * part + 2 * i + half;
+    acc = mfma32(prob[tok][col], vp[(base + tok) * p.v.st], acc);
   }
-  float* out = p.bank + ((bh * p.S + f) * D + row) * D + part * E;
+  if (part)
 #pragma unroll
-  for (int e = 0; e < E; ++e) out[e] = c[e];
+    for (int i = 0; i < 16; ++i) part_c[(part - 1) * CT + ct][i][lane] = acc[i];
+  __syncthreads();
+  if (part) return;
+  float* out = p.bank + ((bh * p.S + f) * D + c0) * D + 32 * ct + col;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    float sum = acc[i];
+#pragma unroll
+    for (int v = 1; v < PARTS; ++v) sum += part_c[(v - 1) * CT + ct][i][lane];
+    out[(size_t)acc_row(i, half) * D] = sum;
+  }
+}
+
+// Both in one launch: they do not depend on each other, and the writer's few
+// workgroups (dispatched first) run beside the local tiles. One workgroup a
+// CU: two of them would share its matrix cores while other CUs are idle (46
+// against 37 us at B1 T2048 H4 D64, measured before the tiles went out in
+// descending order over all heads).
+template <int D>
+__global__ __launch_bounds__(64 * kLocalWaves, 2) void f32_front_kernel(
+    F32Params p, bool vec, int writers) {
+  __shared__ union {
+    F32LocalSmem<D> local;
+    F32WriterSmem writer;
+  } sm;
+  constexpr int SL = D / 32;
+  const int BH = p.B * p.H;
+  const int x = blockIdx.x / BH, bh = blockIdx.x % BH, b = bh / p.H, h = bh % p.H;
+  if (x < writers)
+    writer_slice<D>(p, x / SL, 32 * (x % SL), b, h, sm.writer);
+  else   // the longest windows first
+    local_tile<D>(p, vec, ((int)gridDim.x / BH - 1 - x) * 32, b, h, sm.local);
 }
 
 // -------------------------------------------------------------------- pages
-// Page pg: pz[n - 1] = logsumexp of its first n fines for every prefix n
-// present (a completed page's summary is n = 8, a pending page's the prefix
-// a tile sees), the segment weights exp(z - pz[n - 1]) of those n fines, and,
+// Prefix n of page pg (a workgroup each): pz[n - 1] = logsumexp of its first
+// n fines (a completed page's summary is n = 8, a pending page's the prefix a
+// tile sees), the segment weights exp(z - pz[n - 1]) of those n fines, and,
 // with coarse values, the completed page's value matrix
 // PC[d][e] = sum_s w_s[d] C_s[d][e] (tao_stream.py:486-499).
 template <int D>
-__global__ __launch_bounds__(D) void f32_pages_kernel(F32Params p) {
-  const int pg = blockIdx.x, h = blockIdx.y, b = blockIdx.z, d = threadIdx.x;
+__global__ __launch_bounds__(256) void f32_pages_kernel(F32Params p) {
+  const int pg = blockIdx.x / kGroup, n = 1 + blockIdx.x % kGroup;
+  const int h = blockIdx.y, b = blockIdx.z;
   const size_t bh = (size_t)b * p.H + h;
   const int first = pg * kGroup;
-  const int avail = min(kGroup, p.S - first);
-  float z[kGroup];
-#pragma unroll
-  for (int i = 0; i < kGroup; ++i) z[i] = i < avail ? p.fine_z[(bh * p.S + first + i) * D + d] : 0.0f;
-  float* pz = p.pz + (bh * p.P8 + pg) * kGroup * D;
-  float* sw = p.swt + (bh * p.P8 + pg) * kRowsPerPage * D;
-  float wfull[kGroup];
-  for (int n = 1; n <= avail; ++n) {
+  if (n > p.S - first) return;
+  __shared__ float wfull[kGroup][D];
+  const int d = threadIdx.x;
+  if (d < D) {
+    float z[kGroup], e[kGroup];
     float top = -__builtin_inff();
-    for (int i = 0; i < n; ++i) top = fmaxf(top, z[i]);
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) {
+      z[i] = i < n ? p.fine_z[(bh * p.S + first + i) * D + d] : -__builtin_inff();
+      top = fmaxf(top, z[i]);
+    }
     if (__builtin_isinf(top)) top = 0.0f;
-    float e[kGroup];
 #pragma unroll
     for (int i = 0; i < kGroup; ++i) e[i] = i < n ? exp_cr(z[i] - top) : 0.0f;
     int width = 1;
@@ -285,260 +361,364 @@ __global__ __launch_bounds__(D) void f32_pages_kernel(F32Params p) {
       for (int i = 0; i < kGroup / 2; ++i)
         if (i < half) e[i] = e[i] + e[i + half];
     const float v = log_cr(e[0]) + top;
-    pz[(n - 1) * D + d] = v;
-    const int row0 = n * (n - 1) / 2;
-    for (int j = 0; j < n; ++j) {
-      const float w = exp_cr(z[j] - v);
-      sw[(row0 + j) * D + d] = w;
-      if (n == kGroup) wfull[j] = w;
-    }
-  }
-  if (p.pc && avail == kGroup) {
-    const float* c = p.bank + ((bh * p.S + first) * D + d) * D;
-    float* out = p.pc + ((bh * p.Pc + pg) * D + d) * D;
-    for (int e = 0; e < D; ++e) {
-      float acc = 0.0f;
+    p.pz[((bh * p.P8 + pg) * kGroup + n - 1) * D + d] = v;
+    float* sw = p.swt + ((bh * p.P8 + pg) * kRowsPerPage + n * (n - 1) / 2) * D + d;
 #pragma unroll
-      for (int s = 0; s < kGroup; ++s) acc = fmaf(wfull[s], c[(size_t)s * D * D + e], acc);
-      out[e] = acc;
-    }
+    for (int j = 0; j < kGroup; ++j)
+      if (j < n) {
+        const float w = exp_cr(z[j] - v);
+        sw[(size_t)j * D] = w;
+        wfull[j][d] = w;
+      }
+  }
+  if (!p.pc || n < kGroup) return;
+  __syncthreads();
+  const float* c = p.bank + (bh * p.S + first) * D * D;
+  float* out = p.pc + (bh * p.Pc + pg) * D * D;
+  for (int i = threadIdx.x; i < D * D; i += 256) {
+    float acc = 0.0f;
+#pragma unroll
+    for (int s = 0; s < kGroup; ++s) acc = fmaf(wfull[s][i / D], c[(size_t)s * D * D + i], acc);
+    out[i] = acc;
   }
 }
 
 // --------------------------------------------------------------------- read
-// kChunk queries of one tile and head per block (one wave). Tile prologue:
-// the pages the tile sees (completed pages' summaries, the pending page's
-// prefix summary), page weights softmax over them per channel and, with
-// coarse values, the coarse weights softmax over the completed pages. Per
-// query: h = softmax(raw_q), hv = h * pw, page masses, the chosen pages,
-// candidate masses, the stable top-M, the selected read, the coarse read and
-// the fusion.
+// kChunk queries of one tile and head per workgroup of four waves. Tile
+// prologue: the pages the tile sees (completed pages' summaries, the pending
+// page's prefix summary), page weights softmax over them per channel and,
+// with coarse values, the coarse weights softmax over the completed pages.
+// Then h = softmax(raw_q); page masses of the (query, page) pairs and
+// candidate masses of the (query, candidate) pairs, a lane each with the
+// channel sum in registers; ranks by counting; and the reads on the fp32
+// matrix cores: per fine that any of the queries selected, the rows
+// ch = (h pw) sw of the queries that did (0 for the others) against its
+// matrix, a wave per 16 columns. B1 T2048 H4 D64: 57 us with a wave per query
+// (a cross-lane fold per mass, the read on the VALU), 22 us now.
 constexpr int kMaxPages = 64;
 constexpr int kMaxCand = 256;
-constexpr int kReadWaves = 4;        // waves per block; wave w reads queries t0 + w + 4 k
+constexpr int kReadThreads = 256;
 
-// Orders one wave's LDS accesses across its lanes (scratch private to a wave).
-TAO_DEV void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+// LDS of a read workgroup in floats; pages and cand: the call's largest.
+struct F32ReadLds {
+  int pages, cand;
+  __host__ __device__ size_t floats(int D) const {
+    return (size_t)2 * pages * D + 3 * kChunk * (D + 4) +
+           (size_t)kChunk * cand * 3 + kChunk;
+  }
+};
+
+// Monotone key of a mass: larger mass -> larger key, -0 as +0; a NaN has a
+// place in the order too, so every rank is taken once.
+TAO_DEV uint32_t f32_order_key(float x) {
+  uint32_t u = __float_as_uint(x);
+  if (u == 0x80000000u) u = 0u;
+  return u & 0x80000000u ? ~u : u | 0x80000000u;
 }
 
-TAO_DEV int stable_rank(float mine, int idx, int n, const float* all) {
+TAO_DEV int stable_rank(int idx, int n, const float* all) {
+  const uint32_t mine = f32_order_key(all[idx]);
   int r = 0;
   for (int j = 0; j < n; ++j) {
-    const float o = all[j];
-    r += (o > mine) || (o == mine && j < idx);
+    const uint32_t o = f32_order_key(all[j]);
+    r += o > mine || (o == mine && j < idx);
   }
   return r;
 }
 
+// Fold of (h pw) [sw] over the D channels by one lane: eight partial sums of
+// the channels 8 c + k (blocks e, e + 64 and e + 32, then the chunks c, c + 2
+// and c, c + 1), then k by halves.
+template <int D, bool SW>
+TAO_DEV float lane_fold(const float* h, const float* pw, const float* sw) {
+  auto block = [&](int e0, float (&y)[8]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int v = 0; v < 2; ++v) {
+      const f32x4 a = *(const f32x4*)(h + e0 + 4 * v), c = *(const f32x4*)(pw + e0 + 4 * v);
+      f32x4 x;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) x[k] = a[k] * c[k];
+      if constexpr (SW) {
+        const f32x4 g = *(const f32x4*)(sw + e0 + 4 * v);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) x[k] = x[k] * g[k];
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) y[4 * v + k] = x[k];
+    }
+  };
+  float chunk[4][8];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    float y[D / 32][8];
+#pragma unroll
+    for (int i = 0; i < D / 32; ++i) block(8 * c + 32 * i, y[i]);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      if constexpr (D == 64)
+        chunk[c][k] = y[0][k] + y[1][k];
+      else
+        chunk[c][k] = (y[0][k] + y[2][k]) + (y[1][k] + y[3][k]);
+    }
+  }
+  float s[8];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) s[k] = (chunk[0][k] + chunk[2][k]) + (chunk[1][k] + chunk[3][k]);
+  return ((s[0] + s[4]) + (s[2] + s[6])) + ((s[1] + s[5]) + (s[3] + s[7]));
+}
+
 template <int D>
-__global__ __launch_bounds__(64 * kReadWaves) void f32_read_kernel(F32Params p) {
-  constexpr int R = D / 64;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+__global__ __launch_bounds__(kReadThreads) void f32_read_kernel(F32Params p, F32ReadLds lds) {
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int h = blockIdx.y, b = blockIdx.z;
-  const int t0 = blockIdx.x * kChunk;
-  const int tend = min(p.T, t0 + kChunk);
+  const int t0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * kChunk;
+  const int nq = min(p.T - t0, kChunk);
   const int tile = t0 / kFine;
   const int visible = max(0, tile - kKeep / kFine);
   const size_t bh = (size_t)b * p.H + h;
-  auto out_at = [&](int t, int d) -> float* {
-    return p.out + b * p.out_sb + (int64_t)t * p.out_st + h * p.out_sh + d;
-  };
-  const float* local = p.local;
+  float* out = p.out + b * p.out_sb + (int64_t)t0 * p.out_st + h * p.out_sh;
+  const float* local = p.local + ((size_t)b * p.T + t0) * p.H * D + (size_t)h * D;
+  int32_t* sel_out = p.sel_out ? p.sel_out + (((size_t)b * p.T + t0) * p.H + h) * p.sel_cap : nullptr;
   if (!visible) {   // neither history branch present: the output is local
-    for (int t = t0 + w; t < tend; t += kReadWaves) {
-#pragma unroll
-      for (int r = 0; r < R; ++r)
-        *out_at(t, lane + 64 * r) = local[(((size_t)b * p.T + t) * p.H + h) * D + lane + 64 * r];
-      if (p.sel_out)
-        for (int m = lane; m < p.sel_cap; m += 64)
-          p.sel_out[(((size_t)b * p.T + t) * p.H + h) * p.sel_cap + m] = -1;
-    }
+    for (int i = tid; i < nq * D; i += kReadThreads)
+      out[(i / D) * p.out_st + i % D] = local[(size_t)(i / D) * p.H * D + i % D];
+    if (sel_out)
+      for (int i = tid; i < nq * p.sel_cap; i += kReadThreads)
+        sel_out[(size_t)(i / p.sel_cap) * p.H * p.sel_cap + i % p.sel_cap] = -1;
     return;
   }
   const int completed = visible / kGroup, pending = visible % kGroup;
   const int P = completed + (pending > 0);
   int64_t coarse64 = 0, elig64 = 0, sel64 = 0;
   sched::routed_counts(p.cfg, completed, pending, &coarse64, &elig64, &sel64);
-  const int coarse = (int)coarse64, M = (int)sel64;
+  const int coarse = (int)coarse64, M = (int)sel64, E = coarse * kGroup + pending;
   const bool coarse_on = p.coarse_values && tile * kFine >= kKeep + kGroup * kFine;
 
-  __shared__ float pw[kMaxPages][D];
-  __shared__ float cw[kMaxPages][D];
-  __shared__ float mass_all[kReadWaves][kMaxCand];
-  __shared__ int cand_all[kReadWaves][kMaxCand];
-  __shared__ int sel_all[kReadWaves][kMaxCand];
-  __shared__ float row_all[kReadWaves][D];
-  float* mass_s = mass_all[w];                 // this wave's query scratch
-  int* cand_id = cand_all[w];
-  int* sel_id = sel_all[w];
-  float* row_s = row_all[w];
+  extern __shared__ __align__(16) float read_smem[];
+  constexpr int HP = D + 4;                            // padded h / ch row
+  float* const pw = read_smem;                         // [page][D]
+  float* const cw = pw + lds.pages * D;                // [page][D]
+  float* const hs = cw + lds.pages * D;                // [query][HP]
+  float* const ch = hs + kChunk * HP;                  // [2][query][HP]
+  float* const mass = ch + 2 * kChunk * HP;            // [query][cand]
+  float* const slots = mass + kChunk * lds.cand;       // [query][cand] masses by rank
+  int16_t* const cand = (int16_t*)(slots + kChunk * lds.cand);   // [query][cand] fine ids
+  int16_t* const sel = cand + kChunk * lds.cand;       // [query][cand] ids by rank
+  float* const den = (float*)(sel + kChunk * lds.cand);          // [query]
+  __shared__ uint32_t picked[kChunk][kMaxPages * kGroup / 32];   // bit per fine
+  __shared__ uint32_t open[kChunk][kMaxPages / 32];
+  const int PC = lds.cand;
 
-  // Page z the tile sees, page weights and coarse weights (lanes = pages;
-  // the waves take the channels in turn).
+  for (int i = tid; i < kChunk * (kMaxPages * kGroup / 32); i += kReadThreads) (&picked[0][0])[i] = 0u;
+  if (tid < kChunk * (kMaxPages / 32)) (&open[0][0])[tid] = 0u;
+  // Page z the tile sees, page weights and coarse weights: a thread per
+  // channel for up to 8 pages (the fold over the next power of two), else
+  // lanes = pages and the waves take the channels in turn.
   const float* pzt = p.pz + bh * p.P8 * kGroup * D;
-  for (int d = w; d < D; d += kReadWaves) {
-    const float zp = lane < completed ? pzt[((size_t)lane * kGroup + kGroup - 1) * D + d]
-                   : (lane == completed && pending)
-                       ? pzt[((size_t)completed * kGroup + pending - 1) * D + d]
-                       : -__builtin_inff();
-    const float top = wave_max(zp);
-    const float e = lane < P ? exp_cr(zp - top) : 0.0f;
-    const float total = wave_fold(e);
-    if (lane < P) pw[lane][d] = e / total;
-    if (coarse_on) {
-      const float zc = lane < completed ? zp : -__builtin_inff();
-      const float tc = wave_max(zc);
-      const float ec = lane < completed ? exp_cr(zc - tc) : 0.0f;
-      const float tot = wave_fold(ec);
-      if (lane < completed) cw[lane][d] = ec / tot;
+  auto page_z = [&](int pg, int d) __attribute__((always_inline)) {
+    return pzt[((size_t)pg * kGroup + (pg < completed ? kGroup : pending) - 1) * D + d];
+  };
+  if (P <= kGroup) {
+    for (int i = tid; i < 2 * D; i += kReadThreads) {
+      const int d = i % D, n = i < D ? P : completed;
+      if (i >= D && !coarse_on) break;
+      float e[kGroup];
+      float top = -__builtin_inff();
+#pragma unroll
+      for (int g = 0; g < kGroup; ++g) {
+        e[g] = g < n ? page_z(g, d) : -__builtin_inff();
+        top = fmaxf(top, e[g]);
+      }
+      float s[kGroup];
+#pragma unroll
+      for (int g = 0; g < kGroup; ++g) s[g] = e[g] = g < n ? exp_cr(e[g] - top) : 0.0f;
+#pragma unroll
+      for (int half = kGroup / 2; half >= 1; half >>= 1)
+#pragma unroll
+        for (int g = 0; g < half; ++g) s[g] = s[g] + s[g + half];
+      float* dst = (i < D ? pw : cw) + d;
+#pragma unroll
+      for (int g = 0; g < kGroup; ++g)
+        if (g < n) dst[g * D] = e[g] / s[0];
     }
+  } else {
+    for (int d = w; d < D; d += kReadThreads / 64) {
+      const float zp = lane < P ? page_z(lane, d) : -__builtin_inff();
+      const float top = wave_top(zp);                  // all lanes take part
+      const float e = lane < P ? exp_cr(zp - top) : 0.0f;
+      const float total = wave_fold(e);
+      if (lane < P) pw[lane * D + d] = e / total;
+      if (coarse_on) {
+        const float zc = lane < completed ? zp : -__builtin_inff();
+        const float tc = wave_top(zc);
+        const float ec = lane < completed ? exp_cr(zc - tc) : 0.0f;
+        const float tot = wave_fold(ec);
+        if (lane < completed) cw[lane * D + d] = ec / tot;
+      }
+    }
+  }
+  // h = softmax over channels of raw_q: sixteen lanes a query, lane i of
+  // them the channels i + 16 k.
+  {
+    const int q = tid >> 4, i = tid & 15;
+    float x[D / 16], s[D / 16];
+#pragma unroll
+    for (int k = 0; k < D / 16; ++k) x[k] = ld(p.rq, b, t0 + min(q, nq - 1), h, i + 16 * k);
+    float top = x[0];
+#pragma unroll
+    for (int k = 1; k < D / 16; ++k) top = fmaxf(top, x[k]);
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) top = fmaxf(top, __shfl_xor(top, off));
+#pragma unroll
+    for (int k = 0; k < D / 16; ++k) s[k] = x[k] = exp_cr(x[k] - top);
+#pragma unroll
+    for (int half = D / 32; half >= 1; half >>= 1)
+#pragma unroll
+      for (int k = 0; k < half; ++k) s[k] = s[k] + s[k + half];
+    float total = s[0];
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) total = total + __shfl_xor(total, off);
+#pragma unroll
+    for (int k = 0; k < D / 16; ++k) hs[q * HP + i + 16 * k] = x[k] / total;
   }
   __syncthreads();
 
   const float* swt = p.swt + bh * p.P8 * kRowsPerPage * D;
-  auto sw_row = [&](int id) -> const float* {
+  auto sw_row = [&](int id) __attribute__((always_inline)) {
     const int pg = id / kGroup, j = id % kGroup;
     const int n = pg < completed ? kGroup : pending;
     return swt + ((size_t)pg * kRowsPerPage + n * (n - 1) / 2 + j) * D;
   };
-  const float* bank = p.bank + bh * p.S * D * D;
-  const float* pcb = p.pc ? p.pc + bh * p.Pc * D * D : nullptr;
-  float a[R][3], fb[R][3];
+  // Chosen pages: stable top-`coarse` of the completed pages' masses.
+  if (coarse < completed) {
+    for (int i = tid; i < kChunk * completed; i += kReadThreads) {
+      const int q = i % kChunk, pg = i / kChunk;
+      mass[q * PC + pg] = lane_fold<D, false>(hs + q * HP, pw + pg * D, nullptr);
+    }
+    __syncthreads();
+    for (int i = tid; i < kChunk * completed; i += kReadThreads) {
+      const int q = i % kChunk, pg = i / kChunk;
+      if (stable_rank(pg, completed, mass + q * PC) < coarse)
+        atomicOr(&open[q][pg >> 5], 1u << (pg & 31));
+    }
+    __syncthreads();
+  }
+  for (int i = tid; i < kChunk * P; i += kReadThreads) {
+    const int q = i % kChunk, pg = i / kChunk;
+    int pos = pg;
+    if (coarse < completed && pg < completed) {
+      const uint32_t word = open[q][pg >> 5], bit = 1u << (pg & 31);
+      if (!(word & bit)) continue;
+      pos = __popc(word & (bit - 1)) + (pg >= 32 ? __popc(open[q][0]) : 0);
+    } else if (pg == completed) {
+      pos = coarse;
+    }
+    for (int s = 0; s < (pg < completed ? kGroup : pending); ++s)
+      cand[q * PC + pos * kGroup + s] = (int16_t)(pg * kGroup + s);
+  }
+  __syncthreads();
+  // Candidate masses sum_d (h pw[page]) sw[fine], then the stable top-M.
+  for (int i = tid; i < kChunk * E; i += kReadThreads) {
+    const int q = i % kChunk, c = i / kChunk, id = cand[q * PC + c];
+    mass[q * PC + c] = lane_fold<D, true>(hs + q * HP, pw + (id / kGroup) * D, sw_row(id));
+  }
+  __syncthreads();
+  for (int i = tid; i < kChunk * E; i += kReadThreads) {
+    const int q = i % kChunk, c = i / kChunk, id = cand[q * PC + c];
+    const int rank = stable_rank(c, E, mass + q * PC);
+    if (rank >= M) continue;
+    sel[q * PC + rank] = (int16_t)id;
+    slots[q * PC + rank] = mass[q * PC + c];
+    atomicOr(&picked[q][id >> 5], 1u << (id & 31));
+  }
+  __syncthreads();
+  // den = butterfly over the slots of the selected masses (a wave per query).
+  for (int q = w; q < nq; q += kReadThreads / 64) {
+    int width = 1;
+    while (width < M) width <<= 1;
+    float v[kMaxCand / 64];
 #pragma unroll
-  for (int r = 0; r < R; ++r)
+    for (int k = 0; k < kMaxCand / 64; ++k)
+      v[k] = lane + 64 * k < M ? slots[q * PC + lane + 64 * k] : 0.0f;
+    for (int half = width / 2; half >= 64; half >>= 1)
+#pragma unroll
+      for (int k = 0; k < kMaxCand / 128; ++k)
+        if (k < half / 64) v[k] = v[k] + v[k + half / 64 < kMaxCand / 64 ? k + half / 64 : k];
+    const float total = wave_fold(v[0]);
+    if (lane == 0) den[q] = total;
+    if (sel_out)
+      for (int m = lane; m < p.sel_cap; m += 64)
+        sel_out[(size_t)q * p.H * p.sel_cap + m] = m < M ? sel[q * PC + m] : -1;
+  }
+
+  // Reads: num = sum over fines of ch C, coarse = sum over pages of (h cw) PC.
+  constexpr int TW = D / 64;                           // 16-column tiles a wave
+  const int k4 = lane >> 4, col = lane & 15;
+  f32x4 num[TW] = {}, co[TW] = {};
+  int buf = 0;
+  auto product = [&](const float* c, f32x4 (&acc)[TW]) __attribute__((always_inline)) {
+    const float* row = ch + buf * kChunk * HP + col * HP + k4;
+    const float* cp = c + (size_t)k4 * D + 16 * TW * w + col;
+#pragma unroll 16
+    for (int s = 0; s < D / 4; ++s)
+#pragma unroll
+      for (int j = 0; j < TW; ++j)
+        acc[j] = mfma16(row[4 * s], cp[(size_t)4 * s * D + 16 * j], acc[j]);
+  };
+  // Two row buffers: a buffer is written again only after the barrier of the
+  // other's product, which every wave reaches when it is done with this one.
+  for (int id = 0; id < visible; ++id) {
+    uint32_t any = 0;
+#pragma unroll
+    for (int q = 0; q < kChunk; ++q) any |= picked[q][id >> 5];
+    if (!(any >> (id & 31) & 1u)) continue;            // workgroup-uniform
+    const float* sw = sw_row(id);
+    const float* pg = pw + (id / kGroup) * D;
+    float* dst = ch + buf * kChunk * HP;
+    for (int i = tid; i < kChunk * D; i += kReadThreads) {
+      const int q = i / D, d = i % D;
+      const bool on = picked[q][id >> 5] >> (id & 31) & 1u;
+      dst[q * HP + d] = on ? (hs[q * HP + d] * pg[d]) * sw[d] : 0.0f;
+    }
+    __syncthreads();
+    product(p.bank + (bh * p.S + id) * D * D, num);
+    buf ^= 1;
+  }
+  if (coarse_on) {
+    for (int pg = 0; pg < completed; ++pg) {
+      float* dst = ch + buf * kChunk * HP;
+      for (int i = tid; i < kChunk * D; i += kReadThreads) {
+        const int q = i / D, d = i % D;
+        dst[q * HP + d] = hs[q * HP + d] * cw[pg * D + d];
+      }
+      __syncthreads();
+      product(p.pc + (bh * p.Pc + pg) * D * D, co);
+      buf ^= 1;
+    }
+  }
+  __syncthreads();                                     // den
+
+  // _fuse_training at fp32 (operator.py:21-38); both history branches
+  // present only with coarse values past first_coarse.
+  const float bias = coarse_on ? kLogTwoF32 : 0.0f;
+#pragma unroll
+  for (int j = 0; j < TW; ++j) {
+    const int d = 16 * (TW * w + j) + col;
+    float a[3], fb[3];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      const int d = lane + 64 * r;
-      a[r][i] = load_param(p.fa, p.f_dtype, h * p.fa_s[0] + d * p.fa_s[1] + i * p.fa_s[2]);
-      fb[r][i] = load_param(p.fb, p.f_dtype, h * p.fb_s[0] + d * p.fb_s[1] + i * p.fb_s[2]);
+      a[i] = load_param(p.fa, p.f_dtype, h * p.fa_s[0] + d * p.fa_s[1] + i * p.fa_s[2]);
+      fb[i] = load_param(p.fb, p.f_dtype, h * p.fb_s[0] + d * p.fb_s[1] + i * p.fb_s[2]);
     }
-
-  for (int t = t0 + w; t < tend; t += kReadWaves) {
-    // h = softmax over channels of raw_q
-    float x[R], hq[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) x[r] = ld(p.rq, b, t, h, lane + 64 * r);
-    float top = x[0];
-    if constexpr (R == 2) top = fmaxf(x[0], x[1]);
-    top = wave_max(top);
-    float e[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) e[r] = exp_cr(x[r] - top);
-    const float total = channel_fold<R>(e);
-#pragma unroll
-    for (int r = 0; r < R; ++r) hq[r] = e[r] / total;
-
-    // Chosen pages: stable top-`coarse` of the completed pages' masses.
-    int E = 0;
-    if (coarse) {
-      for (int pg = 0; pg < completed; ++pg) {
-        float hv[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) hv[r] = hq[r] * pw[pg][lane + 64 * r];
-        const float m = channel_fold<R>(hv);
-        if (lane == 0) mass_s[pg] = m;
-      }
-      wave_sync();
-      const bool mine = lane < completed;
-      const int rank = mine ? stable_rank(mass_s[lane], lane, completed, mass_s) : kMaxCand;
-      const bool chosen = rank < coarse;
-      const unsigned long long bal = __ballot(chosen);
-      const int pos = __popcll(bal & ((1ull << lane) - 1ull));
-      wave_sync();
-      if (chosen)
-        for (int s = 0; s < kGroup; ++s) cand_id[pos * kGroup + s] = lane * kGroup + s;
-      E = coarse * kGroup;
-    }
-    if (lane < pending) cand_id[E + lane] = completed * kGroup + lane;
-    E += pending;
-    wave_sync();
-
-    // Candidate masses sum_d (h pw[page]) sw[fine], then the stable top-M.
-    for (int c = 0; c < E; ++c) {
-      const int id = cand_id[c];
-      const int pg = id / kGroup;
-      const float* sw = sw_row(id);
-      float ch[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int d = lane + 64 * r;
-        ch[r] = (hq[r] * pw[pg][d]) * sw[d];
-      }
-      const float m = channel_fold<R>(ch);
-      if (lane == 0) mass_s[c] = m;
-    }
-    wave_sync();
-    for (int c = lane; c < E; c += 64) {
-      const int rank = stable_rank(mass_s[c], c, E, mass_s);
-      if (rank < M) sel_id[rank] = cand_id[c];
-    }
-    wave_sync();
-    if (p.sel_out)
-      for (int m = lane; m < p.sel_cap; m += 64)
-        p.sel_out[(((size_t)b * p.T + t) * p.H + h) * p.sel_cap + m] = m < M ? sel_id[m] : -1;
-
-    // Selected read: num = sum_m ch_m C_m, den = butterfly over slots of the
-    // butterfly channel sums; fine = num / den.
-    float num[R] = {};
-    float slot[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int m = 0; m < M; ++m) {
-      const int id = sel_id[m];
-      const int pg = id / kGroup;
-      const float* sw = sw_row(id);
-      float ch[R];
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const int d = lane + 64 * r;
-        ch[r] = (hq[r] * pw[pg][d]) * sw[d];
-        row_s[d] = ch[r];
-      }
-      const float ps = channel_fold<R>(ch);
-      if ((m & 63) == lane) slot[m >> 6] = ps;
-      wave_sync();
-      const float* c = bank + (size_t)id * D * D;
-      for (int dd = 0; dd < D; ++dd) {
-        const float w = row_s[dd];
-#pragma unroll
-        for (int r = 0; r < R; ++r) num[r] = fmaf(w, c[dd * D + lane + 64 * r], num[r]);
-      }
-      wave_sync();
-    }
-    const float den = slot_fold<4>(slot, M);
-    float fine[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) fine[r] = num[r] / den;
-
-    // Coarse read over the completed pages (coarse value branch).
-    float coarse_v[R] = {};
-    if (coarse_on) {
-      for (int pg = 0; pg < completed; ++pg) {
-#pragma unroll
-        for (int r = 0; r < R; ++r) row_s[lane + 64 * r] = hq[r] * cw[pg][lane + 64 * r];
-        wave_sync();
-        const float* c = pcb + (size_t)pg * D * D;
-        for (int dd = 0; dd < D; ++dd) {
-          const float w = row_s[dd];
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-            coarse_v[r] = fmaf(w, c[dd * D + lane + 64 * r], coarse_v[r]);
-        }
-        wave_sync();
-      }
-    }
-
-    // _fuse_training at fp32 (operator.py:21-38); both history branches
-    // present only with coarse values past first_coarse.
-    const float bias = coarse_on ? kLogTwoF32 : 0.0f;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int d = lane + 64 * r;
-      const float loc = local[(((size_t)b * p.T + t) * p.H + h) * D + d];
+    for (int r = 0; r < 4; ++r) {
+      const int q = 4 * k4 + r;
+      if (q >= nq) continue;
+      const float x = ld(p.rq, b, t0 + q, h, d);
+      const float loc = local[(size_t)q * p.H * D + d];
       float s[3];
 #pragma unroll
-      for (int i = 0; i < 3; ++i) s[i] = (a[r][i] * x[r]) + fb[r][i];
+      for (int i = 0; i < 3; ++i) s[i] = (a[i] * x) + fb[i];
       s[0] = s[0] + bias;
       if (!coarse_on) s[1] = -__builtin_inff();
       const float top3 = fmaxf(s[0], fmaxf(s[1], s[2]));
@@ -548,9 +728,9 @@ __global__ __launch_bounds__(64 * kReadWaves) void f32_read_kernel(F32Params p) 
       const float tot = (e0 + e2) + e1;   // butterfly order over [e0, e1, e2, 0]
       const float r0 = e0 / tot, r1 = e1 / tot, r2 = e2 / tot;
       const float lt = r0 * (2.0f * loc);
-      const float ct = r1 * (p.gain * coarse_v[r]);
-      const float ft = r2 * (p.gain * fine[r]);
-      *out_at(t, d) = (lt + ct) + ft;
+      const float ct = r1 * (p.gain * co[j][r]);
+      const float ft = r2 * (p.gain * (num[j][r] / den[q]));
+      out[q * p.out_st + d] = (lt + ct) + ft;
     }
   }
 }
@@ -599,33 +779,39 @@ int f32_limits(const tao_stream_cfg& cfg, int64_t T, int64_t* pages, int64_t* ca
   return *pages <= kMaxPages && *cand <= kMaxCand && sel <= kMaxCand;
 }
 
-hipError_t launch_full_f32(const F32Params& p, hipStream_t s, bool own_local) {
-  const dim3 heads((unsigned)p.H, (unsigned)p.B);
-  auto grid = [&](int64_t x) { return dim3((unsigned)x, heads.x, heads.y); };
-  if (p.D == 64) {
-    if (own_local)
-      hipLaunchKernelGGL(f32_local_kernel<64>, grid((p.T + 63) / 64), dim3(64 * kLocalWaves<64>),
-                         0, s, p);
-    if (p.S) {
-      hipLaunchKernelGGL(f32_writer_kernel<64>, grid(p.S), dim3(256), 0, s, p);
-      hipLaunchKernelGGL(f32_pages_kernel<64>, grid(p.P8), dim3(64), 0, s, p);
-    }
-    hipLaunchKernelGGL(f32_read_kernel<64>, grid((p.T + kChunk - 1) / kChunk), dim3(64 * kReadWaves),
-                       0, s, p);
-  } else if (p.D == 128) {
-    if (own_local)
-      hipLaunchKernelGGL(f32_local_kernel<128>, grid((p.T + 63) / 64), dim3(64 * kLocalWaves<128>),
-                         0, s, p);
-    if (p.S) {
-      hipLaunchKernelGGL(f32_writer_kernel<128>, grid(p.S), dim3(512), 0, s, p);
-      hipLaunchKernelGGL(f32_pages_kernel<128>, grid(p.P8), dim3(128), 0, s, p);
-    }
-    hipLaunchKernelGGL(f32_read_kernel<128>, grid((p.T + kChunk - 1) / kChunk),
-                       dim3(64 * kReadWaves), 0, s, p);
-  } else {
-    return hipErrorInvalidValue;
+namespace {
+
+template <int D>
+hipError_t launch_d(const F32Params& p, hipStream_t s, bool own_local) {
+  auto grid = [&](int64_t x) { return dim3((unsigned)x, (unsigned)p.H, (unsigned)p.B); };
+  const int64_t writers = (int64_t)p.S * (D / 32), tiles = own_local ? (p.T + 31) / 32 : 0;
+  if (writers + tiles)
+    hipLaunchKernelGGL(f32_front_kernel<D>, dim3((unsigned)((writers + tiles) * p.B * p.H)),
+                       dim3(64 * kLocalWaves), 0, s, p, rows_aligned(p.q) && rows_aligned(p.k),
+                       (int)writers);
+  if (p.S) hipLaunchKernelGGL(f32_pages_kernel<D>, grid((int64_t)p.P8 * kGroup), dim3(256), 0, s, p);
+  int64_t pages = 0, cand = 0;
+  f32_limits(p.cfg, p.T, &pages, &cand);
+  // Rows of an odd number of 4-byte words: a column of them spreads over the
+  // banks.
+  const F32ReadLds lds{(int)(pages ? pages : 1), (int)(cand < pages ? pages : cand) | 1};
+  const size_t bytes = lds.floats(D) * sizeof(float);
+  if (bytes > 60 * 1024) {
+    const hipError_t e = hipFuncSetAttribute((const void*)f32_read_kernel<D>,
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+    if (e != hipSuccess) return e;
   }
+  hipLaunchKernelGGL(f32_read_kernel<D>, grid((p.T + kChunk - 1) / kChunk), dim3(kReadThreads),
+                     bytes, s, p, lds);
   return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_full_f32(const F32Params& p, hipStream_t s, bool own_local) {
+  if (p.D == 64) return launch_d<64>(p, s, own_local);
+  if (p.D == 128) return launch_d<128>(p, s, own_local);
+  return hipErrorInvalidValue;
 }
 
 }  // namespace tao

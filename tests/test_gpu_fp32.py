@@ -151,3 +151,30 @@ def test_fp32_contract_errors():
     with pytest.raises(TypeError):
         tao_attention(dev[0].to(torch.bfloat16), *dev[1:3], raw_q=dev[3], raw_k=dev[4],
                       fusion_a=fa.cuda(), fusion_b=fb.cuda(), alpha=0.5)
+
+
+@pytest.mark.parametrize("batch,tokens,heads,width,index_only", [
+    (1, 1, 1, 64, True),           # one query, one key
+    (2, 33, 3, 128, True),         # a block of 32 queries and one query more
+    (1, 769, 1, 64, False),        # one query with history
+    (1, 2561, 2, 128, False),      # the first query of the first completed page
+    (1, 17500, 1, 64, False),      # nine pages: a lane per page, chosen pages
+])
+def test_fp32_tile_edges_and_unaligned_rows(batch, tokens, heads, width, index_only):
+    """Ragged query blocks and read tiles, and operand rows at 4-byte offsets
+    (no 16-byte loads), bitwise equal to the contiguous call."""
+    xs, fa, fb = config0_inputs(batch, tokens, heads, width, 31)
+    cfg = TaoConfig(coarse_index_only=index_only)
+    print(f"fp32 edges B{batch} T{tokens} H{heads} D{width}", flush=True)
+    dev = [x.cuda() for x in xs]
+    with torch.no_grad():
+        out, sel = training.forward_f32(*dev, fa.cuda(), fb.cuda(), 0.5, cfg, return_routes=True)
+        odd = [torch.nn.functional.pad(x, (1, 2))[..., 1:-2] for x in dev]
+        shifted = tao_attention(*odd[:3], raw_q=odd[3], raw_k=odd[4], fusion_a=fa.cuda(),
+                                fusion_b=fb.cuda(), alpha=0.5, config=cfg)
+    assert torch.equal(out, shifted)
+    ref, routes = O.training_forward(*xs, fa, fb, 0.5, O.Geometry.from_config(cfg),
+                                     return_routes=True)
+    if routes:
+        check_routes(sel, routes, tokens)
+    torch.testing.assert_close(out.cpu(), ref, **TOL32)
