@@ -15,10 +15,10 @@
 // association_solve_kernel (association_writer.py:21-32): one workgroup per
 //   [D, D] pair, loaded in one round of float4 loads. The system
 //   gram + (trace / D) I is factored in LDS by a blocked right-looking
-//   Cholesky (16-column panels: the diagonal block by one wave in
-//   registers, the rows below it one thread each, rank-16 trailing updates
-//   on 4 x 4 register tiles), then cross is solved in place by forward and
-//   back substitution, 16 rows a step with 4 x 4 tiles; C = bf16(X).
+//   Cholesky (16-column panels: the diagonal block and its inverse by one
+//   wave in registers, panels and trailing updates on fp32 MFMAs), then
+//   cross^T is solved in place by both substitutions, 16 rows a wave;
+//   C = bf16(X).
 // structured_matrix_kernel (structured_writer.py:16-34): one workgroup per
 //   pair; per-channel vectors and their sums in LDS, then thread e walks
 //   column e of cross twice (hb and mass . hb, then the result).
@@ -185,38 +185,104 @@ __global__ __launch_bounds__(kStatThreads) void writer_stats_kernel(WriterStatsP
   }
 }
 
-constexpr int kSolveThreads = 1024;   // one workgroup per CU at D128 (135 KB LDS): 16 waves
-constexpr int kSolvePanel = 16;       // Cholesky panel width and substitution block
+template <int D>
+constexpr int kSolveThreads = 4 * D;  // a wave per 16 columns of the right-hand side
 
 template <int D>
 struct SolveSmem {
-  float a[D][D + 4];     // system, then its lower factor (rows 16-byte aligned)
-  float x[D][D + 4];     // cross, then Y, then X
-  float inv[D];          // reciprocal square roots of the pivots (1 / L[j][j])
-  float red[kSolveThreads / 64];
+  float a[D][D + 4];     // system, then its lower factor; diagonal blocks hold their inverses
+  float xt[D][D + 4];    // cross^T, then Y^T, then X^T (row e)
+  float red[kSolveThreads<D> / 64];
 };
 
 TAO_DEV float read_lane(float v, int lane) {
   return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
-// acc[i] -= l[i] * r (componentwise), as one fp32 FMA per element.
-TAO_DEV void sub_outer(float4 (&acc)[4], const float (&l)[4], const float4& r) {
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// acc -= A B over 16 columns of A, on the fp32 matrix instructions (fp32
+// products and sums): A's 16 rows at `a` (stride LD), B[k][c] = b[c][k] with
+// B_ROWS (a row of b per column), else b[k][c].
+template <int LD, bool B_ROWS>
+TAO_DEV f32x4 sub_product(const float* a, const float* b, f32x4 acc, int lane) {
+  const int r = lane & 15, k4 = lane >> 4;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    acc[i].x = fmaf(-l[i], r.x, acc[i].x);
-    acc[i].y = fmaf(-l[i], r.y, acc[i].y);
-    acc[i].z = fmaf(-l[i], r.z, acc[i].z);
-    acc[i].w = fmaf(-l[i], r.w, acc[i].w);
+  for (int s = 0; s < 4; ++s) {
+    const int k = 4 * s + k4;
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(-a[r * LD + k], B_ROWS ? b[r * LD + k] : b[k * LD + r],
+                                               acc, 0, 0, 0);
   }
+  return acc;
+}
+// Accumulator i of a lane is row 4 (lane / 16) + i of column lane % 16.
+template <int LD>
+TAO_DEV f32x4 load_block(const float* p, int lane) {
+  f32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = p[(4 * (lane >> 4) + i) * LD + (lane & 15)];
+  return v;
+}
+template <int LD>
+TAO_DEV void store_block(float* p, f32x4 v, int lane) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) p[(4 * (lane >> 4) + i) * LD + (lane & 15)] = v[i];
 }
 
+// Orders one wave's LDS accesses across its lanes.
+TAO_DEV void solve_wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Factor of a 16 x 16 diagonal block and its inverse, by one wave: lane
+// c < 16 holds column c of the rows (the block is symmetric), lane 16 + c
+// column c of the identity; eliminating row by row leaves L^T in the first
+// and L^-1 in the second half. The block is replaced by L^-1 (zeros above its
+// diagonal), all that the panel and the substitutions need of it. Pivots are
+// taken by v_rsq_f32 (about 1 ulp). Returns the first column (from j0 + 1)
+// whose pivot is not positive, or `bad`.
+template <int LD>
+TAO_DEV int factor_block(float* blk, int j0, int lane, int bad) {
+  float r[16];
+#pragma unroll
+  for (int c = 0; c < 16; ++c)
+    r[c] = lane < 16 ? blk[c * LD + lane] : (lane == 16 + c ? 1.0f : 0.0f);
+#pragma unroll
+  for (int c = 0; c < 16; ++c) {
+    const float piv = read_lane(r[c], c);
+    if (!(piv > 0.0f)) bad = bad ? bad : j0 + c + 1;
+    r[c] *= __builtin_amdgcn_rsqf(piv);
+#pragma unroll
+    for (int k = c + 1; k < 16; ++k) r[k] = fmaf(-read_lane(r[c], k), r[c], r[k]);
+  }
+  solve_wave_sync();
+  if (lane >= 16 && lane < 32) {
+#pragma unroll
+    for (int c = 0; c < 16; ++c) blk[c * LD + lane - 16] = r[c];
+  }
+  solve_wave_sync();
+  return bad;
+}
+
+// (gram + tr(gram)/D I)^-1 cross by a blocked Cholesky factorization and two
+// triangular solves, one workgroup per system. A system is one serial chain
+// (a CU holds one at D = 128), so the chain is what counts: 16-column steps
+// whose products run on the fp32 matrix instructions, the next diagonal block
+// factored by wave 0 while the others update the rest of the trailing
+// triangle (two barriers a step), and the solves as X^T rows: a wave owns 16
+// right-hand sides, so both substitutions need no barrier at all. With
+// rank-16 updates and substitutions on the VALU (4 x 4 tiles from LDS, five
+// barriers a step): 68 us for up to 256 D128 systems; 37 us now.
 template <int D>
-__global__ __launch_bounds__(kSolveThreads) void association_solve_kernel(AssocSolveParams p) {
+__global__ __launch_bounds__(kSolveThreads<D>) void association_solve_kernel(AssocSolveParams p) {
   extern __shared__ __align__(16) unsigned char solve_smem[];
   SolveSmem<D>& sm = *reinterpret_cast<SolveSmem<D>*>(solve_smem);
+  constexpr int LD = D + 4, NB = D / 16, NW = NB, NT = kSolveThreads<D>;
   const int mat = blockIdx.x;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int blk = (p.to_slots || p.rhs_t) ? mat / (p.B * p.H) : 0;
   if (p.to_slots == 2 && (p.fine_first + blk) % p.group != p.group - 1) return;   // uniform
   const float* g = p.gram + (size_t)mat * D * D;
@@ -226,233 +292,141 @@ __global__ __launch_bounds__(kSolveThreads) void association_solve_kernel(AssocS
     const int b = (mat / p.H) % p.B, h = mat % p.H;
     rt = p.rhs_t + (((size_t)b * p.H + h) * p.rhs_cap + blk) * D * D;
   }
-  // Every load of the system in one round: the diagonal (for the ridge),
-  // then gram and the right-hand side as float4 (rows of D floats).
-  constexpr int V4 = D * D / 4 / kSolveThreads;   // float4 per thread and matrix
-  static_assert(D * D % (4 * kSolveThreads) == 0, "whole float4 per thread");
+  // Every load of the system in one round. The right-hand side turns on its
+  // way into LDS: a wave takes 16 x 16 pieces (16 rows d, four float4 each),
+  // whose transposed stores fall in 64 different banks.
+  constexpr int V4 = D * D / 4 / NT;              // float4 per thread and matrix
   const float gd = tid < D ? g[(size_t)tid * D + tid] : 0.0f;
   float4 gv[V4], cv[V4];
+  auto piece = [&](int k, int& d, int& e) __attribute__((always_inline)) {
+    const int t = k * NW + w;
+    d = 16 * (t / NB) + (lane & 15);
+    e = 16 * (t % NB) + 4 * (lane >> 4);
+  };
 #pragma unroll
   for (int k = 0; k < V4; ++k) {
-    const int i4 = tid + k * kSolveThreads;
-    gv[k] = ((const float4*)g)[i4];
-    cv[k] = ((const float4*)(rt ? rt : c))[i4];
+    gv[k] = ((const float4*)g)[tid + k * NT];
+    if (rt) {
+      cv[k] = ((const float4*)rt)[tid + k * NT];
+    } else {
+      int d, e;
+      piece(k, d, e);
+      cv[k] = *(const float4*)(c + (size_t)d * D + e);
+    }
   }
 #pragma unroll
   for (int k = 0; k < V4; ++k) {
-    const int i = 4 * (tid + k * kSolveThreads), r = i / D, col = i % D;
+    const int i = 4 * (tid + k * NT), r = i / D, col = i % D;
     *(float4*)&sm.a[r][col] = gv[k];
-    if (rt) {   // rt[e][d] with e = r, d = col .. col + 3: x[d][e]
-      sm.x[col][r] = cv[k].x;
-      sm.x[col + 1][r] = cv[k].y;
-      sm.x[col + 2][r] = cv[k].z;
-      sm.x[col + 3][r] = cv[k].w;
+    if (rt) {
+      *(float4*)&sm.xt[r][col] = cv[k];
     } else {
-      *(float4*)&sm.x[r][col] = cv[k];
+      int d, e;
+      piece(k, d, e);
+      sm.xt[e][d] = cv[k].x;
+      sm.xt[e + 1][d] = cv[k].y;
+      sm.xt[e + 2][d] = cv[k].z;
+      sm.xt[e + 3][d] = cv[k].w;
     }
   }
   // ridge = trace / D, added to the staged diagonal
   const float tr = wave_sum_fold(gd);
-  if ((tid & 63) == 0) sm.red[tid >> 6] = tr;
+  if (lane == 0) sm.red[w] = tr;
   __syncthreads();
   float trace = 0.0f;
 #pragma unroll
-  for (int i = 0; i < kSolveThreads / 64; ++i) trace += sm.red[i];
+  for (int i = 0; i < NW; ++i) trace += sm.red[i];
   const float ridge = trace / (float)D;
   if (tid < D) sm.a[tid][tid] = gd + ridge;
-  // Blocked right-looking Cholesky, PB columns a step. Wave 0 factors the
-  // panel's PB x PB diagonal block in registers (lane l holds row jb + l;
-  // the pivot and the multipliers L[jb + c2][j] come from their lanes by
-  // readlane); then thread t solves row jb + PB + t of the panel against
-  // it, column by column; then every thread applies the rank-PB update to
-  // 4 x 4 tiles of the trailing lower triangle from float4 rows (the upper
-  // triangle is never read, so diagonal tiles are updated whole). Each
-  // element sees the operations of the unblocked factorization in the same
-  // order: one fp32 FMA per earlier column, in column order, then the
-  // scaling by its column's pivot. Pivots are taken by v_rsq_f32 (about
-  // 1 ulp): L[j][j] = pivot * rsq(pivot), and every division by L[j][j],
-  // here and in the substitutions, is a product with rsq(pivot) (kept in
-  // sm.inv); these ulp-level differences sit far below the bf16 rounding of
-  // the result.
-  constexpr int PB = kSolvePanel;
-  static_assert(D % PB == 0 && PB <= 64, "panel layout");
+  __syncthreads();
   int bad = 0;
-  const int lane = tid & 63;
-  for (int jb = 0; jb < D; jb += PB) {
-    __syncthreads();
-    if (tid < 64) {
-      float pr[PB];
-      const int rowk = jb + lane;
-#pragma unroll
-      for (int c = 0; c < PB; ++c) pr[c] = lane < PB ? sm.a[rowk][jb + c] : 0.0f;
-#pragma unroll
-      for (int c = 0; c < PB; ++c) {
-        const int j = jb + c;
-        const float piv = read_lane(pr[c], c);           // row j: lane c
-        if (!(piv > 0.0f)) bad = bad ? bad : j + 1;
-        const float rj = __builtin_amdgcn_rsqf(piv);
-        if (lane > c) pr[c] = pr[c] * rj;
-        if (lane == c) pr[c] = piv * rj;
-        if (lane == 0) sm.inv[j] = rj;
-#pragma unroll
-        for (int c2 = c + 1; c2 < PB; ++c2) {
-          const float f = read_lane(pr[c], c2);          // L[jb + c2][j]
-          if (lane >= c2) pr[c2] = fmaf(-pr[c], f, pr[c2]);
-        }
-      }
-      if (lane < PB) {
-#pragma unroll
-        for (int c = 0; c < PB; ++c)
-          if (c <= lane) sm.a[rowk][jb + c] = pr[c];
-      }
+  if (w == 0) bad = factor_block<LD>(&sm.a[0][0], 0, lane, bad);
+  for (int b = 0; b + 1 < NB; ++b) {
+    const int jb = 16 * b;
+    __syncthreads();                              // block b's inverse, the trailing blocks
+    // L of the rows below: A L_b^-T, a block of 16 rows a wave
+    for (int i = b + 1 + w; i < NB; i += NW) {
+      float* rows = &sm.a[16 * i][jb];
+      // sub_product subtracts: the negated product
+      const f32x4 v = sub_product<LD, true>(rows, &sm.a[jb][jb], f32x4{}, lane);
+      solve_wave_sync();
+      store_block<LD>(rows, -v, lane);
     }
     __syncthreads();
-    if (tid < D - jb - PB) {
-      const int rowk = jb + PB + tid;
-      float l[PB];
-#pragma unroll
-      for (int q = 0; q < PB / 4; ++q) {
-        const float4 v = *(const float4*)&sm.a[rowk][jb + 4 * q];
-        l[4 * q] = v.x; l[4 * q + 1] = v.y; l[4 * q + 2] = v.z; l[4 * q + 3] = v.w;
+    // Trailing triangle; wave 0 goes on to factor the next diagonal block.
+    const int n = NB - 1 - b;
+    if (w == 0) {
+      float* next = &sm.a[jb + 16][jb + 16];
+      const float* row = &sm.a[jb + 16][jb];
+      const f32x4 v = sub_product<LD, true>(row, row, load_block<LD>(next, lane), lane);
+      store_block<LD>(next, v, lane);
+      solve_wave_sync();
+      bad = factor_block<LD>(next, jb + 16, lane, bad);
+    } else {
+      for (int t = w; t < n * (n + 1) / 2; t += NW - 1) {   // t = 0 is wave 0's
+        int i = 0;
+        while ((i + 1) * (i + 2) / 2 <= t) ++i;
+        const int j = t - i * (i + 1) / 2;
+        float* dst = &sm.a[jb + 16 + 16 * i][jb + 16 + 16 * j];
+        store_block<LD>(dst, sub_product<LD, true>(&sm.a[jb + 16 + 16 * i][jb],
+                                                   &sm.a[jb + 16 + 16 * j][jb],
+                                                   load_block<LD>(dst, lane), lane), lane);
       }
-#pragma unroll
-      for (int c = 0; c < PB; ++c) {
-        float v = l[c];
-#pragma unroll
-        for (int u = 0; u < c; ++u) v = fmaf(-l[u], sm.a[jb + c][jb + u], v);
-        l[c] = v * sm.inv[jb + c];
-      }
-#pragma unroll
-      for (int q = 0; q < PB / 4; ++q)
-        *(float4*)&sm.a[rowk][jb + 4 * q] = make_float4(l[4 * q], l[4 * q + 1], l[4 * q + 2],
-                                                        l[4 * q + 3]);
-    }
-    __syncthreads();
-    const int r0 = jb + PB, nt = (D - r0) / 4;
-    for (int t = tid; t < nt * (nt + 1) / 2; t += kSolveThreads) {
-      int kt = (int)((__builtin_sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
-      while (kt * (kt + 1) / 2 > t) --kt;
-      while ((kt + 1) * (kt + 2) / 2 <= t) ++kt;
-      const int ct = t - kt * (kt + 1) / 2;
-      const int k0 = r0 + 4 * kt, c0 = r0 + 4 * ct;
-      float4 acc[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = *(const float4*)&sm.a[k0 + i][c0];
-#pragma unroll
-      for (int q = 0; q < PB / 4; ++q) {
-        float4 lk[4], lc[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          lk[i] = *(const float4*)&sm.a[k0 + i][jb + 4 * q];
-          lc[i] = *(const float4*)&sm.a[c0 + i][jb + 4 * q];
-        }
-        // column jb + 4q + s: acc[i][j] -= L[k0 + i][.] * L[c0 + j][.]
-        const float lks[4][4] = {{lk[0].x, lk[1].x, lk[2].x, lk[3].x},
-                                 {lk[0].y, lk[1].y, lk[2].y, lk[3].y},
-                                 {lk[0].z, lk[1].z, lk[2].z, lk[3].z},
-                                 {lk[0].w, lk[1].w, lk[2].w, lk[3].w}};
-        const float4 lcs[4] = {make_float4(lc[0].x, lc[1].x, lc[2].x, lc[3].x),
-                               make_float4(lc[0].y, lc[1].y, lc[2].y, lc[3].y),
-                               make_float4(lc[0].z, lc[1].z, lc[2].z, lc[3].z),
-                               make_float4(lc[0].w, lc[1].w, lc[2].w, lc[3].w)};
-#pragma unroll
-        for (int sidx = 0; sidx < 4; ++sidx) sub_outer(acc, lks[sidx], lcs[sidx]);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *(float4*)&sm.a[k0 + i][c0] = acc[i];
     }
   }
   __syncthreads();
   if (p.info && tid == 0) p.info[mat] = bad;
-  // Forward (L Y = X) then back (L^T X = Y) substitution, PB rows a step:
-  // thread e solves the step's rows of column e, then every thread removes
-  // them from a 4 x 4 tile of the remaining rows (one FMA per solved row, in
-  // row order); two barriers a step.
-  constexpr int NCT = D / 4;
-  for (int ib = 0; ib < D; ib += PB) {
-    if (tid < D) {
-      const int e = tid;
-      float y[PB];
-#pragma unroll
-      for (int t = 0; t < PB; ++t) {
-        float v = sm.x[ib + t][e];
-#pragma unroll
-        for (int u = 0; u < t; ++u) v = fmaf(-sm.a[ib + t][ib + u], y[u], v);
-        y[t] = v * sm.inv[ib + t];
-        sm.x[ib + t][e] = y[t];
-      }
-    }
-    __syncthreads();
-    const int r0 = ib + PB;
-    for (int t = tid; t < (D - r0) / 4 * NCT; t += kSolveThreads) {
-      const int k0 = r0 + 4 * (t / NCT), e0 = 4 * (t % NCT);
-      float4 acc[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = *(const float4*)&sm.x[k0 + i][e0];
-#pragma unroll
-      for (int q = 0; q < PB / 4; ++q) {
-        float4 lk[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) lk[i] = *(const float4*)&sm.a[k0 + i][ib + 4 * q];
-        const float lks[4][4] = {{lk[0].x, lk[1].x, lk[2].x, lk[3].x},
-                                 {lk[0].y, lk[1].y, lk[2].y, lk[3].y},
-                                 {lk[0].z, lk[1].z, lk[2].z, lk[3].z},
-                                 {lk[0].w, lk[1].w, lk[2].w, lk[3].w}};
-#pragma unroll
-        for (int sidx = 0; sidx < 4; ++sidx)
-          sub_outer(acc, lks[sidx], *(const float4*)&sm.x[ib + 4 * q + sidx][e0]);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *(float4*)&sm.x[k0 + i][e0] = acc[i];
-    }
-    __syncthreads();
+  // Forward (Y^T L^T = X^T) and back (Z^T L = Y^T): this wave's 16 rows of
+  // X^T, 16 columns a step, all earlier columns subtracted first.
+  float* const x = &sm.xt[16 * w][0];
+#pragma unroll 1
+  for (int b = 0; b < NB; ++b) {
+    f32x4 v = load_block<LD>(x + 16 * b, lane);
+    for (int j = 0; j < b; ++j) v = sub_product<LD, true>(x + 16 * j, &sm.a[16 * b][16 * j], v, lane);
+    store_block<LD>(x + 16 * b, v, lane);
+    solve_wave_sync();
+    v = sub_product<LD, true>(x + 16 * b, &sm.a[16 * b][16 * b], f32x4{}, lane);
+    solve_wave_sync();
+    store_block<LD>(x + 16 * b, -v, lane);
+    solve_wave_sync();
   }
-  for (int ib = D - PB; ib >= 0; ib -= PB) {
-    if (tid < D) {
-      const int e = tid;
-      float xv[PB];
-#pragma unroll
-      for (int t = PB - 1; t >= 0; --t) {
-        float v = sm.x[ib + t][e];
-#pragma unroll
-        for (int u = t + 1; u < PB; ++u) v = fmaf(-sm.a[ib + u][ib + t], xv[u], v);
-        xv[t] = v * sm.inv[ib + t];
-        sm.x[ib + t][e] = xv[t];
-      }
-    }
-    __syncthreads();
-    for (int t = tid; t < ib / 4 * NCT; t += kSolveThreads) {
-      const int k0 = 4 * (t / NCT), e0 = 4 * (t % NCT);
-      float4 acc[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] = *(const float4*)&sm.x[k0 + i][e0];
-#pragma unroll
-      for (int t2 = 0; t2 < PB; ++t2) {
-        // row ib + t2 of L, columns k0 .. k0 + 3 (L^T[k][ib + t2])
-        const float4 lr = *(const float4*)&sm.a[ib + t2][k0];
-        const float l4[4] = {lr.x, lr.y, lr.z, lr.w};
-        sub_outer(acc, l4, *(const float4*)&sm.x[ib + t2][e0]);
-      }
-#pragma unroll
-      for (int i = 0; i < 4; ++i) *(float4*)&sm.x[k0 + i][e0] = acc[i];
-    }
-    __syncthreads();
+#pragma unroll 1
+  for (int b = NB - 1; b >= 0; --b) {
+    f32x4 v = load_block<LD>(x + 16 * b, lane);
+    for (int j = NB - 1; j > b; --j)
+      v = sub_product<LD, false>(x + 16 * j, &sm.a[16 * j][16 * b], v, lane);
+    store_block<LD>(x + 16 * b, v, lane);
+    solve_wave_sync();
+    v = sub_product<LD, false>(x + 16 * b, &sm.a[16 * b][16 * b], f32x4{}, lane);
+    solve_wave_sync();
+    store_block<LD>(x + 16 * b, -v, lane);
+    solve_wave_sync();
   }
-  if (p.out_f32) {
-    float* out = p.out_f32 + (size_t)mat * D * D;
-    for (int i = tid; i < D * D; i += kSolveThreads) out[i] = sm.x[i / D][i % D];
+  if (p.out_f32 || !p.to_slots) {                 // rows d, columns e: other waves' rows
+    __syncthreads();
+    for (int i = tid; i < D * D; i += NT) {
+      const float v = sm.xt[i % D][i / D];
+      if (p.out_f32)
+        p.out_f32[(size_t)mat * D * D + i] = v;
+      else
+        p.out[(size_t)mat * D * D + i] = f2bf(v);
+    }
     return;
   }
-  if (!p.to_slots) {
-    bf16_t* out = p.out + (size_t)mat * D * D;
-    for (int i = tid; i < D * D; i += kSolveThreads) out[i] = f2bf(sm.x[i / D][i % D]);
-    return;
-  }
-  // C^T into a bank (fine) or page slot: dst[e][d] = X[d][e]
+  // C^T into a bank (fine) or page slot: this wave's rows e, 8 channels a lane
   const int b = (mat / p.H) % p.B, h = mat % p.H;
   const int slot = p.to_slots == 1 ? p.first_slot + blk : (p.fine_first + blk) / p.group;
-  bf16_t* dst = p.out + (((size_t)b * p.H + h) * p.cap + slot) * D * D;
-  for (int i = tid; i < D * D; i += kSolveThreads) dst[i] = f2bf(sm.x[i % D][i / D]);
+  bf16_t* dst = p.out + (((size_t)b * p.H + h) * p.cap + slot) * D * D + 16 * w * D;
+  for (int i = lane; i < 2 * D; i += 64) {
+    const float* src = x + (8 * i / D) * LD + 8 * i % D;
+    const float4 u = *(const float4*)src, v = *(const float4*)(src + 4);
+    uint4 o;
+    o.x = pack_bf16x2(u.x, u.y);
+    o.y = pack_bf16x2(u.z, u.w);
+    o.z = pack_bf16x2(v.x, v.y);
+    o.w = pack_bf16x2(v.z, v.w);
+    *(uint4*)(dst + 8 * i) = o;
+  }
 }
 
 template <int D>
@@ -645,10 +619,10 @@ hipError_t launch_association_solve(const AssocSolveParams& p, int head_dim, hip
       attr = true;
     }
     hipLaunchKernelGGL(association_solve_kernel<128>, dim3((unsigned)p.count),
-                       dim3(kSolveThreads), bytes, s, p);
+                       dim3(kSolveThreads<128>), bytes, s, p);
   } else if (head_dim == 64) {
     hipLaunchKernelGGL(association_solve_kernel<64>, dim3((unsigned)p.count),
-                       dim3(kSolveThreads), sizeof(SolveSmem<64>), s, p);
+                       dim3(kSolveThreads<64>), sizeof(SolveSmem<64>), s, p);
   } else {
     return hipErrorInvalidValue;
   }

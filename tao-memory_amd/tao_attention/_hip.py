@@ -75,6 +75,7 @@ class StreamCfg(ctypes.Structure):
 
 PLAN_HEADER = 16
 PLAN_ATTN_TILES = 1
+PLAN_WRITES = 2
 
 
 def without_attention(plan):

@@ -38,7 +38,14 @@ from .config import TaoConfig
 
 DEFAULT_CONFIG = TaoConfig()
 _QTILE = 256
-_STATS_CAP = 8          # blocks per statistics pass of the regularized writer
+_STATS_CAP = 8          # blocks per statistics pass of a seal (the state's own scratch)
+
+
+def stats_blocks(blocks, batch, heads):
+    """Blocks per statistics pass of a call that seals `blocks`: a pass's
+    solves are one serial chain each, so a pass holds at least one system for
+    each of the 256 CUs (17 blocks of 8 heads: one pass, not three)."""
+    return min(blocks, max(_STATS_CAP, -(-256 // (batch * heads))))
 # Fine writers the stream implements: the softmax writer and the regularized
 # association writer (same z and read, association value matrices).
 _STREAM_WRITERS = ("softmax", "regularized_association", "feature_mass_association",
@@ -79,7 +86,8 @@ def _zeroed_views(device, specs):
 class _DeviceState:
     """Device buffers of one state and the C-ABI view of them."""
 
-    def __init__(self, config, batch, heads, head_dim, device, fine_cap, plan_words=4096):
+    def __init__(self, config, batch, heads, head_dim, device, fine_cap, plan_words=4096,
+                 stats_cap=_STATS_CAP):
         self.config = config
         self.B, self.H, self.D = batch, heads, head_dim
         self.device = device
@@ -117,16 +125,20 @@ class _DeviceState:
                      None if pending is None else (pending[0], f32),
                      None if pending is None else (pending[1], f32)])
         self.stats = None
-        if self.association:
-            self.stats = torch.empty((2, _STATS_CAP * batch, heads, head_dim, head_dim),
-                                     dtype=f32, device=device)
-        elif self.feature:
-            words = _STATS_CAP * batch * heads * head_dim
-            self.stats = torch.empty(words * (2 * head_dim + 1), dtype=f32, device=device)
+        self.stats_cap = stats_cap
+        if self.association or self.feature:
+            self.stats = self.stats_scratch(stats_cap)
         self.generation = next(_SERIAL)   # renewed whenever the buffers move
         self.fine_cap = 0
         self.plan_words = max(plan_words, 4096)
         self._allocate(fine_cap, copy_fines=0)
+
+    def stats_scratch(self, blocks):
+        """fp32 scratch for the statistics of `blocks` blocks (gram, cross and,
+        for the feature writers, the feature mass)."""
+        words = blocks * self.B * self.H * self.D
+        return torch.empty(words * (2 * self.D + (1 if self.feature else 0)),
+                           dtype=torch.float32, device=self.device)
 
     def _allocate(self, fine_cap, copy_fines):
         cfg = self.config
@@ -205,10 +217,10 @@ class _DeviceState:
         if self.association:
             st.pending_gram = self.pending_gram.data_ptr()
             st.pending_cross = self.pending_cross.data_ptr()
-            st.stats, st.stats_cap = self.stats.data_ptr(), _STATS_CAP
+            st.stats, st.stats_cap = self.stats.data_ptr(), self.stats_cap
         if self.feature:
             st.fine_writer, st.fine_mass = self.feature, self.fine_mass.data_ptr()
-            st.stats, st.stats_cap = self.stats.data_ptr(), _STATS_CAP
+            st.stats, st.stats_cap = self.stats.data_ptr(), self.stats_cap
             st.pending_gram = self.pending_gram.data_ptr()
             st.pending_cross = self.pending_cross.data_ptr()
         st.workspace = self.workspace.data_ptr()
@@ -554,11 +566,20 @@ class StreamCache:
                 pools.coarse_first = info["coarse_first"]
                 pools.coarse_count = info["coarse_count"]
                 keep.append(coarse_pool)
+        struct = dev.struct
+        if dev.stats is not None:
+            # Statistics of the call's own width, on scratch of the call.
+            blocks = stats_blocks(int(plan_np[_hip.PLAN_WRITES]), dev.B, dev.H)
+            if blocks > dev.stats_cap:
+                stats = dev.stats_scratch(blocks)
+                struct = _hip.StateDev.from_buffer_copy(struct)
+                struct.stats, struct.stats_cap = stats.data_ptr(), blocks
+                keep.append(stats)
         out_s = (ctypes.c_int64 * 3)(*(_hip.strides_bth(out) if out is not None else (0, 0, 0)))
         dummy = dev.workspace.data_ptr()
         with self._timed("prefill"):
             _hip.check(_hip.lib().tao_prefill(
-                ctypes.byref(dev.struct), ctypes.byref(tok), ctypes.byref(fu), plan_arr,
+                ctypes.byref(struct), ctypes.byref(tok), ctypes.byref(fu), plan_arr,
                 len(plan), ctypes.byref(pools),
                 local.data_ptr() if local is not None else dummy,
                 out.data_ptr() if out is not None else dummy, out_s, dev.stream()))

@@ -84,7 +84,7 @@ class _Workspace:
     """
 
     def __init__(self, config, b, tokens, heads, d, device):
-        from .tao_stream import _DeviceState
+        from .tao_stream import _DeviceState, _STATS_CAP, stats_blocks
 
         self.plan, self.info = plan(config, tokens)
         info = self.info
@@ -92,7 +92,10 @@ class _Workspace:
         # The same plan without its local attention (local from a plugin).
         self.plan_ext = _hip.without_attention(self.plan)
         self.plan_ext_arr = self.plan_ext.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))
-        self.dev = _DeviceState(config, b, heads, d, device, max(info["fines"], 8))
+        cap = (stats_blocks(info["fines"], b, heads) if config.fine_writer in _FEATURE_WRITERS
+               else _STATS_CAP)
+        self.dev = _DeviceState(config, b, heads, d, device, max(info["fines"], 8),
+                                stats_cap=max(cap, _STATS_CAP))
         self.dev.ensure_plan(len(self.plan))
         self.local = torch.empty((b, tokens, heads, d), dtype=torch.bfloat16, device=device)
         self.pools = _hip.PrefillPools()

@@ -424,3 +424,64 @@ def test_full_sequence_feature_writers(device, writer, width, tokens, batch, ind
     api = tao_attention(q, k, v, raw_q=rq, raw_k=rk, fusion_a=fa.to(device),
                         fusion_b=fb.to(device), alpha=0.5, config=cfg)
     assert torch.equal(api, out)
+
+
+@pytest.mark.parametrize("writer,heads,width,values", [
+    ("regularized_association", 2, 128, True),
+    ("regularized_association", 3, 64, False),
+    ("feature_mass_association", 2, 64, True),
+    ("structured_gram_association", 2, 128, True),
+])
+def test_one_statistics_pass_equals_seals_by_chunk(device, writer, heads, width, values):
+    """A call that seals more blocks than a pass of the state's own scratch
+    holds (here 12 of them at once) leaves the state of the same tokens sealed
+    a few at a time, bit for bit: the same blocks, solves and in-order sums."""
+    from tao_attention import TaoConfig, new_state, tao_attention_prefill
+    tokens = 768 + 11 * 256 + 40
+    g = torch.Generator(device=device).manual_seed(width + heads)
+    xs = [torch.randn(1, tokens, heads, width, generator=g, device=device).to(torch.bfloat16)
+          for _ in range(5)]
+    fa, fb = (torch.randn(heads, width, 3, generator=g, device=device) * 0.02 for _ in range(2))
+    config = TaoConfig(fine_writer=writer, coarse_index_only=not values)
+    snaps = []
+    for step in (tokens, 700):
+        state = new_state(0, config)
+        for at in range(0, tokens, step):
+            cut = [x[:, at:at + step].contiguous() for x in xs]
+            _, state = tao_attention_prefill(*cut[:3], raw_q=cut[3], raw_k=cut[4], fusion_a=fa,
+                                             fusion_b=fb, alpha=0.5, state=state,
+                                             position=state.get_pos())
+        snaps.append(state.export())
+
+    def leaves(x):
+        if torch.is_tensor(x):
+            return [x]
+        if isinstance(x, dict):
+            return [t for k in sorted(x, key=str) for t in leaves(x[k])]
+        if isinstance(x, (list, tuple)):
+            return [t for y in x for t in leaves(y)]
+        return []
+
+    one, many = (leaves(s) for s in snaps)
+    assert len(one) == len(many) and len(one) > 8
+    for a, b in zip(one, many):
+        assert a.shape == b.shape and torch.equal(a, b)
+
+
+@pytest.mark.parametrize("width", [64, 128])
+def test_association_solve_against_float64(device, width):
+    """The solve to its own rounding: fp32 elimination of systems whose
+    condition number is at most width + 1 (the ridge is the mean eigenvalue),
+    then one bf16 rounding (2^-9 of each entry); 2e-5 of the largest entry
+    covers the fp32 part (about (width + 1) 2^-24 times a small factor)."""
+    from tao_attention.association_writer import association_matrix, association_statistics
+    g = torch.Generator(device=device).manual_seed(width)
+    k, v = (torch.randn(5, 256, 3, width, generator=g, device=device).to(torch.bfloat16)
+            for _ in range(2))
+    gram, cross = association_statistics(k, v)
+    got = association_matrix(gram, cross).double()
+    ridge = gram.double().diagonal(dim1=-2, dim2=-1).mean(-1)
+    system = gram.double() + ridge[..., None, None] * torch.eye(width, device=device).double()
+    want = torch.linalg.solve(system, cross.double())
+    bound = want.abs() * 2 ** -8 + 2e-5 * want.abs().amax((-1, -2), keepdim=True)
+    assert bool(((got - want).abs() <= bound).all())
