@@ -1553,7 +1553,7 @@ struct TrainBwdLayout {
   size_t pstats, psol_y, psol_w, psgram, dpc;
   // feature writers: masses, d mass, structured adjoints, d z of the fines'
   // and pages' descriptors, the mixture weights and d masses per query rank
-  size_t fmass, fdmass, fdsq, fdms, fdz, fdpz, wv, dmv, pdsq, pdms;
+  size_t fmass, fdmass, fdsq, fdms, fdz, fdpz, wv, dmv, pdsq, pdms, mix_part;
   size_t zero_begin, zero_end;                                  // accumulators to clear
   size_t total;
   int n_tiles, v_max;
@@ -1624,6 +1624,11 @@ TrainBwdLayout train_bwd_layout(const tao_state_dev* st, int64_t tokens, int fin
       l.dmv = take(rows * tao::kMixMaxRank * 4);
       l.pdsq = take(pvec);
       l.pdms = take(pvec);
+      const int keep = st->local_keep, ft = st->fine_tokens, np = (int)pages;
+      const size_t fparts = (size_t)fines * tao::mix_splits(fines, (int)BH, (int)T, keep + ft);
+      const size_t pparts =
+          pages * tao::mix_splits(np, (int)BH, (int)T, keep + st->coarse_group * ft);
+      l.mix_part = take(std::max(fparts, pparts) * BH * (mat + (size_t)D * 4));
     }
   }
   l.total = off;
@@ -1662,6 +1667,8 @@ hipError_t feature_read_backward(const tao_state_dev* st, const tao_prefill_pool
   mx.keep = st->local_keep;
   mx.group = G;
   mx.first_query = st->local_keep + st->fine_tokens;
+  mx.splits = tao::mix_splits(mx.n_items, B * H, T, mx.first_query);
+  mx.part = (float*)(ws + l.mix_part);
   e = tao::launch_mix_bwd(mx, D, s);
   if (e != hipSuccess || !st->page_c || fines / G < 1) return e;
   tao::MixBwdParams mc = mx;
@@ -1675,6 +1682,7 @@ hipError_t feature_read_backward(const tao_state_dev* st, const tao_prefill_pool
   mc.dz = (float*)(ws + l.fdpz);
   mc.n_items = fines / G;
   mc.first_query = st->local_keep + G * st->fine_tokens;
+  mc.splits = tao::mix_splits(mc.n_items, B * H, T, mc.first_query);
   return tao::launch_mix_bwd(mc, D, s);
 }
 

@@ -263,15 +263,21 @@ __global__ __launch_bounds__(2 * D) void mix_query_bwd_kernel(MixBwdParams p) {
 }
 
 // ---------------------------------------------------------------------------
-// Item-major pass. One 256-thread workgroup per (item, batch, head): over the
+// Item-major pass. 256-thread workgroups per (item, batch, head): over the
 // queries that can read the item, in chunks of 32, dC^T[e][d] = sum_q
 // dout[q][e] r(w_q h[q][d]) (A = dout^T chunk [e][q], B = channel^T chunk
 // [d][q], both staged in LDS; only queries that read the item contribute)
-// and dz[d] = exp(z[d]) sum_q dmass_q h[q][d].
+// and dz[d] = exp(z[d]) sum_q dmass_q h[q][d]. A chunk is three dependent
+// memory round trips (selection, weights, rows) for 4 MFMAs a wave, so the
+// pass is bound by how many chunks are in flight: the chunks of an item are
+// dealt to p.splits workgroups, whose partial sums mix_item_sum_kernel adds
+// in split order. B1 T3001 H8 D64 (9 fines, 1 page): 280 us a pass with one
+// workgroup per item (72 and 8 of them), 28 us now, the sum included.
 template <int D>
 struct MixISmem {
   bf16_t xt[D][40];                   // dout^T [e][q]
   bf16_t yt[D][40];                   // channel^T [d][q]
+  bf16_t hq[32][D];                   // h rows
   float wq[32], dmq[32];
 };
 
@@ -281,7 +287,7 @@ __global__ __launch_bounds__(256) void mix_item_bwd_kernel(MixBwdParams p) {
   __shared__ MixISmem<D> sm;
   const int BH = p.B * p.H;
   const int bh = blockIdx.x % BH;
-  const int item = blockIdx.x / BH;
+  const int item = blockIdx.x / BH % p.n_items, split = blockIdx.x / BH / p.n_items;
   const int b = bh / p.H, h = bh % p.H;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int li = lane & 31, hl = lane >> 5;
@@ -297,7 +303,7 @@ __global__ __launch_bounds__(256) void mix_item_bwd_kernel(MixBwdParams p) {
     for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
   float dzacc = 0.0f;
   auto row_of = [&](int q) { return (((size_t)b * p.T + q) * p.H + h); };
-  for (int c0 = q_begin; c0 < p.T; c0 += 32) {
+  for (int c0 = q_begin + 32 * split; c0 < p.T; c0 += 32 * p.splits) {
     int reads = 0;
     if (tid < 32) {
       const int q = c0 + tid;
@@ -329,19 +335,21 @@ __global__ __launch_bounds__(256) void mix_item_bwd_kernel(MixBwdParams p) {
       const int q = i / D, e = i % D;
       const int tq = c0 + q;
       const bool live = tq < p.T && sm.wq[q] != 0.0f;
-      const size_t row = row_of(live ? tq : c0);
+      const bool moved = tq < p.T && sm.dmq[q] != 0.0f;
+      const size_t row = row_of(live || moved ? tq : c0);
+      const bf16_t hv = p.h[row * D + e];
+      sm.hq[q][e] = hv;
       sm.xt[e][q] = f2bf(live ? p.dout[row * D + e] : 0.0f);
-      sm.yt[e][q] = f2bf(live ? sm.wq[q] * bf2f(p.h[row * D + e]) : 0.0f);
-    }
-    if (tid < D) {
-      float s = 0.0f;
-      for (int q = 0; q < 32; ++q) {
-        const int tq = c0 + q;
-        if (tq < p.T && sm.dmq[q] != 0.0f) s += sm.dmq[q] * bf2f(p.h[row_of(tq) * D + tid]);
-      }
-      dzacc += s;
+      sm.yt[e][q] = f2bf(live ? sm.wq[q] * bf2f(hv) : 0.0f);
     }
     __syncthreads();
+    if (tid < D) {
+      float s = 0.0f;
+#pragma unroll
+      for (int q = 0; q < 32; ++q)
+        if (c0 + q < p.T && sm.dmq[q] != 0.0f) s += sm.dmq[q] * bf2f(sm.hq[q][tid]);
+      dzacc += s;
+    }
 #pragma unroll
     for (int t = 0; t < TPW; ++t) {
       const int tile = w * TPW + t;
@@ -356,7 +364,9 @@ __global__ __launch_bounds__(256) void mix_item_bwd_kernel(MixBwdParams p) {
     }
     __syncthreads();
   }
-  float* out = p.dmat + ((size_t)bh * p.n_items + item) * D * D;
+  const size_t mat = (size_t)bh * p.n_items + item;
+  const size_t mats = (size_t)BH * p.n_items;
+  float* out = p.splits > 1 ? p.part + (split * mats + mat) * (D * D + D) : p.dmat + mat * D * D;
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
     const int tile = w * TPW + t;
@@ -370,8 +380,29 @@ __global__ __launch_bounds__(256) void mix_item_bwd_kernel(MixBwdParams p) {
     }
   }
   if (tid < D) {
-    const float ez = __expf(bf2f(p.z[((size_t)bh * p.cap + item) * D + tid]));
-    p.dz[((size_t)bh * p.n_items + item) * D + tid] = dzacc * ez;
+    if (p.splits > 1)
+      out[D * D + tid] = dzacc;
+    else
+      p.dz[mat * D + tid] = dzacc * __expf(bf2f(p.z[((size_t)bh * p.cap + item) * D + tid]));
+  }
+}
+
+// Sum of the splits' partials: a thread per element.
+template <int D>
+__global__ __launch_bounds__(256) void mix_item_sum_kernel(MixBwdParams p) {
+  constexpr int N = D * D + D;
+  const size_t mats = (size_t)p.B * p.H * p.n_items;
+  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= mats * N) return;
+  const size_t mat = i / N;
+  const int k = (int)(i % N);
+  float s = 0.0f;
+  for (int v = 0; v < p.splits; ++v) s += p.part[v * mats * N + i];
+  if (k < D * D) {
+    p.dmat[mat * D * D + k] = s;
+  } else {
+    const size_t bh = mat / p.n_items, item = mat % p.n_items;
+    p.dz[mat * D + k - D * D] = s * __expf(bf2f(p.z[(bh * p.cap + item) * D + k - D * D]));
   }
 }
 
@@ -584,15 +615,20 @@ hipError_t launch_mix_bwd(const MixBwdParams& p, int head_dim, hipStream_t s) {
                  p.qsel_words > 16))
     return hipErrorInvalidValue;
   if (!p.qsel && p.n_items > kMixMaxRank) return hipErrorInvalidValue;
+  if (p.splits < 1 || (p.splits > 1 && !p.part)) return hipErrorInvalidValue;
   const int BH = p.B * p.H;
   const dim3 qgrid((unsigned)(((p.T + 31) / 32) * BH));
-  const dim3 igrid((unsigned)(p.n_items * BH));
+  const dim3 igrid((unsigned)(p.n_items * BH * p.splits));
+  const size_t sums = (size_t)BH * p.n_items * head_dim * (head_dim + 1);
+  const dim3 sgrid((unsigned)((sums + 255) / 256));
   if (head_dim == 128) {
     hipLaunchKernelGGL(mix_query_bwd_kernel<128>, qgrid, dim3(256), 0, s, p);
     hipLaunchKernelGGL(mix_item_bwd_kernel<128>, igrid, dim3(256), 0, s, p);
+    if (p.splits > 1) hipLaunchKernelGGL(mix_item_sum_kernel<128>, sgrid, dim3(256), 0, s, p);
   } else if (head_dim == 64) {
     hipLaunchKernelGGL(mix_query_bwd_kernel<64>, qgrid, dim3(128), 0, s, p);
     hipLaunchKernelGGL(mix_item_bwd_kernel<64>, igrid, dim3(256), 0, s, p);
+    if (p.splits > 1) hipLaunchKernelGGL(mix_item_sum_kernel<64>, sgrid, dim3(256), 0, s, p);
   } else {
     return hipErrorInvalidValue;
   }

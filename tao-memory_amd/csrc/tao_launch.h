@@ -557,7 +557,18 @@ struct MixBwdParams {
   int n_items;            // visible fines, or completed pages
   int B, H, T, ft, keep, group;
   int first_query;        // first token with this read (first_fine or first_coarse)
+  int splits;             // workgroups an item's queries are dealt to (mix_splits)
+  float* part;            // splits > 1: [splits][B*H*n_items][D*D + D] partial sums
 };
+// Workgroups per item of the item-major pass: about 1,024 over all items (four
+// a CU), at most 16 and at most one per 32-query chunk of the first item.
+inline int mix_splits(int items, int bh, int T, int first_query) {
+  if (items <= 0 || T <= first_query) return 1;
+  const int chunks = (T - first_query + 31) / 32;
+  const int want = 1024 / (items * bh);
+  const int n = want < 16 ? want : 16;
+  return n < 1 ? 1 : n < chunks ? n : chunks;
+}
 constexpr int kMixMaxRank = 64;      // items one query reads
 constexpr int kMixMaxItems = 512;    // fine ids a query block can select
 hipError_t launch_mix_bwd(const MixBwdParams& p, int head_dim, hipStream_t s);

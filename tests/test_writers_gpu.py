@@ -485,3 +485,25 @@ def test_association_solve_against_float64(device, width):
     want = torch.linalg.solve(system, cross.double())
     bound = want.abs() * 2 ** -8 + 2e-5 * want.abs().amax((-1, -2), keepdim=True)
     assert bool(((got - want).abs() <= bound).all())
+
+
+def test_feature_backward_is_the_same_for_any_number_of_heads(device):
+    """d raw_k and d v of one head alone (its items' queries dealt to sixteen
+    workgroups each) and as the first of 64 heads (a workgroup per item):
+    fp32 sums in another order, then one bf16 rounding (2^-8 of an entry, and
+    1e-3 of the largest for the fp32 chains behind it)."""
+    from tao_attention import TaoConfig, tao_attention
+    g = torch.Generator(device=device).manual_seed(5)
+    config = TaoConfig(fine_writer="feature_mass_association")
+    xs = [torch.randn(1, 5100, 64, 64, generator=g, device=device).to(torch.bfloat16)
+          for _ in range(6)]
+    fa, fb = (torch.randn(64, 64, 3, generator=g, device=device) * 0.02 for _ in range(2))
+    grads = []
+    for heads in (64, 1):
+        leaves = [x[:, :, :heads].contiguous().requires_grad_(True) for x in xs[:5]]
+        out = tao_attention(*leaves[:3], raw_q=leaves[3], raw_k=leaves[4], fusion_a=fa[:heads],
+                            fusion_b=fb[:heads], alpha=0.5, config=config)
+        got = torch.autograd.grad(out, leaves, xs[5][:, :, :heads].contiguous())
+        grads.append([x[:, :, :1].float() for x in got])
+    for a, b in zip(*grads):
+        assert bool(((a - b).abs() <= 2 ** -8 * b.abs() + 1e-3 * b.abs().max()).all())
