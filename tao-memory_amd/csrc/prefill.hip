@@ -126,9 +126,11 @@ constexpr int kGroupThreads = 64 * kGroupWaves;
 constexpr int kBitWords = kMaxFineIds / 32;
 constexpr int kMaxUnion = kGroupWaves * kMaxM;
 
-template <int D>
+template <int D, bool COARSE>
 struct GroupSmem {
   union {
+    // Epilogue: each wave's fine (and coarse) values of its 32 queries.
+    bf16_t tile[kGroupWaves][COARSE ? 2 : 1][32 * D];
     struct {
       uint32_t bits[kBitWords];
       int pre[kBitWords];
@@ -163,6 +165,12 @@ TAO_DEV uint4 slice_weights(const uint4& pw, const uint4& sw) {
                     pack_bf16x2(a[4] * b[4], a[5] * b[5]), pack_bf16x2(a[6] * b[6], a[7] * b[7]));
 }
 
+// acc + a . b over a bf16 pair, in fp32.
+TAO_DEV float dot_pair(uint32_t a, uint32_t b, float acc) {
+  return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, a),
+                                         __builtin_bit_cast(bf16x2, b), acc, false);
+}
+
 // One 16-byte slice of C^T scaled by the slice's weights, rounded to bf16.
 TAO_DEV uint4 scale_slice(const uint4& c, const uint4& wr) {
   float a[8], b[8];
@@ -171,6 +179,11 @@ TAO_DEV uint4 scale_slice(const uint4& c, const uint4& wr) {
   return make_uint4(pack_bf16x2(a[0] * b[0], a[1] * b[1]), pack_bf16x2(a[2] * b[2], a[3] * b[3]),
                     pack_bf16x2(a[4] * b[4], a[5] * b[5]), pack_bf16x2(a[6] * b[6], a[7] * b[7]));
 }
+
+template <int D, bool COARSE, bool STAGED>
+TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], const bf16_t* tile_f,
+                       const bf16_t* tile_c, int lane, int b, int h, int q_first, int nq,
+                       bool coarse_on);
 
 // Turn-group read: one 512-thread workgroup per (8 consecutive read tiles,
 // batch, head); wave w owns tile w (<= 32 queries sharing one route, its
@@ -200,13 +213,13 @@ TAO_DEV uint4 scale_slice(const uint4& c, const uint4& wr) {
 // every staged C^T and MFMA; the numerator and denominator of a query sum
 // exactly its selected fines (selected_read.py:156-173).
 template <int D, bool COARSE, bool PERQ, bool FEAT>
-__global__ __launch_bounds__(kGroupThreads) void read_groups_kernel(ReadTilesParams p) {
+__global__ __launch_bounds__(kGroupThreads, D == 64 && !FEAT ? 4 : 2) void read_groups_kernel(ReadTilesParams p) {
   static_assert(!FEAT || PERQ, "the group read's mixture serves per-query reads");
   constexpr int KK = D / 16, ET = D / 32, CPR = D / 8;   // k-steps, e-tiles, uint4 per row
   constexpr int CPT = D * CPR / kGroupThreads;           // C^T uint4 per thread
   static_assert(CPT == 1 || CPT == 4, "head width 64 or 128");
   static_assert(kGroupThreads % CPR == 0, "a thread's C^T chunks share one column slice");
-  __shared__ GroupSmem<D> sm;
+  __shared__ GroupSmem<D, COARSE> sm;
   const int BH = p.B * p.H;
   const int bh = blockIdx.x % BH;
   // Tiles in reverse plan order: the latest tiles read the most fines, so
@@ -317,9 +330,10 @@ __global__ __launch_bounds__(kGroupThreads) void read_groups_kernel(ReadTilesPar
   for (int t = 0; t < ET; ++t)
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
-  floatx16 acc_den;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) acc_den[i] = 0.0f;
+  // den of query li, this lane's half of the channels: the A rows against the
+  // fine's weights by bf16 pair dot products (fp32 sums) on the VALU. On the
+  // matrix core it was one product more for every two (D = 64) or four.
+  float den_part = 0.0f;
 
   const bf16_t* bank = p.bank + (size_t)bh * p.fine_cap * D * D;
   const bf16_t* sw_base = p.sw + (size_t)bh * p.fine_cap * D;
@@ -517,7 +531,7 @@ __global__ __launch_bounds__(kGroupThreads) void read_groups_kernel(ReadTilesPar
 #pragma unroll
           for (int t = 0; t < ET; ++t) {
             const bf16x8 bq = as_bf16x8(*(const uint4*)&sm.u.c[buf][32 * t + li][d0]);
-            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bq, acc[t], 0, 0, 0);
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bq, a, acc[t], 0, 0, 0);
           }
         }
         return;
@@ -531,11 +545,13 @@ __global__ __launch_bounds__(kGroupThreads) void read_groups_kernel(ReadTilesPar
 #pragma unroll
         for (int t = 0; t < ET; ++t) {
           const bf16x8 bq = as_bf16x8(*(const uint4*)&sm.u.c[buf][32 * t + li][d0]);
-          acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bq, acc[t], 0, 0, 0);
+          acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bq, a, acc[t], 0, 0, 0);
         }
-        // den: the same A against the fine's weights in every column.
-        const bf16x8 wq = as_bf16x8(*(const uint4*)&sm.wr[buf][d0]);
-        acc_den = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, wq, acc_den, 0, 0, 0);
+        const uint4 wq = *(const uint4*)&sm.wr[buf][d0];
+        den_part = dot_pair(av.x, wq.x, den_part);
+        den_part = dot_pair(av.y, wq.y, den_part);
+        den_part = dot_pair(av.z, wq.z, den_part);
+        den_part = dot_pair(av.w, wq.w, den_part);
       }
     };
     uint4 a0, a1, a2, a3, ap, as, b0, b1, b2, b3, bp, bs;
@@ -586,28 +602,47 @@ __global__ __launch_bounds__(kGroupThreads) void read_groups_kernel(ReadTilesPar
     }
     return part + __shfl_xor(part, 32, 64);
   };
-  float totc = 0.0f;
-  if constexpr (FEAT && COARSE) {
-    if (coarse_on)
-      for (int pg = 0; pg < cpages; ++pg) totc += page_mass(pg);
+  // The wave's fine and coarse values go through its LDS tiles, so the fusion
+  // runs on rows: eight channels a lane, 16-byte loads and stores. A lane of
+  // the accumulators holds query li and channels e = 32 t + 8 g + 4 hl + j
+  // (accumulator 4 g + j). Fused an element a lane from 2-byte loads, the
+  // epilogue was 59 of 132 us at B2 T8192 H12 D64.
+  auto unit_at = [&](int row, int unit) __attribute__((always_inline)) {
+    return row * D + 8 * (unit ^ (row % CPR));
+  };
+  bf16_t* const tile_f = sm.u.tile[w][0];
+  bf16_t* const tile_c = sm.u.tile[w][COARSE ? 1 : 0];
+  auto put = [&](bf16_t* tile, int t, const floatx16& v) __attribute__((always_inline)) {
+#pragma unroll
+    for (int g = 0; g < 4; ++g)
+      *(uint2*)&tile[unit_at(li, 4 * t + g) + 4 * hl] = make_uint2(
+          pack_bf16x2(v[4 * g], v[4 * g + 1]), pack_bf16x2(v[4 * g + 2], v[4 * g + 3]));
+  };
+  // fine = r(r(num) / r(den)); a row without a selection (past the tile) is
+  // never stored. The feature writers' read has no denominator.
+  float den = 1.0f;
+  if constexpr (!FEAT) den = rbf(den_part + __shfl_xor(den_part, 32, 64));
+  if (p.save_den && hl == 0 && li < nq)   // FEAT: 1 keeps the adjoint's d num = d fine / den exact
+    p.save_den[((size_t)b * p.T + q_first + li) * p.H + h] = den;
+  if constexpr (!FEAT) {
+    const float inv_den = __builtin_amdgcn_rcpf(den);
+#pragma unroll
+    for (int t = 0; t < ET; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[t][i] = rbf(acc[t][i]) * inv_den;
   }
-  // One e-tile of the accumulator (called with constant t, so acc stays in
-  // registers).
-  auto emit = [&](const floatx16& av, int t) __attribute__((always_inline)) {
-    const int e = 32 * t + li;
-    float ae[3], be[3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i) {
-      ae[i] = load_param(p.fa, p.f_dtype, h * p.fa_s[0] + e * p.fa_s[1] + i * p.fa_s[2]);
-      be[i] = load_param(p.fb, p.f_dtype, h * p.fb_s[0] + e * p.fb_s[1] + i * p.fb_s[2]);
-    }
-    // coarse[q][e] = h_q . G^T[e]: A = the wave's h rows, B = G^T rows of
-    // this e-tile (k = d contiguous).
-    floatx16 cacc;
+  for (int t = 0; t < ET; ++t) put(tile_f, t, acc[t]);
+  if constexpr (COARSE) {
+    if (coarse_on) {
+      floatx16 cacc[ET];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) cacc[i] = 0.0f;
-    if constexpr (COARSE && FEAT) {
-      if (coarse_on) {
+      for (int t = 0; t < ET; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) cacc[t][i] = 0.0f;
+      if constexpr (FEAT) {
+        float totc = 0.0f;
+        for (int pg = 0; pg < cpages; ++pg) totc += page_mass(pg);
         for (int pg = 0; pg < cpages; ++pg) {
           const float mix = page_mass(pg) / totc;
 #pragma unroll
@@ -617,61 +652,38 @@ __global__ __launch_bounds__(kGroupThreads) void read_groups_kernel(ReadTilesPar
             const bf16x8 a = as_bf16x8(make_uint4(
                 pack_bf16x2(mix * hv[0], mix * hv[1]), pack_bf16x2(mix * hv[2], mix * hv[3]),
                 pack_bf16x2(mix * hv[4], mix * hv[5]), pack_bf16x2(mix * hv[6], mix * hv[7])));
-            const uint4 gb = *(const uint4*)(pcb + ((size_t)pg * D + e) * D + 16 * kk + 8 * hl);
-            cacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, as_bf16x8(gb), cacc, 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < ET; ++t) {
+              const uint4 gb =
+                  *(const uint4*)(pcb + ((size_t)pg * D + 32 * t + li) * D + 16 * kk + 8 * hl);
+              cacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(gb), a, cacc[t], 0, 0, 0);
+            }
           }
         }
-      }
-    } else if constexpr (COARSE) {
-      if (coarse_on) {
-        uint4 gb[KK];
+      } else {
+        // coarse[q][e] = h_q . G^T[e]
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk)
-          gb[kk] = *(const uint4*)(gc + (size_t)e * D + 16 * kk + 8 * hl);
+        for (int t = 0; t < ET; ++t) {
+          uint4 gb[KK];
 #pragma unroll
-        for (int kk = 0; kk < KK; ++kk)
-          cacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(hA[kk]), as_bf16x8(gb[kk]),
-                                                         cacc, 0, 0, 0);
-      }
-    }
-    // Every operand of the 16 outputs first (rows past the tile clamped),
-    // so the loads are in flight together rather than one round trip per
-    // output behind the previous output's store.
-    float lv[16], xv[16];
+          for (int kk = 0; kk < KK; ++kk)
+            gb[kk] = *(const uint4*)(gc + (size_t)(32 * t + li) * D + 16 * kk + 8 * hl);
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int q = min(8 * (i / 4) + 4 * hl + (i % 4), nq - 1);
-      const int tq = q_first + q;
-      lv[i] = bf2f(p.local[(((size_t)b * p.T + tq) * p.H + h) * D + e]);
-      xv[i] = bf2f(p.rq.p[b * p.rq.sb + (int64_t)tq * p.rq.st + h * p.rq.sh + e]);
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int q = 8 * (i / 4) + 4 * hl + (i % 4);
-      if (q < nq) {
-        const int tq = q_first + q;
-        const float fine =
-            FEAT ? rbf(av[i]) : rbf(rbf(av[i]) * __builtin_amdgcn_rcpf(rbf(acc_den[i])));
-        const size_t row = ((size_t)b * p.T + tq) * p.H + h;
-        if (p.save_fine) {
-          p.save_fine[row * D + e] = f2bf(fine);
-          p.save_coarse[row * D + e] = f2bf(rbf(cacc[i]));
-          // The mixture read has no denominator: 1 keeps the fusion
-          // adjoint's d num = d fine / den exact.
-          if (e == 0) p.save_den[row] = FEAT ? 1.0f : rbf(acc_den[i]);
+          for (int kk = 0; kk < KK; ++kk)
+            cacc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(gb[kk]), as_bf16x8(hA[kk]),
+                                                              cacc[t], 0, 0, 0);
         }
-        p.out[b * p.out_sb + (int64_t)tq * p.out_st + h * p.out_sh + e] =
-            fuse_element(xv[i], lv[i], rbf(cacc[i]), fine, ae, be, p.gain, coarse_on ? 1 : 0, 1);
       }
+#pragma unroll
+      for (int t = 0; t < ET; ++t) put(tile_c, t, cacc[t]);
     }
-  };
-  static_assert(ET == 2 || ET == 4, "head width 64 or 128");
-  emit(acc[0], 0);
-  emit(acc[1], 1);
-  if constexpr (ET == 4) {
-    emit(acc[2], 2);
-    emit(acc[3], 3);
   }
+  static_assert(ET == 2 || ET == 4, "head width 64 or 128");
+  // The wave's own LDS rows: ordered by the wave, not by a barrier.
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  fuse_rows<D, COARSE, false>(p, nullptr, tile_f, tile_c, lane, b, h, q_first, nq, coarse_on);
 }
 
 
