@@ -795,12 +795,13 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
 // read_stream_kernel serves the prefill (turn routes; per-query routes take
 // read_groups_kernel). It is read_groups_kernel's turn-group read with the
 // staging replaced: each fine's C^T goes from HBM straight into one of
-// kRing LDS slots (global_load_lds_dwordx4: lane i of a wave writes 16
+// kRing<D> LDS slots (global_load_lds_dwordx4: lane i of a wave writes 16
 // bytes at the slot's base + 16 i, so the lane picks which global chunk
 // lands there; rows are stored with their 16-byte chunks XOR-swizzled by the
-// row index, which keeps the B-operand reads free of bank conflicts). Fines
-// go in pairs: fines u and u + 1 are read from two slots while u + 2 and
-// u + 3 load into the other two, one barrier per pair. Wave 0 also moves a
+// row index, which keeps the B-operand reads free of bank conflicts). At D = 64
+// fines go in pairs: fines u and u + 1 are read from two slots while u + 2 and
+// u + 3 load into the other two, one barrier per pair; at D = 128 one fine is
+// read while the next loads. Wave 0 also moves a
 // fine's pw and sw rows into LDS and turns them into the fine's weights
 // w = r(pw * sw) before the barrier that publishes the fine. A selecting
 // wave's A operand is r(h * w), and den[q] is the fp32 sum of that operand's
@@ -814,20 +815,34 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
 // the kernel reads them with explicit ds_read_b128 and orders them itself:
 // a wave waits for its own loads of a fine (s_waitcnt vmcnt) before the
 // barrier that publishes it, and for its reads (lgkmcnt) before using them.
-constexpr int kRing = 4;
+//
+// Four waves a workgroup, two workgroups a CU (D = 64: three): one workgroup's
+// set-up, softmax, fusion and barrier waits run beside the other's matrix
+// products. With eight waves and a four-slot ring at D = 128 a CU held one
+// workgroup, all of it in the same phase: 672 us at 16K (H32 D128), 604 now,
+// of which 156 are set-up, softmax and fusion and about 210 the waits for a
+// fine's rows, which one slot ahead does not cover.
+constexpr int kStreamWaves = 4;
+constexpr int kStreamThreads = 64 * kStreamWaves;
+constexpr int kStreamUnion = kStreamWaves * kMaxM;
+template <int D>
+constexpr int kRing = D == 64 ? 4 : 2;
 typedef __attribute__((address_space(3))) void lds_void_t;
 
 template <int D>
 struct StreamSmem {
   uint32_t bits[kBitWords];
   int pre[kBitWords];
-  float wf[kRing][D];                // per slot: the fine's weights r(pw * sw), widened
-  int ids[kGroupWaves][kMaxM];
-  int uni[kMaxUnion];
-  uint32_t mask[kMaxUnion / 4];
+  float wf[kRing<D>][D];                // per slot: the fine's weights r(pw * sw), widened
+  int ids[kStreamWaves][kMaxM];
+  int uni[kStreamUnion];
+  uint32_t mask[kStreamUnion / 4];
   int n_union;
-  int erels[kGroupWaves];
+  int erels[kStreamWaves];
 };
+
+// A value that is the same in every lane, in a scalar register.
+TAO_DEV int wave_uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
 // s_waitcnt with vmcnt <= N (expcnt and lgkmcnt not waited for).
 template <int N>
@@ -890,20 +905,20 @@ TAO_DEV uint32_t lds_addr(const void* p) {
 }
 
 template <int D, bool COARSE, bool FEAT>
-__global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesParams p) {
+__global__ __launch_bounds__(kStreamThreads, 2) void read_stream_kernel(ReadTilesParams p) {
 
   constexpr int KK = D / 16, ET = D / 32, CPR = D / 8;   // k-steps, e-tiles, chunks per row
-  constexpr int CPT = D * CPR / (64 * kGroupWaves);      // 1 KB wave loads per fine and wave
-  static_assert(CPT * 64 * kGroupWaves == D * CPR, "whole wave loads per fine");
-  static_assert(kRing == 4, "two fines read while two load");
+  constexpr int CPT = D * CPR / (64 * kStreamWaves);      // 1 KB wave loads per fine and wave
+  static_assert(CPT * 64 * kStreamWaves == D * CPR, "whole wave loads per fine");
+  constexpr int R = kRing<D>, STEP = R / 2;              // fines read while as many load
   __shared__ StreamSmem<D> sm;
   // The ring of staged C^T (swizzled rows); after the last pass, each wave's
   // fine and coarse tiles for the epilogue's transpose.
-  constexpr int kRingElems = kRing * D * D, kEpiElems = kGroupWaves * 2 * 32 * D;
+  constexpr int kRingElems = R * D * D, kEpiElems = kStreamWaves * 2 * 32 * D;
   __shared__ __attribute__((aligned(16))) bf16_t ring_mem[kRingElems > kEpiElems ? kRingElems
                                                                                  : kEpiElems];
   bf16_t (*ring)[D * D] = reinterpret_cast<bf16_t (*)[D * D]>(ring_mem);
-  __shared__ __attribute__((aligned(16))) bf16_t pwsw[kRing][2][D];     // staged pw and sw rows
+  __shared__ __attribute__((aligned(16))) bf16_t pwsw[R][2][D];     // staged pw and sw rows
   // D = 128: the head's fusion parameters, widened, fpar[0][d][i] =
   // a[h][d][i] and fpar[1][d][i] = b[h][d][i], loaded at the start and read
   // by the epilogue (not for D = 64, whose LDS would then exceed half a CU's).
@@ -913,12 +928,24 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
   const int bh = blockIdx.x % BH;
   // Tiles in reverse plan order: the latest tiles read the most fines, so
   // they start first and the light early tiles fill the end of the launch.
-  const int grp = (p.n_tiles + kGroupWaves - 1) / kGroupWaves - 1 - (int)blockIdx.x / BH;
+  const int grp = (p.n_tiles + kStreamWaves - 1) / kStreamWaves - 1 - (int)blockIdx.x / BH;
   const int b = bh / p.H, h = bh % p.H;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wu = wave_uniform(w);                        // the wave, in a scalar
+  // A wave's 1 KB blocks of a slot hold RPB rows each; the swizzle repeats
+  // every PERIOD blocks, so PERIOD lane offsets serve all of them.
+  constexpr int RPB = 64 / CPR, PERIOD = CPR / RPB;
+  static_assert(CPT % PERIOD == 0, "a wave's blocks start at a swizzle period");
+  static_assert(PERIOD <= 4, "lane offsets");
+  uint32_t off[4];
+#pragma unroll
+  for (int i = 0; i < PERIOD; ++i) {
+    const int row = RPB * i + lane / CPR;
+    off[i] = (uint32_t)(row * D + ((lane % CPR) ^ (row % CPR)) * 8);
+  }
   const int li = lane & 31, hl = lane >> 5;
-  const int t0 = grp * kGroupWaves;
-  const int nt = min(kGroupWaves, p.n_tiles - t0);
+  const int t0 = grp * kStreamWaves;
+  const int nt = min(kStreamWaves, p.n_tiles - t0);
 
   // This wave's tile.
   int q_first = 0, nq = 0, slot = 0, M = 0, erel = 0, fine_on = 0, cpages = 0;
@@ -939,7 +966,7 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
     }
   }
   if (lane == 0) sm.erels[w] = reads ? erel : -1;
-  for (int i = tid; kStageParams && i < 2 * D * 3; i += kGroupThreads) {
+  for (int i = tid; kStageParams && i < 2 * D * 3; i += kStreamThreads) {
     const int which = i / (D * 3), d = (i % (D * 3)) / 3, j = i % 3;
     fpar[which][d * 3 + j] =
         which == 0 ? load_param(p.fa, p.f_dtype, h * p.fa_s[0] + d * p.fa_s[1] + j * p.fa_s[2])
@@ -1029,7 +1056,7 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
   for (int pass_erel = -1;;) {
     int next = 0x7FFFFFFF;
 #pragma unroll
-    for (int v = 0; v < kGroupWaves; ++v) {
+    for (int v = 0; v < kStreamWaves; ++v) {
       const int e = sm.erels[v];
       if (e > pass_erel && e < next) next = e;
     }
@@ -1043,8 +1070,8 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
         p.psw_pool ? p.psw_pool + ((size_t)pass_erel * BH + bh) * 8 * D : nullptr;
 
     // ---- union of the pass's selected sets (ascending fine id), per-wave masks
-    for (int i = tid; i < kBitWords; i += kGroupThreads) sm.bits[i] = 0;
-    for (int i = tid; i < kMaxUnion / 4; i += kGroupThreads) sm.mask[i] = 0;
+    for (int i = tid; i < kBitWords; i += kStreamThreads) sm.bits[i] = 0;
+    for (int i = tid; i < kStreamUnion / 4; i += kStreamThreads) sm.mask[i] = 0;
     if (in_pass) {
       const int32_t* sel = p.sel_pool + ((size_t)slot * BH + bh) * p.sel_cap;
       for (int m = lane; m < M; m += 64) sm.ids[w][m] = sel[m];
@@ -1076,7 +1103,7 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
       if (lane == 63) sm.n_union = incl;
     }
     __syncthreads();
-    for (int i = tid; i < kBitWords; i += kGroupThreads) {
+    for (int i = tid; i < kBitWords; i += kStreamThreads) {
       uint32_t bits = sm.bits[i];
       int r = sm.pre[i];
       while (bits) {
@@ -1096,17 +1123,14 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
 
     // ---- stream the union through the ring
     auto issue = [&](int f) __attribute__((always_inline)) {
-      const int s = f % kRing;
-      const int fid = sm.uni[f];
-      const bf16_t* base = bank + (size_t)fid * D * D;
+      const int s = f % R;
+      const int fid = wave_uniform(sm.uni[f]);
+      const bf16_t* base = bank + (size_t)fid * D * D + (size_t)wu * CPT * RPB * D;
 #pragma unroll
-      for (int i = 0; i < CPT; ++i) {
-        const int J = w * CPT + i;            // this wave's 1 KB block of the slot
-        const int L = J * 64 + lane;          // 16-byte chunk index in the slot
-        const int row = L / CPR, pos = L % CPR;
-        __builtin_amdgcn_global_load_lds(base + (size_t)row * D + (pos ^ (row % CPR)) * 8,
-                                         (lds_void_t*)(&ring[s][0] + J * 64 * 8), 16, 0, 0);
-      }
+      for (int i = 0; i < CPT; ++i)
+        __builtin_amdgcn_global_load_lds(base + (i / PERIOD) * PERIOD * RPB * D + off[i % PERIOD],
+                                         (lds_void_t*)(&ring[s][0] + (wu * CPT + i) * 64 * 8), 16, 0,
+                                         0);
       if (FEAT && w == 0 && lane < CPR) {
         const bf16_t* src = p.fine_z + ((size_t)bh * p.fine_cap + fid) * D + lane * 8;
         __builtin_amdgcn_global_load_lds(src, (lds_void_t*)&pwsw[s][0][0], 16, 0, 0);
@@ -1121,7 +1145,7 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
     };
     // Wave 0 turns the fine's pw and sw rows into its weights.
     auto make_wr = [&](int f) __attribute__((always_inline)) {
-      const int s = f % kRing;
+      const int s = f % R;
       if (FEAT && w == 0 && lane < CPR) {
         // Feature writers: exp(z) of the fine's descriptor.
         u32x4 zv = lds_read16(lds_addr(&pwsw[s][0][lane * 8]));
@@ -1146,7 +1170,7 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
     // (feature_read_coefficients), read against C^T with no denominator.
     auto consume_feat = [&](int u) __attribute__((always_inline)) {
       if (!(in_pass && ((sm.mask[u >> 2] >> ((u & 3) * 8 + w)) & 1u))) return;
-      const int s = u % kRing;
+      const int s = u % R;
       const uint32_t cs = lds_addr(&ring[s][0]);
       float part = 0.0f;
 #pragma unroll
@@ -1181,7 +1205,7 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
     };
     auto consume = [&](int u) __attribute__((always_inline)) {
       if (!(in_pass && ((sm.mask[u >> 2] >> ((u & 3) * 8 + w)) & 1u))) return;
-      const int s = u % kRing;
+      const int s = u % R;
       const uint32_t cs = lds_addr(&ring[s][0]);
       const uint32_t ws = lds_addr(&sm.wf[s][8 * hl]);
       // Step kk runs the ET MFMAs of k-step kk and, between them, builds the
@@ -1292,27 +1316,31 @@ __global__ __launch_bounds__(kGroupThreads) void read_stream_kernel(ReadTilesPar
       wait_lds();
       __builtin_amdgcn_s_barrier();
     };
-    // Fines go in pairs, one barrier per pair: pair (u, u + 1) is read from
-    // ring slots u % 4 and (u + 1) % 4 while fines u + 2 and u + 3 load into
-    // the two slots the previous pair freed. A wave's time per barrier is
-    // then its consume of two fines, and the two fines' slowest waves are
-    // often different ones.
-    for (int f = 0; f < min(U, 2); ++f) issue(f);
-    wait_vmcnt<0>();
-    for (int f = 0; f < min(U, 2); ++f) make_wr(f);
-    ring_barrier();
-    for (int u = 0; u < U; u += 2) {
-      // A wave that reads fine u issues after it: the other waves' issues
-      // have just filled the memory pipeline.
+    // STEP fines a barrier: they are read from their ring slots while the
+    // next STEP load into the slots the previous ones freed. In pairs a
+    // wave's time per barrier is its consume of two fines, whose slowest
+    // waves are often different ones.
+    auto read = [&](int u) __attribute__((always_inline)) {
       if constexpr (FEAT) consume_feat(u);
       else consume(u);
-      for (int f = u + 2; f < min(U, u + 4); ++f) issue(f);
-      if (u + 1 < U) {
-        if constexpr (FEAT) consume_feat(u + 1);
-        else consume(u + 1);
+    };
+    for (int f = 0; f < min(U, STEP); ++f) issue(f);
+    wait_vmcnt<0>();
+    for (int f = 0; f < min(U, STEP); ++f) make_wr(f);
+    ring_barrier();
+    for (int u = 0; u < U; u += STEP) {
+      if constexpr (STEP == 2) {
+        // A wave that reads fine u issues after it: the other waves' issues
+        // have just filled the memory pipeline.
+        read(u);
+        for (int f = u + 2; f < min(U, u + 4); ++f) issue(f);
+        if (u + 1 < U) read(u + 1);
+      } else {
+        if (u + 1 < U) issue(u + 1);
+        read(u);
       }
-      wait_vmcnt<0>();        // this wave's loads of fines u + 2 and u + 3
-      for (int f = u + 2; f < min(U, u + 4); ++f) make_wr(f);
+      wait_vmcnt<0>();        // this wave's loads of the next fines
+      for (int f = u + STEP; f < min(U, u + 2 * STEP); ++f) make_wr(f);
       ring_barrier();
     }
     wait_vmcnt<0>();
@@ -1460,8 +1488,10 @@ hipError_t launch_epochs(const EpochParams& p, int head_dim, hipStream_t s) {
 hipError_t launch_read_tiles(const ReadTilesParams& p, int head_dim, hipStream_t s) {
   if (p.n_tiles <= 0) return hipSuccess;
   if (p.fine_cap > kMaxFineIds) return hipErrorInvalidValue;
-  const int groups = (p.n_tiles + kGroupWaves - 1) / kGroupWaves;
-  const dim3 grid((unsigned)(groups * p.B * p.H));
+  auto groups = [&](int waves) {
+    return dim3((unsigned)((p.n_tiles + waves - 1) / waves * p.B * p.H));
+  };
+  const dim3 grid = groups(kGroupWaves), sgrid = groups(kStreamWaves);
   const bool coarse = p.coarse_pool != nullptr;
   const bool perq = p.qsel != nullptr;
   if (perq && (p.qsel_words < 1 || p.qsel_words > kBitWords)) return hipErrorInvalidValue;
@@ -1470,9 +1500,9 @@ hipError_t launch_read_tiles(const ReadTilesParams& p, int head_dim, hipStream_t
 #define TAO_MIXTURE_LAUNCH(D_, C_)                                                            \
   hipLaunchKernelGGL((read_groups_kernel<D_, C_, true, true>), grid, dim3(kGroupThreads), 0, s, p)
 #define TAO_STREAM_LAUNCH(D_, C_)                                                             \
-  hipLaunchKernelGGL((read_stream_kernel<D_, C_, false>), grid, dim3(kGroupThreads), 0, s, p)
+  hipLaunchKernelGGL((read_stream_kernel<D_, C_, false>), sgrid, dim3(kStreamThreads), 0, s, p)
 #define TAO_FEATURE_LAUNCH(D_, C_)                                                            \
-  hipLaunchKernelGGL((read_stream_kernel<D_, C_, true>), grid, dim3(kGroupThreads), 0, s, p)
+  hipLaunchKernelGGL((read_stream_kernel<D_, C_, true>), sgrid, dim3(kStreamThreads), 0, s, p)
   if (head_dim != 128 && head_dim != 64) return hipErrorInvalidValue;
   if (p.fine_z) {
     // Feature writers, no saves: per-query routes index-only; turn routes
