@@ -74,12 +74,20 @@ def _zeroed_views(device, specs):
         offsets.append((total, nbytes))
         total += (nbytes + 255) // 256 * 256
     arena = torch.zeros(max(total, 256), dtype=torch.uint8, device=device)
-    views = []
+    typed, views = {}, []
     for spec, off in zip(specs, offsets):
         if spec is None:
             views.append(None)
-        else:
-            views.append(arena[off[0]:off[0] + off[1]].view(spec[1]).view(spec[0]))
+            continue
+        shape, dtype = spec
+        base = typed.get(dtype)           # one retyped view per dtype, one view per buffer
+        if base is None:
+            base = typed[dtype] = arena.view(dtype)
+        strides, step = [], 1
+        for n in reversed(shape):
+            strides.append(step)
+            step *= n
+        views.append(base.as_strided(shape, strides[::-1], off[0] // dtype.itemsize))
     return views
 
 
@@ -129,6 +137,7 @@ class _DeviceState:
         if self.association or self.feature:
             self.stats = self.stats_scratch(stats_cap)
         self.generation = next(_SERIAL)   # renewed whenever the buffers move
+        self.home = self.stream()         # the stream the buffers belong to
         self.fine_cap = 0
         self.plan_words = max(plan_words, 4096)
         self._allocate(fine_cap, copy_fines=0)
@@ -366,6 +375,7 @@ class StreamCache:
         # The regional graph serves the memo-backed index-only read only
         # (tao_stream.py:238-248). Replay mechanism: see HistoryRegionGraph.
         self._graph_mode = 0
+        self._drain = False          # a call ran on another stream than the buffers'
         if (config.q1_history_region_graph and config.q1_page_normalization_memo
                 and config.coarse_index_only):
             replay = os.environ.get("TAO_GRAPH_REPLAY", "dispatch")
@@ -420,8 +430,13 @@ class StreamCache:
                 self._handle, _hip.GRAPH_REASONS.index(reason)))
 
     def _close_driver(self):
+        """Close the native driver. The caller's stream is drained first where
+        the driver holds captured steps or a call ran on another stream; a
+        driver without a graph holds no device memory, and the state's buffers
+        are freed in their stream's order (a server's next request is then
+        issued while the last one still runs)."""
         if self._handle is not None:
-            if self._dev is not None:
+            if self._dev is not None and (self._graph_mode or self._drain):
                 torch.cuda.current_stream(self._dev.device).synchronize()
             if self.history_region is not None:
                 self.history_region._stats()         # keep the final counters
@@ -471,7 +486,15 @@ class StreamCache:
         elif self._dev.reserve(fines, schedule.fines_at(self.position, self.config)):
             self._release_graph("capacity")
             self._handle_dirty = True
+        self._note_stream(self._dev.stream())
         return self._dev
+
+    def _note_stream(self, stream):
+        """A call on another stream than the buffers' own: the caching
+        allocator orders a freed buffer's reuse after its own stream only, so
+        such a state is drained before its buffers go."""
+        if stream != self._dev.home:
+            self._drain = True
 
     # ----------------------------------------------------------------- kernels
     def _timed(self, name):
@@ -732,9 +755,11 @@ class StreamCache:
         nat = self._native
         if nat is not None and self.position < self._fast_limit and not self._handle_dirty:
             pos = self.position
+            stream = _hip.raw_stream(self._stream_index)
+            if stream != self._dev.home:
+                self._drain = True
             try:
-                r = nat(q, k, v, raw_q, raw_k, fusion_a, fusion_b, alpha, pos,
-                        _hip.raw_stream(self._stream_index))
+                r = nat(q, k, v, raw_q, raw_k, fusion_a, fusion_b, alpha, pos, stream)
             except TypeError:
                 r = None
             if r is not None:
@@ -810,6 +835,7 @@ class StreamCache:
         out_ptr, out_s = out.data_ptr(), self._out_s
         info = self._info
         stream = _hip.raw_stream(self._stream_index)
+        self._note_stream(stream)
         if self._probe is None:
             rc = self._call(self._handle, self._tok_ref, self._fu_ref, out_ptr, out_s, stream,
                             info)
@@ -868,6 +894,7 @@ class StreamCache:
         self._check_supported(q)
         if not self._replayable_next():
             raise RuntimeError("the next token seals or changes its route; decode it eagerly")
+        self._drain = True               # the caller's graph replays on any stream
         q, k, v, raw_q, raw_k = _hip.vector_operands(q, k, v, raw_q, raw_k)
         tok = _hip.tokens(q, k, v, raw_q, raw_k)
         fu = _hip.fusion(fusion_a, fusion_b, alpha, False, True, like=q)
@@ -989,6 +1016,8 @@ class StreamCache:
         """Owned tensors in the reference snapshot schema (tao_stream.py:853-877)."""
         cfg = self.config
         dev = self._dev
+        if dev is not None:
+            self._note_stream(dev.stream())
         fines = schedule.fines_at(self.position, cfg)
         group = cfg.coarse_group
         completed, pending = divmod(fines, group)
@@ -1305,6 +1334,7 @@ class DecodeBatch:
             if dev.B != 1:
                 raise ValueError("batched decode takes one-request states (batch 1)")
             st._driver(dev)
+            st._drain = True              # the batch's calls do not note their stream
         key = tuple((id(st), st._handle_serial) for st in self.states)
         gens = tuple(st._dev.generation for st in self.states)
         lib = _hip.lib()

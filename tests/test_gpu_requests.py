@@ -1,0 +1,63 @@
+"""Requests issued one after another without waiting for the GPU: a finished
+request's state is freed in its stream's order while its kernels still run."""
+import pytest
+import torch
+
+from tao_attention import (TaoConfig, new_state, tao_attention_decode, tao_attention_prefill)
+
+pytestmark = pytest.mark.gpu
+
+
+def _request(xs, fusion, config, steps):
+    state, outs = new_state(0, config), []
+    cuts = [(0, xs[0].shape[1] - steps)] + [(i, 1) for i in range(xs[0].shape[1] - steps,
+                                                                  xs[0].shape[1])]
+    for at, n in cuts:
+        q, k, v, rq, rk = (x[:, at:at + n].contiguous() for x in xs)
+        call = tao_attention_prefill if n > 1 else tao_attention_decode
+        out, state = call(q, k, v, raw_q=rq, raw_k=rk, fusion_a=fusion[0], fusion_b=fusion[1],
+                          alpha=0.5, state=state, position=state.get_pos())
+        outs.append(out)
+    return torch.cat(outs, 1), state
+
+
+@pytest.mark.parametrize("side_stream", [False, True])
+def test_requests_in_flight_do_not_share_memory(device, side_stream):
+    g = torch.Generator(device=device).manual_seed(9)
+    config = TaoConfig()
+    fusion = [torch.randn(4, 128, 3, generator=g, device=device) * 0.02 for _ in range(2)]
+    inputs = [[torch.randn(1, n, 4, 128, generator=g, device=device).to(torch.bfloat16)
+               for _ in range(5)] for n in (2900, 1100, 3300)]
+    want = []
+    for xs in inputs:
+        want.append(_request(xs, fusion, config, 3)[0])
+        torch.cuda.synchronize()
+    stream = torch.cuda.Stream() if side_stream else torch.cuda.current_stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        got = [_request(inputs[i % 3], fusion, config, 3)[0] for i in range(12)]
+    torch.cuda.synchronize()
+    for i, out in enumerate(got):
+        assert torch.equal(out, want[i % 3])
+
+
+def test_a_state_used_on_another_stream_is_drained(device):
+    """Buffers of the default stream, a decode on a side stream: closing the
+    driver waits for the side stream before the buffers are freed."""
+    g = torch.Generator(device=device).manual_seed(10)
+    fusion = [torch.randn(2, 64, 3, generator=g, device=device) * 0.02 for _ in range(2)]
+    xs = [torch.randn(1, 801, 2, 64, generator=g, device=device).to(torch.bfloat16)
+          for _ in range(5)]
+    _, state = _request([x[:, :800] for x in xs], fusion, TaoConfig(), 1)
+    assert not state._drain
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    q, k, v, rq, rk = (x[:, 800:].contiguous() for x in xs)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        _, state = tao_attention_decode(q, k, v, raw_q=rq, raw_k=rk, fusion_a=fusion[0],
+                                        fusion_b=fusion[1], alpha=0.5, state=state,
+                                        position=state.get_pos())
+        assert state._drain
+        del state
+        assert side.query()
