@@ -193,9 +193,9 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
 // workgroup stages each fine's C^T already weighted (r(C^T * w), padded LDS,
 // double-buffered, the next fine's rows and weight slices in flight in
 // registers) and every tile's A operand is its queries' h, which stays in
-// registers for the whole kernel: a selecting wave runs 4 x 8
-// v_mfma_f32_32x32x16_bf16 into its 32 x D accumulator plus 8 against the
-// weights for den[q] = sum over its fines of h_q . w, with no per-fine VALU.
+// registers for the whole kernel: a selecting wave runs D / 32 x D / 16
+// v_mfma_f32_32x32x16_bf16 into its 32 x D accumulator and takes den[q] = sum
+// over its fines of h_q . w from bf16 pair dot products beside them.
 // The workgroup takes one pass per distinct epoch among its tiles (a group
 // straddles at most a seal): each pass streams the union of its tiles'
 // selected sets. fine = r(r(num) / r(den)), then the fusion epilogue. The
@@ -921,7 +921,7 @@ __global__ __launch_bounds__(kStreamThreads, 2) void read_stream_kernel(ReadTile
   __shared__ __attribute__((aligned(16))) bf16_t pwsw[R][2][D];     // staged pw and sw rows
   // D = 128: the head's fusion parameters, widened, fpar[0][d][i] =
   // a[h][d][i] and fpar[1][d][i] = b[h][d][i], loaded at the start and read
-  // by the epilogue (not for D = 64, whose LDS would then exceed half a CU's).
+  // by the epilogue. D = 64 reads them from memory.
   constexpr bool kStageParams = D == 128;
   __shared__ __attribute__((aligned(16))) float fpar[2][kStageParams ? D * 3 : 4];
   const int BH = p.B * p.H;
