@@ -726,8 +726,8 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
         be[j][i] = load_param(p.fb, p.f_dtype, h * p.fb_s[0] + (8 * c + j) * p.fb_s[1] + i * p.fb_s[2]);
       }
   }
-  // Without the coarse branch: the paired two-channel fusion on the rounded
-  // parameters and the signed-zero coarse term.
+  // The rounded parameters, and the signed-zero coarse term of a tile without
+  // the coarse branch.
   float ra[8][3], rb[8][3];
 #pragma unroll
   for (int j = 0; j < 8; ++j)
@@ -769,17 +769,12 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
     uint32_t o[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if constexpr (!COARSE) {
+      if (COARSE && coarse_on)
+        o[j] = fuse_pair_all(&xv[2 * j], &lv[2 * j], &cv[2 * j], &fv[2 * j], &ra[2 * j],
+                             &rb[2 * j], p.gain);
+      else
         o[j] = fuse_pair_local_fine(&xv[2 * j], &lv[2 * j], &fv[2 * j], &ra[2 * j], &rb[2 * j],
                                     p.gain, ct0);
-      } else {
-        const bf16_t lo = fuse_element(xv[2 * j], lv[2 * j], cv[2 * j], fv[2 * j], ae[2 * j],
-                                       be[2 * j], p.gain, coarse_on ? 1 : 0, 1);
-        const bf16_t hi = fuse_element(xv[2 * j + 1], lv[2 * j + 1], cv[2 * j + 1], fv[2 * j + 1],
-                                       ae[2 * j + 1], be[2 * j + 1], p.gain, coarse_on ? 1 : 0, 1);
-        o[j] = (uint32_t)__builtin_bit_cast(uint16_t, lo) |
-               ((uint32_t)__builtin_bit_cast(uint16_t, hi) << 16);
-      }
     }
     *(uint4*)(p.out + b * p.out_sb + (int64_t)tq * p.out_st + h * p.out_sh + 8 * c) =
         make_uint4(o[0], o[1], o[2], o[3]);

@@ -60,12 +60,6 @@ TAO_DEV bf16_t fuse_mix(const FuseWeights& w, float local, float coarse, float f
   return f2bf(rbf(lt + ct) + ft);
 }
 
-TAO_DEV bf16_t fuse_element(float q, float local, float coarse, float fine,
-                            const float a[3], const float b[3], float gain,
-                            int coarse_on, int fine_on) {
-  return fuse_mix(fuse_weights(q, a, b, coarse_on, fine_on), local, coarse, fine, gain);
-}
-
 // Rounds x and y to bf16 with one packed conversion.
 TAO_DEV void rbf2(float& x, float& y) {
   const uint32_t pk = pack_bf16x2(x, y);
@@ -75,8 +69,8 @@ TAO_DEV void rbf2(float& x, float& y) {
 
 // Two adjacent channels of the fusion with the fine branch present and the
 // coarse branch absent, packed as bf16x2 (channel 0 low). Bit-identical to
-// fuse_element(q[j], local[j], 0, fine[j], a[j], b[j], gain, 0, 1) with
-// ra = rbf(a), rb = rbf(b): each rounding point is the same, paired over
+// fuse_mix(fuse_weights(q[j], a[j], b[j], 0, 1), local[j], 0, fine[j], gain)
+// with ra = rbf(a), rb = rbf(b): each rounding point is the same, paired over
 // the two channels, and the coarse terms are folded. Without the coarse
 // branch the local bias is 0, so rbf(s0 + 0) differs from s0 only in the
 // sign of a zero, which no later step sees (exp(s - top) is 1 for either
@@ -104,21 +98,18 @@ TAO_DEV uint32_t fuse_pair_local_fine(const float q[2], const float local[2], co
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
     // exp(p - top) of the larger branch is exp(0) = 1 exactly, so only the
-    // other one's exp is computed (a NaN lands in that exp, so it still
-    // makes both weights NaN).
+    // other one's exp is computed, at -|p0 - p2| (a NaN lands in that exp,
+    // so it still makes both weights NaN).
     const bool first = p0[j] >= p2[j];
-    const float top = first ? p0[j] : p2[j], low = first ? p2[j] : p0[j];
-    const float xl = __expf(low - top);
-    const float x0 = first ? 1.0f : xl, x2 = first ? xl : 1.0f;
-    const float inv = __builtin_amdgcn_rcpf(x0 + x2);
-    e0[j] = x0 * inv;
-    e2[j] = x2 * inv;
-    l2[j] = 2.0f * local[j];
+    const float xl = __expf(-fabsf(p0[j] - p2[j]));
+    const float inv = __builtin_amdgcn_rcpf(1.0f + xl), low = xl * inv;
+    e0[j] = first ? inv : low;
+    e2[j] = first ? low : inv;
+    l2[j] = 2.0f * local[j];            // a bf16 value doubled is one, or infinite
     gf[j] = gain * fine[j];
   }
   rbf2(e0[0], e0[1]);
   rbf2(e2[0], e2[1]);
-  rbf2(l2[0], l2[1]);
   rbf2(gf[0], gf[1]);
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -128,6 +119,55 @@ TAO_DEV uint32_t fuse_pair_local_fine(const float q[2], const float local[2], co
   rbf2(l2[0], l2[1]);
   rbf2(gf[0], gf[1]);
   return pack_bf16x2((l2[0] + ct0) + gf[0], (l2[1] + ct0) + gf[1]);
+}
+
+// Two adjacent channels with all three branches present, packed as bf16x2:
+// fuse_mix(fuse_weights(q[j], a[j], b[j], 1, 1), local[j], coarse[j], fine[j],
+// gain) with ra = rbf(a), rb = rbf(b), bit for bit. A read tile's fusion is
+// VALU work; one conversion rounds two channels, and the doubled local value
+// needs none: the per-query read of B2 T8192 H12 D64 went from 109 to 97 us
+// (the turn-group read without the coarse branch, B1 T16384 H32 D128, from
+// 599 to 588 with its two-branch form's shorter softmax).
+TAO_DEV uint32_t fuse_pair_all(const float q[2], const float local[2], const float coarse[2],
+                               const float fine[2], const float ra[2][3], const float rb[2][3],
+                               float gain) {
+  float s[3][2], e[3][2], v[3][2];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    s[i][0] = ra[0][i] * q[0];
+    s[i][1] = ra[1][i] * q[1];
+    rbf2(s[i][0], s[i][1]);
+    s[i][0] = s[i][0] + rb[0][i];
+    s[i][1] = s[i][1] + rb[1][i];
+    rbf2(s[i][0], s[i][1]);
+  }
+  s[0][0] = s[0][0] + kLogTwoBf16;
+  s[0][1] = s[0][1] + kLogTwoBf16;
+  rbf2(s[0][0], s[0][1]);
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const float top = fmaxf(s[0][j], fmaxf(s[1][j], s[2][j]));
+#pragma unroll
+    for (int i = 0; i < 3; ++i) e[i][j] = __expf(s[i][j] - top);
+    const float inv = __builtin_amdgcn_rcpf((e[0][j] + e[2][j]) + e[1][j]);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) e[i][j] = e[i][j] * inv;
+    v[0][j] = 2.0f * local[j];          // a bf16 value doubled is one, or infinite
+    v[1][j] = gain * coarse[j];
+    v[2][j] = gain * fine[j];
+  }
+  rbf2(v[1][0], v[1][1]);
+  rbf2(v[2][0], v[2][1]);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    rbf2(e[i][0], e[i][1]);
+    v[i][0] = e[i][0] * v[i][0];
+    v[i][1] = e[i][1] * v[i][1];
+    rbf2(v[i][0], v[i][1]);
+  }
+  float m[2] = {v[0][0] + v[1][0], v[0][1] + v[1][1]};
+  rbf2(m[0], m[1]);
+  return pack_bf16x2(m[0] + v[2][0], m[1] + v[2][1]);
 }
 
 }  // namespace tao
