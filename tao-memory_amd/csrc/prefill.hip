@@ -814,9 +814,11 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
 // Four waves a workgroup, two workgroups a CU (D = 64: three): one workgroup's
 // set-up, softmax, fusion and barrier waits run beside the other's matrix
 // products. With eight waves and a four-slot ring at D = 128 a CU held one
-// workgroup, all of it in the same phase: 672 us at 16K (H32 D128), 604 now,
-// of which 156 are set-up, softmax and fusion and about 210 the waits for a
-// fine's rows, which one slot ahead does not cover.
+// workgroup, all of it in the same phase: 672 us at 16K (H32 D128), 588 now
+// (604 before the fusion's shorter arithmetic), of which about 145 are set-up,
+// softmax and fusion and about 210 the waits for a fine's rows, which one slot
+// ahead does not cover. Giving each XCD one or two heads at a time (their fines
+// then fit its L2) measured the same.
 constexpr int kStreamWaves = 4;
 constexpr int kStreamThreads = 64 * kStreamWaves;
 constexpr int kStreamUnion = kStreamWaves * kMaxM;
