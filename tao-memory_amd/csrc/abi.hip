@@ -1111,6 +1111,7 @@ int tao_prefill(const tao_state_dev* st, const tao_tokens* tok, const tao_fusion
   }
   // ---- turns
   bool turns_ascend = true;
+  int64_t turn_keys = 0;             // most pages or candidates of a turn
   for (int64_t i = 0; i < n_turns; ++i) {
     const int64_t* t = plan + off_turns + 8 * i;
     if (i && t[1] < t[1 - 8]) turns_ascend = false;
@@ -1122,6 +1123,7 @@ int tao_prefill(const tao_state_dev* st, const tao_tokens* tok, const tao_fusion
         t[6] >= pools->sel_slots || (t[7] != 0 && t[7] != 1) || t[2] > 2048 ||
         eligible > 2048 || t[4] > st->chosen_cap)
       return fail(TAO_E_ARGUMENT, "invalid route turn in the plan");
+    turn_keys = std::max(turn_keys, std::max(t[2], eligible));
   }
   // ---- read tiles
   if (n_read > 0 && need_pools && st->fine_cap > 16384)
@@ -1316,6 +1318,7 @@ int tao_prefill(const tao_state_dev* st, const tao_tokens* tok, const tao_fusion
     rp.chosen_cap = st->chosen_cap;
     rp.group = G;
     rp.max_epoch = (int)(first_epoch + n_epochs - 1);
+    rp.max_keys = (int)turn_keys;
     rp.n_epochs = turns_ascend ? (int)n_epochs : 0;
     e = tao::launch_route(rp, D, s);
     if (e != hipSuccess) return check_hip(e, "tao_prefill routes");

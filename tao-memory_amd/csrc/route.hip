@@ -14,6 +14,7 @@
 // << 32 | ~index) ranked by counting (<= 512 keys) or an LDS bitonic network.
 // Eight waves issue the loads of eight rows each before reducing them, so a
 // refresh costs a few memory latencies rather than one per row.
+#include "route_lds.h"
 #include "tao_launch.h"
 #include "tao_common.h"
 
@@ -895,22 +896,6 @@ TAO_DEV void quad_select(const uint16_t* keys, int n, int m, int lane, const Emi
     quad_select_n<0>(keys, n, m, lane, emit);
 }
 
-// LDS of a per-query routing workgroup: h rows, fine keys and page keys of its
-// query slots. A key row holds an odd number of words, so a column of them
-// over the lanes spreads over the banks. Once the masses are formed the open
-// pages (a bit each) and the selection lie where the h rows were.
-struct RouteLds {
-  int slots, fkeys, pkeys;           // slots; 16-bit keys of a row
-  __host__ __device__ size_t bytes(int D) const {
-    return (size_t)slots * (2 * (D + 8) + 2 * fkeys + 2 * pkeys);
-  }
-};
-static RouteLds route_lds(int slots, int max_epoch) {
-  auto odd = [](int keys) { return 2 * (((keys + 1) / 2) | 1); };
-  return RouteLds{slots, odd(max_epoch), odd(max_epoch / 8 + 1)};
-}
-constexpr size_t kLdsBytes = 160 * 1024;
-
 // Opens the pages a query reads (open: one bit a page, zeroed) and clears the
 // keys of the other pages' fines; four lanes a query.
 TAO_DEV void quad_open_pages(const uint16_t* pkey, uint16_t* fkey, uint32_t* open, int K,
@@ -1021,9 +1006,6 @@ __global__ __launch_bounds__(kQThreads, 2) void route_queries_kernel(QueryRouteP
 // 87 us with a lane per (turn, row) pair in groups of sixteen turns over two
 // or three epochs, 57 us now; one 16K call at 128K (rows beyond that form's
 // LDS, a workgroup per turn): 350 -> 150 us.
-constexpr int kTurnSlots = 16;
-constexpr int kTurnMaxEpoch = 2048;
-
 TAO_DEV uint32_t score_key32(float score_bf, int index) {
   bf16_t bits = f2bf(score_bf);
   if (bits == 0x8000) bits = 0;                      // -0 ties with +0, as in torch's sort
@@ -1182,12 +1164,14 @@ hipError_t launch_route(const RouteParams& p, int head_dim, hipStream_t s) {
     return hipErrorInvalidValue;
   if (p.turns && p.gate.header) return hipErrorInvalidValue;   // gates serve single turns
   // Turn mode: a workgroup per epoch when the turns ascend by epoch and the
-  // keys of sixteen turns fit the LDS; a workgroup per turn otherwise.
-  if (p.turns && p.n_turns > 0 && p.n_epochs > 0 && p.group == 8 && p.max_epoch >= 1 &&
-      p.max_epoch <= kTurnMaxEpoch && (head_dim == 64 || head_dim == 128)) {
-    // A turn has at most its epoch's candidates and pages, p.max_epoch of both.
-    const int cap = 4 * ((p.max_epoch + 3) / 4) + 4;
-    const size_t bytes = (size_t)kTurnSlots * (2 * (head_dim + 8) + 5 * cap);
+  // keys of sixteen turns fit the LDS (those of a route of up to 512 fines, all
+  // that a state keeps, do: at most 1,031 candidates); a workgroup per turn
+  // otherwise.
+  if (p.turns && p.n_turns > 0 && p.n_epochs > 0 && p.group == 8 &&
+      (head_dim == 64 || head_dim == 128) &&
+      turn_route_fits(head_dim, p.max_epoch, p.max_keys)) {
+    const int cap = turn_route_cap(p.max_keys);
+    const size_t bytes = turn_route_bytes(head_dim, cap);
     const dim3 tgrid((unsigned)(p.B * p.H * p.n_epochs));
     const auto kernel = head_dim == 128 ? route_turns_kernel<128> : route_turns_kernel<64>;
     if (bytes > 60 * 1024) {

@@ -266,6 +266,7 @@ struct RouteParams {
   int B, H, fine_cap, page_cap, sel_cap, chosen_cap, group;
   int completed, pending, coarse, selected;
   int max_epoch;                 // turn mode: largest epoch of any turn (0: unknown)
+  int max_keys;                  // turn mode: most pages or candidates of any turn
   int n_epochs;                  // turn mode: epochs of the turns, which ascend by epoch (0: unordered)
   TurnGate gate;                 // single-turn mode only
 };

@@ -10,7 +10,8 @@ import pytest
 import torch
 
 from oracle import tao_oracle as O
-from tao_attention import TaoConfig, new_state, tao_attention, tao_attention_prefill, training
+from tao_attention import (TaoConfig, new_state, tao_attention, tao_attention_decode,
+                           tao_attention_prefill, training)
 from test_gpu_parity import inputs, run_oracle, to_dev, run_hip, compare_snapshots, TOL
 
 pytestmark = pytest.mark.gpu
@@ -67,3 +68,28 @@ def test_turn_routes_of_any_period_match_the_oracle(device, period, layer):
     ora, ref = run_oracle(layer, xs, fa, fb, splits, geometry=O.Geometry.from_config(config))
     torch.testing.assert_close(out.cpu().float(), ref.float(), **TOL)
     compare_snapshots(state.export(), ora.export())
+
+
+@pytest.mark.parametrize("width", [64, 128])
+def test_turn_routes_near_two_thousand_fines(device, width):
+    """A prompt chunk at 2,044 and 2,045 visible fines: its last turn routes
+    as a decode step's refresh at the same token does (another kernel, the same
+    arithmetic), bit for bit; the heads differ by the bf16 rounding of the two
+    reads (about 4e-3 each)."""
+    print(f"turn routes near 2,048 fines D={width}", flush=True)
+    turn = 524280                                  # 768 + 24 k
+    (q, k, v, rq, rk), (fa, fb) = _tokens(turn + 1, 1, width, width)
+    xs = (q, k, v, rq, rk)
+    named = dict(fusion_a=fa, fusion_b=fb, alpha=0.5)
+    outs, routes = [], []
+    for cut, call in ((turn - 300, tao_attention_prefill), (turn, tao_attention_decode)):
+        state = new_state(0, TaoConfig(coarse_index_only=True))
+        state._ingest(*(x[:, :cut].contiguous() for x in xs))
+        c = [x[:, cut:].contiguous() for x in xs]
+        out, state = call(*c[:3], raw_q=c[3], raw_k=c[4], state=state, position=cut, **named)
+        outs.append(out[:, -1].double())
+        routes.append(state.export()["route_ids"])
+        del state
+    for a, b in zip(*routes):
+        assert torch.equal(a, b)
+    assert ((outs[0] - outs[1]).norm() / outs[1].norm()).item() < 0.03

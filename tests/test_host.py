@@ -284,6 +284,54 @@ def test_native_train_plan_matches_read_training_tiling():
             assert starts == list(range(0, tokens, 32))
 
 
+_ROUTE_LDS = r'''
+#include <cstdio>
+#include <initializer_list>
+#include "%(csrc)s/route_lds.h"
+#include "%(csrc)s/schedule.h"
+using namespace tao;
+int main() {
+  tao_stream_cfg cfg{};
+  cfg.local_keep = 512; cfg.fine_tokens = 256; cfg.coarse_group = 8;
+  cfg.budget_root_scale = 2; cfg.budget_offset = 2;
+  for (int D = 64; D <= 128; D += 64) {
+    for (int fines = 1; fines <= 2049; ++fines) {
+      int64_t coarse = 0, eligible = 0, selected = 0;
+      sched::routed_counts(cfg, fines / 8, fines %% 8, &coarse, &eligible, &selected);
+      const int turn = (int)(fines / 8 > eligible ? fines / 8 : eligible);
+      // a stream's own turns fit up to 2,048 fines, and nothing that does not
+      // fit is accepted, up to every fine being a candidate
+      if (turn_route_fits(D, fines, turn) != (fines <= 2048)) return 1;
+      for (int keys : {turn, 1031, fines})
+        if (turn_route_fits(D, fines, keys) &&
+            turn_route_bytes(D, turn_route_cap(keys)) + kTurnOpenBytes > kLdsBytes) return 2;
+      if (fines <= 2048 && !turn_route_fits(D, fines, fines < 1031 ? fines : 1031)) return 3;
+      if (turn_route_cap(turn) < turn) return 4;
+    }
+    if (turn_route_fits(D, 2048, 2048)) return 5;
+    for (int fines = 1; fines <= 1024; ++fines) {
+      const bool two = route_lds(64, fines).bytes(D) <= kLdsBytes;
+      if (two != (D == 64 || fines <= 1014)) return 6;
+      if (route_lds(32, fines).bytes(D) > kLdsBytes) return 7;
+    }
+  }
+  std::puts("ok");
+}
+'''
+
+
+def test_routing_kernels_fit_the_lds_at_every_size(tmp_path):
+    """Each number of visible fines gets a routing kernel whose LDS a CU has:
+    turn routes of any route that a state can keep up to 2,048 fines, per-query
+    routes (two read tiles a workgroup, one past 1,014 fines at width 128)."""
+    import subprocess
+    src, exe = tmp_path / "lds.cpp", tmp_path / "lds"
+    src.write_text(_ROUTE_LDS % {"csrc": os.path.join(ROOT, "tao-memory_amd", "csrc")})
+    subprocess.run(["g++", "-std=c++17", "-o", str(exe), str(src)], check=True)
+    got = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert (got.returncode, got.stdout) == (0, "ok\n")
+
+
 def test_graph_stat_layout_matches_header():
     """The Python view of the driver's epoch counters uses the header's enums."""
     text = open(os.path.join(ROOT, "include", "tao_memory.h")).read()
