@@ -507,10 +507,12 @@ __global__ __launch_bounds__(kReadThreads) void f32_read_kernel(F32Params p, F32
   float* const den = (float*)(sel + kChunk * lds.cand);          // [query]
   __shared__ uint32_t picked[kChunk][kMaxPages * kGroup / 32];   // bit per fine
   __shared__ uint32_t open[kChunk][kMaxPages / 32];
+  __shared__ uint32_t bad;                             // queries whose numerator holds a NaN
   const int PC = lds.cand;
 
   for (int i = tid; i < kChunk * (kMaxPages * kGroup / 32); i += kReadThreads) (&picked[0][0])[i] = 0u;
   if (tid < kChunk * (kMaxPages / 32)) (&open[0][0])[tid] = 0u;
+  if (tid == 0) bad = 0u;
   // Page z the tile sees, page weights and coarse weights: a thread per
   // channel for up to 8 pages (the fold over the next power of two), else
   // lanes = pages and the waves take the channels in turn.
@@ -696,7 +698,40 @@ __global__ __launch_bounds__(kReadThreads) void f32_read_kernel(F32Params p, F32
       buf ^= 1;
     }
   }
-  __syncthreads();                                     // den
+  // A query that did not select a fine of the union has rows of 0 against its
+  // matrix, and 0 times an infinite or NaN entry is NaN. A NaN outlives the
+  // sums, so a query that holds one sums its own fines again.
+  uint32_t mine = 0;
+#pragma unroll
+  for (int j = 0; j < TW; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (num[j][r] != num[j][r]) mine |= 1u << (4 * k4 + r);
+  if (mine) atomicOr(&bad, mine);
+  __syncthreads();                                     // den, bad
+  for (uint32_t left = bad; left; left &= left - 1) {
+    const int q = __builtin_ctz(left);
+    float sum[TW] = {};
+    for (int m = 0; q < nq && m < M; ++m) {
+      const int id = sel[q * PC + m];
+      const float* sw = sw_row(id);
+      const float* pg = pw + (id / kGroup) * D;
+      const float* c = p.bank + (bh * p.S + id) * D * D + 16 * TW * w + col;
+      for (int d = k4; d < D; d += 4) {
+        const float x = (hs[q * HP + d] * pg[d]) * sw[d];
+#pragma unroll
+        for (int j = 0; j < TW; ++j) sum[j] = fmaf(x, c[(size_t)d * D + 16 * j], sum[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < TW; ++j) {
+      sum[j] += __shfl_xor(sum[j], 16);
+      sum[j] += __shfl_xor(sum[j], 32);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * k4 + r == q) num[j][r] = sum[j];
+    }
+  }
 
   // _fuse_training at fp32 (operator.py:21-38); both history branches
   // present only with coarse values past first_coarse.

@@ -178,3 +178,26 @@ def test_fp32_tile_edges_and_unaligned_rows(batch, tokens, heads, width, index_o
     if routes:
         check_routes(sel, routes, tokens)
     torch.testing.assert_close(out.cpu(), ref, **TOL32)
+
+
+def test_fp32_infinite_value_reaches_only_its_readers(device):
+    """One infinite value in a sealed fine: queries that did not select the
+    fine keep their outputs, those that did lose the one channel. The products
+    put sixteen queries together, and the sums of those that a product made
+    NaN are formed again: fp32 sums in another order."""
+    tokens, width, channel = 5200, 64, 7
+    xs, fa, fb = config0_inputs(1, tokens, 1, width, 41)
+    cfg = TaoConfig(coarse_index_only=True)
+    dev = [x.to(device) for x in xs]
+    with torch.no_grad():
+        want, sel = training.forward_f32(*dev, fa.to(device), fb.to(device), 0.5, cfg,
+                                         return_routes=True)
+        dev[2][0, 100, 0, channel] = float("inf")
+        got = training.forward_f32(*dev, fa.to(device), fb.to(device), 0.5, cfg)
+    got, want = got[0, 768:, 0], want[0, 768:, 0]            # past the token's local window
+    reads = (sel[0, 768:, 0] == 0).any(-1)                   # fine 0 holds the token
+    assert 0 < int(reads.sum()) < len(reads)
+    torch.testing.assert_close(got[~reads], want[~reads], **TOL32)
+    other = torch.arange(width, device=device) != channel
+    torch.testing.assert_close(got[:, other], want[:, other], **TOL32)
+    assert not torch.isfinite(got[reads, channel]).any()
