@@ -103,6 +103,7 @@ struct F32LocalSmem {
     float red[kLocalWaves][16][kLocalRows];
   };
   float wm[kLocalWaves][32], wl[kLocalWaves][32];
+  uint32_t bad;                                  // queries whose output holds a NaN
 };
 
 // Orders one wave's LDS accesses across its lanes (scratch private to a wave).
@@ -110,6 +111,36 @@ TAO_DEV void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Local attention of query t over its keys [k0, t], by one wave: lane = channel.
+template <int D>
+TAO_DEV void local_row(const F32Params& p, int k0, int t, int b, int h, int lane) {
+  constexpr int R = D / 64;
+  const float scale = 1.0f / sqrtf((float)D);
+  float q[R], acc[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    q[r] = ld(p.q, b, t, h, lane + 64 * r);
+    acc[r] = 0.0f;
+  }
+  float m = -__builtin_inff(), l = 0.0f;
+  for (int key = k0; key <= t; ++key) {
+    float dot = 0.0f;
+#pragma unroll
+    for (int r = 0; r < R; ++r) dot = fmaf(q[r], ld(p.k, b, key, h, lane + 64 * r), dot);
+    const float s = wave_fold(dot) * scale;
+    if (s == -__builtin_inff()) continue;        // weighs 0; the same in every lane
+    const float mn = fmaxf(m, s), corr = expf(m - mn), wgt = expf(s - mn);
+    l = l * corr + wgt;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+      acc[r] = fmaf(wgt, ld(p.v, b, key, h, lane + 64 * r), acc[r] * corr);
+    m = mn;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    p.local[(((size_t)b * p.T + t) * p.H + h) * D + lane + 64 * r] = acc[r] / l;
 }
 
 template <int D>
@@ -131,6 +162,7 @@ TAO_DEV void local_tile(const F32Params& p, bool vec, int t0, int b, int h, F32L
   for (int i = 0; i < D / 8; ++i) q[i] = ld4(qp + 4 * i, vec);
   f32x16 acc[CT] = {};
   float m = -__builtin_inff(), l = 0.0f;
+  if (threadIdx.x == 0) sm.bad = 0u;             // published by the merge's barriers
   // Keys past the sequence (the last block's) repeat its last row; the causal
   // mask drops them. K rows come whole (a row per 16 or 32 lanes) and turn to
   // a row per lane in LDS: read a row per lane from memory, every load touches
@@ -182,15 +214,17 @@ TAO_DEV void local_tile(const F32Params& p, bool vec, int t0, int b, int h, F32L
       s[i] = kb + acc_row(i, half) <= t ? s[i] * scale : -__builtin_inff();
       top = fmaxf(top, s[i]);
     }
-    top = fmaxf(top, __shfl_xor(top, 32));   // finite: key kb <= t0 is every query's
+    top = fmaxf(top, __shfl_xor(top, 32));
     const float mn = fmaxf(m, top);
-    const float corr = expf(m - mn);
+    // No finite score yet (every visible one -inf): they weigh 0.
+    const float at = mn > -__builtin_inff() ? mn : 0.0f;
+    const float corr = expf(m - at);
     l *= corr;
 #pragma unroll
     for (int c = 0; c < CT; ++c) acc[c] *= corr;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      s[i] = expf(s[i] - mn);
+      s[i] = expf(s[i] - at);
       l += s[i];
     }
 #pragma unroll
@@ -200,8 +234,8 @@ TAO_DEV void local_tile(const F32Params& p, bool vec, int t0, int b, int h, F32L
     m = mn;
   }
   l += __shfl_xor(l, 32);
-  // Merge the waves' partials (a wave without a block has m = -inf and weighs
-  // 0; the block of the query's own key makes M finite).
+  // Merge the waves' partials (a wave without a block or a finite score has
+  // m = -inf and weighs 0).
   if (half == 0) wm[w][col] = m;
   __syncthreads();                               // also: the K blocks are read
   float top = wm[0][col];
@@ -225,8 +259,19 @@ TAO_DEV void local_tile(const F32Params& p, bool vec, int t0, int b, int h, F32L
         sum += red[v][(ch >> 3) * 4 + (ch & 3)][qi + 32 * ((ch >> 2) & 1)];
         lsum += wl[v][qi];
       }
-      p.local[(((size_t)b * p.T + t0 + qi) * p.H + h) * D + 32 * c + ch] = sum / lsum;
+      const float o = sum / lsum;
+      p.local[(((size_t)b * p.T + t0 + qi) * p.H + h) * D + 32 * c + ch] = o;
+      if (o != o) atomicOr(&sm.bad, 1u << qi);
     }
+  }
+  __syncthreads();
+  // The products give a key that a query does not see a weight of 0, and 0
+  // times an infinite or NaN value is NaN. A NaN outlives every later sum, so
+  // the queries that hold one are computed again over their own keys alone, a
+  // wave each.
+  for (uint32_t bad = sm.bad; bad; bad &= bad - 1) {
+    const int qi = __builtin_ctz(bad);
+    if (qi % kLocalWaves == w) local_row<D>(p, k0, t0 + qi, b, h, lane);
   }
 }
 

@@ -201,3 +201,27 @@ def test_fp32_infinite_value_reaches_only_its_readers(device):
     other = torch.arange(width, device=device) != channel
     torch.testing.assert_close(got[:, other], want[:, other], **TOL32)
     assert not torch.isfinite(got[reads, channel]).any()
+
+
+@pytest.mark.parametrize("width", [64, 128])
+def test_fp32_local_attention_of_values_that_are_not_finite(device, width):
+    """Keys that score -inf alone, a whole block of 32 of them, and the first
+    key of a block of queries (the only one its first query sees there) weigh
+    nothing; an infinite value reaches no query before it."""
+    tokens, at, channel = 300, 155, 7
+    xs, fa, fb = config0_inputs(1, tokens, 1, width, 42)
+    q, k, v = xs[:3]
+    q[..., 0] = 1.0
+    for low, high in ((64, 96), (128, 129), (131, 132), (256, 257)):
+        k[0, low:high, 0, 0] = -float("inf")
+    s = q[0, :, 0].double() @ k[0, :, 0].double().T / width ** 0.5
+    s = s.masked_fill(torch.ones(tokens, tokens).triu(1).bool(), -float("inf"))
+    want = (torch.softmax(s, -1) @ v[0, :, 0].double()).float()
+    v[0, at, 0, channel] = float("inf")
+    with torch.no_grad():
+        got = training.forward_f32(*(x.to(device) for x in xs), fa.to(device), fb.to(device), 0.5,
+                                   TaoConfig()).cpu()[0, :, 0]
+    other = torch.arange(width) != channel
+    torch.testing.assert_close(got[:, other], want[:, other], **TOL32)
+    torch.testing.assert_close(got[:at, channel], want[:at, channel], **TOL32)
+    assert not torch.isfinite(got[at:, channel]).any()
