@@ -579,10 +579,14 @@ __global__ __launch_bounds__(kRefreshThreads) void refresh_fold_kernel(RoutePara
 // rows in LDS needed about 9, and a wave per query 10 and a cross-lane fold
 // per row). Masses of every visible fine are formed, also those of pages a
 // query did not choose: the lanes of a wave choose different pages.
-// A workgroup's four waves take pages p = w, w + 4, ....
-// Measured (B1 T16384 H8 D128): 463 us with a wave per query, 103 us now, of
-// which the masses' VALU is about 56; (B2 T8192 H12 D64): 116 us with a lane
-// per (query, row) pair, 59 us now.
+// A workgroup's waves share the fines evenly (with whole pages dealt to them, a
+// short sequence's one page was a chain of up to eight fines in one wave), and
+// a tile that reads every visible fine forms no mass.
+// Measured (T16384 H7 D128): 404 us with a wave per query, 83 us now;
+// (T16384 H32 D64): 403 us with a lane per (query, row) pair, 180 us now;
+// (T2105 H7 D64): 11.3 us so, 3.7 now; (T3300 H1 D64): 10.8 so, 11.3 now.
+// D = 128 is held to the 168 registers of three waves a SIMD: with 169, two a
+// SIMD, T16384 H7 takes 101 us.
 constexpr int kQThreads = 256;
 constexpr int kQWaves = kQThreads / 64;
 
@@ -634,13 +638,14 @@ TAO_DEV uint16_t mass_key(float mass) {
   return (uint16_t)(key ? key : 1u);
 }
 
-// Page and fine keys of one query per lane, pages w, w + 4, ... of the wave.
+// Keys of the fines [first, last) and of the pages that begin among them, one
+// query per lane.
 template <int D>
-TAO_DEV void lane_masses(const bf16_t* hrow, int w, bool write, bool pages, int K, int epoch,
+TAO_DEV void lane_masses(const bf16_t* hrow, int first, int last, bool write, bool pages, int K,
                          const bf16_t* pw, const SwRows& sw, uint16_t* pkey, uint16_t* fkey) {
   constexpr int G = 8, HALF = D / 2;
-  const int P = (epoch + G - 1) / G;
-  for (int p = w; p < P; p += kQWaves) {
+  for (int f = first; f < last;) {
+    const int p = f / G, end = min(last, G * p + G);
     const const_words pwr = uniform_row(pw + (size_t)p * D);
     float x[D];
 #pragma unroll
@@ -656,21 +661,20 @@ TAO_DEV void lane_masses(const bf16_t* hrow, int w, bool write, bool pages, int 
         x[HALF + c + k] = word_bf(u, 1);
       }
     }
-    if (pages && p < K) {
+    if (pages && p < K && f == G * p) {
       const float m = fold_tree<D, 0, 1>([&](int e) __attribute__((always_inline)) {
         return x[e] + x[e + HALF];
       });
       if (write) pkey[p] = mass_key(rbf(m));
     }
-    const int n = min(G, epoch - G * p);
-    for (int j = 0; j < n; ++j) {
-      const const_words s = uniform_row(sw.row(G * p + j, D));
+    const_words s = uniform_row(sw.row(f, D));       // a page's rows are consecutive
+    for (; f < end; ++f, s += D / 2) {
       const float m = fold_tree<D, 0, 1>([&](int e) __attribute__((always_inline)) {
         const uint32_t u = pack_bf16x2(x[e] * word_bf(s[e / 2], e & 1),
                                        x[e + HALF] * word_bf(s[(e + HALF) / 2], e & 1));
         return word_bf(u, 0) + word_bf(u, 1);
       });
-      if (write) fkey[G * p + j] = mass_key(rbf(m));
+      if (write) fkey[f] = mass_key(rbf(m));
     }
   }
 }
@@ -916,9 +920,9 @@ TAO_DEV void quad_open_pages(const uint16_t* pkey, uint16_t* fkey, uint32_t* ope
 // Per-query routes: a workgroup takes the queries of slots / 32 consecutive
 // read tiles of one (batch, head). Selections are bitmasks over fine ids (the
 // read needs the set, not the order).
-template <int D>
-__global__ __launch_bounds__(kQThreads, 2) void route_queries_kernel(QueryRouteParams p,
-                                                                     RouteLds lds) {
+template <int D, int W>
+__global__ __launch_bounds__(64 * W, D == 128 ? 3 : 4) void route_queries_kernel(QueryRouteParams p,
+                                                                  RouteLds lds) {
   extern __shared__ __align__(16) unsigned char route_smem[];
   constexpr int G = 8, PAD = D + 8;                // coarse_group (checked at launch)
   bf16_t* const hs = (bf16_t*)route_smem;
@@ -950,10 +954,22 @@ __global__ __launch_bounds__(kQThreads, 2) void route_queries_kernel(QueryRouteP
     const bf16_t* pw = p.pw_pool + ((size_t)erel * BH + bh) * p.pool_pcap * D;
     const SwRows sw{p.sw + (size_t)bh * p.fine_cap * D,
                     p.psw_pool + ((size_t)erel * BH + bh) * 8 * D, K * G};
+    if (M == epoch) {          // every visible fine: no mass decides (up to six fines)
+      for (int tl = a; tl < z; ++tl) {
+        const int first = (int)desc[8 * tl], nq = (int)desc[8 * tl + 1];
+        for (int i = threadIdx.x; i < nq * words; i += 64 * W) {
+          const int q = i / words, left = epoch - 32 * (i - q * words);
+          p.qsel[((size_t)(b * p.T + first + q) * p.H + h) * p.qsel_words + (i - q * words)] =
+              left >= 32 ? ~0u : (1u << left) - 1u;
+        }
+      }
+      a = z;
+      continue;
+    }
     // ---- h of each query
     for (int tl = a; tl < z; ++tl) {
       const int first = (int)desc[8 * tl], nq = (int)desc[8 * tl + 1];
-      for (int q0 = 4 * w; q0 < nq; q0 += 4 * kQWaves)
+      for (int q0 = 4 * w; q0 < nq; q0 += 4 * W)
         query_rows<D>(
             min(4, nq - q0), lane,
             [&](int i) __attribute__((always_inline)) {
@@ -966,14 +982,14 @@ __global__ __launch_bounds__(kQThreads, 2) void route_queries_kernel(QueryRouteP
     {
       const int slot = lane & (lds.slots - 1);
       const bool write = lane >= 32 * a && lane < 32 * z;
-      lane_masses<D>(hs + slot * PAD, w, write, coarse < K, K, epoch, pw, sw,
-                     pkeys + slot * lds.pkeys, fkeys + slot * lds.fkeys);
+      lane_masses<D>(hs + slot * PAD, w * epoch / W, (w + 1) * epoch / W, write, coarse < K, K,
+                     pw, sw, pkeys + slot * lds.pkeys, fkeys + slot * lds.fkeys);
     }
     __syncthreads();
     // ---- selection: four lanes a query; open pages and bitmasks where h was
     uint32_t* const bits = (uint32_t*)hs;                    // [slot][words]
     uint32_t* const opens = bits + lds.slots * words;        // [slot][4]
-    for (int i = threadIdx.x; i < lds.slots * (words + 4); i += kQThreads) bits[i] = 0u;
+    for (int i = threadIdx.x; i < lds.slots * (words + 4); i += 64 * W) bits[i] = 0u;
     __syncthreads();
     const int slot = 16 * w + (lane >> 2), tl = slot >> 5;
     if (tl >= a && tl < z && (slot & 31) < (int)desc[8 * tl + 1]) {
@@ -984,7 +1000,7 @@ __global__ __launch_bounds__(kQThreads, 2) void route_queries_kernel(QueryRouteP
       });
     }
     __syncthreads();
-    for (int i = threadIdx.x + 32 * a * words; i < 32 * z * words; i += kQThreads) {
+    for (int i = threadIdx.x + 32 * a * words; i < 32 * z * words; i += 64 * W) {
       const int s = i / words, wd = i - s * words;
       const int64_t* d = desc + 8 * (s >> 5);
       if ((s & 31) < (int)d[1])
@@ -1142,20 +1158,32 @@ hipError_t launch_route_queries(const QueryRouteParams& p, int head_dim, hipStre
   if (p.qsel_words < 1 || p.group != 8 || p.max_epoch < 1 || p.max_epoch > kQueryRouteMaxEpoch)
     return hipErrorInvalidValue;
   if (head_dim != 64 && head_dim != 128) return hipErrorInvalidValue;
-  // Two read tiles a workgroup fill a wave's lanes; one where their keys
-  // would not fit the LDS (beyond about 900 visible fines at D128).
+  // Two read tiles a workgroup fill a wave's lanes (T16384 H16 D64: 95 us, 154
+  // with one). One where the chip would not be full of them, up to four
+  // workgroups a CU (D = 128: three): half of a wave's lanes idle, but so would
+  // CUs (T3300 H7 D64: 14.5 us with two, 11.7 with one; T9008 H7: 24 with two,
+  // 32 with one). And one where the keys of two do not fit the LDS (from 1,015
+  // fines at D = 128).
+  const int64_t singles = (int64_t)p.n_tiles * p.B * p.H;
   RouteLds lds = route_lds(64, p.max_epoch);
-  if (lds.bytes(head_dim) > kLdsBytes) lds = route_lds(32, p.max_epoch);
+  if (singles <= (head_dim == 64 ? 1024 : 768) || lds.bytes(head_dim) > kLdsBytes)
+    lds = route_lds(32, p.max_epoch);
   const size_t bytes = lds.bytes(head_dim);
   const int per = lds.slots / 32;
   const dim3 grid((unsigned)((p.n_tiles + per - 1) / per * p.B * p.H));
-  const auto kernel = head_dim == 128 ? route_queries_kernel<128> : route_queries_kernel<64>;
+  // Eight waves where few workgroups route many fines: a wave's share of the
+  // fines is then a serial chain (T9008 H2 D64: 20.5 us with four, 17.5 with
+  // eight; T5000 H2: 12.4 with four, 13.0 with eight).
+  const bool wide = per == 1 && p.max_epoch >= 32 && singles <= (head_dim == 64 ? 576 : 384);
+  const auto kernel = head_dim == 128
+                          ? (wide ? route_queries_kernel<128, 8> : route_queries_kernel<128, 4>)
+                          : (wide ? route_queries_kernel<64, 8> : route_queries_kernel<64, 4>);
   if (bytes > 64 * 1024) {
     const hipError_t e = hipFuncSetAttribute(
         (const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(kernel, grid, dim3(kQThreads), bytes, s, p, lds);
+  hipLaunchKernelGGL(kernel, grid, dim3(wide ? 512 : 256), bytes, s, p, lds);
   return hipGetLastError();
 }
 

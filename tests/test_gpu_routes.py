@@ -29,7 +29,10 @@ def _tokens(tokens, heads, width, seed):
     (1057, 2, 128),        # a ragged second tile: slots of one workgroup in two epochs
     (2337, 3, 64),         # seven fines, the last read tile holds one query
     (9001, 2, 128),        # chosen pages below all pages
-    (17000, 1, 64),        # more than 64 fines: selection keys stay in LDS
+    (9001, 1, 128),        # eight waves a workgroup
+    (5003, 6, 128),        # two read tiles a workgroup
+    (9001, 5, 64),         # the same
+    (17000, 1, 64),        # more than 64 fines: selection keys stay in LDS; eight waves
     (262900, 1, 128),      # 1024 fines: one read tile per workgroup
 ])
 def test_query_routes_equal_single_turn_routes(device, tokens, heads, width):
