@@ -212,8 +212,13 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
 // unless its own query selected the fine, so a wave's 32 queries still share
 // every staged C^T and MFMA; the numerator and denominator of a query sum
 // exactly its selected fines (selected_read.py:156-173).
-template <int D, bool COARSE, bool PERQ, bool FEAT>
-__global__ __launch_bounds__(kGroupThreads, D == 64 && !FEAT ? 4 : 2) void read_groups_kernel(ReadTilesParams p) {
+//
+// PACKED (D = 64): within 128 registers, so that two workgroups share a CU. The
+// form with the coarse branch then spills 13 of them, which costs more than it
+// gives where a CU has one workgroup anyway (see launch_read_tiles).
+template <int D, bool COARSE, bool PERQ, bool FEAT, bool PACKED>
+__global__ __launch_bounds__(kGroupThreads, PACKED ? 4 : 2) void read_groups_kernel(ReadTilesParams p) {
+  static_assert(!PACKED || (D == 64 && !FEAT), "only these fit");
   static_assert(!FEAT || PERQ, "the group read's mixture serves per-query reads");
   constexpr int KK = D / 16, ET = D / 32, CPR = D / 8;   // k-steps, e-tiles, uint4 per row
   constexpr int CPT = D * CPR / kGroupThreads;           // C^T uint4 per thread
@@ -1492,10 +1497,10 @@ hipError_t launch_read_tiles(const ReadTilesParams& p, int head_dim, hipStream_t
   const bool coarse = p.coarse_pool != nullptr;
   const bool perq = p.qsel != nullptr;
   if (perq && (p.qsel_words < 1 || p.qsel_words > kBitWords)) return hipErrorInvalidValue;
-#define TAO_READ_LAUNCH(D_, C_, Q_)                                                           \
-  hipLaunchKernelGGL((read_groups_kernel<D_, C_, Q_, false>), grid, dim3(kGroupThreads), 0, s, p)
+#define TAO_READ_LAUNCH(D_, C_, P_)                                                           \
+  hipLaunchKernelGGL((read_groups_kernel<D_, C_, true, false, P_>), grid, dim3(kGroupThreads), 0, s, p)
 #define TAO_MIXTURE_LAUNCH(D_, C_)                                                            \
-  hipLaunchKernelGGL((read_groups_kernel<D_, C_, true, true>), grid, dim3(kGroupThreads), 0, s, p)
+  hipLaunchKernelGGL((read_groups_kernel<D_, C_, true, true, false>), grid, dim3(kGroupThreads), 0, s, p)
 #define TAO_STREAM_LAUNCH(D_, C_)                                                             \
   hipLaunchKernelGGL((read_stream_kernel<D_, C_, false>), sgrid, dim3(kStreamThreads), 0, s, p)
 #define TAO_FEATURE_LAUNCH(D_, C_)                                                            \
@@ -1525,13 +1530,20 @@ hipError_t launch_read_tiles(const ReadTilesParams& p, int head_dim, hipStream_t
   }
   if (head_dim == 128) {
     if (perq) {
-      if (coarse) TAO_READ_LAUNCH(128, true, true); else TAO_READ_LAUNCH(128, false, true);
+      if (coarse) TAO_READ_LAUNCH(128, true, false); else TAO_READ_LAUNCH(128, false, false);
     } else {
       if (coarse) TAO_STREAM_LAUNCH(128, true); else TAO_STREAM_LAUNCH(128, false);
     }
   } else {
     if (perq) {
-      if (coarse) TAO_READ_LAUNCH(64, true, true); else TAO_READ_LAUNCH(64, false, true);
+      // Up to five workgroups on four CUs the second place on a CU is hardly
+      // used and the spills show (T9008 H2: 61 us packed, 56 not; T5000 H16, 320
+      // workgroups: 44 and 41); beyond it the packed form wins (T3300 H32, 416:
+      // 39 and 40; T9008 H16, 576: 69 and 93). Without the coarse branch
+      // nothing spills.
+      if (!coarse) TAO_READ_LAUNCH(64, false, true);
+      else if (grid.x > 320) TAO_READ_LAUNCH(64, true, true);
+      else TAO_READ_LAUNCH(64, true, false);
     } else {
       if (coarse) TAO_STREAM_LAUNCH(64, true); else TAO_STREAM_LAUNCH(64, false);
     }

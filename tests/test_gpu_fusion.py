@@ -30,3 +30,18 @@ def test_tile_fusion_matches_oracle(device, width, scale, alpha):
         top = ref[:, lo:hi].abs().max()
         assert (out[:, lo:hi] - ref[:, lo:hi]).abs().max() < 2e-2 * top
     assert torch.isfinite(out).all()
+
+
+@pytest.mark.parametrize("index_only", [False, True])
+def test_heads_read_the_same_alone_and_among_many(device, index_only):
+    """Two heads alone (a workgroup a CU) and among 28 (two a CU, another build
+    of the read; two query tiles a routing workgroup): the same bits."""
+    g = torch.Generator(device=device).manual_seed(61)
+    tokens, heads, width = 2900, 28, 64
+    xs = [torch.randn(1, tokens, heads, width, generator=g, device=device).to(torch.bfloat16)
+          for _ in range(5)]
+    fa, fb = (torch.randn(heads, width, 3, generator=g, device=device) * 0.02 for _ in range(2))
+    cfg = TaoConfig(coarse_index_only=index_only)
+    many = training.forward(*xs, fa, fb, 0.5, cfg)
+    few = training.forward(*(x[:, :, :2].contiguous() for x in xs), fa[:2], fb[:2], 0.5, cfg)
+    assert torch.equal(many[:, :, :2], few)
