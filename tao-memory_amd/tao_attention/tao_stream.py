@@ -137,7 +137,6 @@ class _DeviceState:
         if self.association or self.feature:
             self.stats = self.stats_scratch(stats_cap)
         self.generation = next(_SERIAL)   # renewed whenever the buffers move
-        self.home = self.stream()         # the stream the buffers belong to
         self.fine_cap = 0
         self.plan_words = max(plan_words, 4096)
         self._allocate(fine_cap, copy_fines=0)
@@ -375,7 +374,8 @@ class StreamCache:
         # The regional graph serves the memo-backed index-only read only
         # (tao_stream.py:238-248). Replay mechanism: see HistoryRegionGraph.
         self._graph_mode = 0
-        self._drain = False          # a call ran on another stream than the buffers'
+        self._streams = {}           # streams that calls ran on, by handle
+        self._drain = False          # several of them, or steps in a caller's graph
         if (config.q1_history_region_graph and config.q1_page_normalization_memo
                 and config.coarse_index_only):
             replay = os.environ.get("TAO_GRAPH_REPLAY", "dispatch")
@@ -430,14 +430,17 @@ class StreamCache:
                 self._handle, _hip.GRAPH_REASONS.index(reason)))
 
     def _close_driver(self):
-        """Close the native driver. The caller's stream is drained first where
-        the driver holds captured steps or a call ran on another stream; a
-        driver without a graph holds no device memory, and the state's buffers
-        are freed in their stream's order (a server's next request is then
-        issued while the last one still runs)."""
+        """Close the native driver. A driver without a graph holds no device
+        memory and no kernel reads its host memory, and the state's buffers are
+        freed in the order of the one stream that uses them, so that a server's
+        next request is issued while the last one still runs. Where there are
+        captured steps or several streams, their work is waited for first."""
+        if self._dev is not None and (self._drain or
+                                      (self._graph_mode and self._handle is not None)):
+            current = torch.cuda.current_stream(self._dev.device)
+            for stream in {current, *self._streams.values()}:
+                stream.synchronize()
         if self._handle is not None:
-            if self._dev is not None and (self._graph_mode or self._drain):
-                torch.cuda.current_stream(self._dev.device).synchronize()
             if self.history_region is not None:
                 self.history_region._stats()         # keep the final counters
             _hip.lib().tao_stream_close(self._handle)
@@ -490,11 +493,14 @@ class StreamCache:
         return self._dev
 
     def _note_stream(self, stream):
-        """A call on another stream than the buffers' own: the caching
-        allocator orders a freed buffer's reuse after its own stream only, so
-        such a state is drained before its buffers go."""
-        if stream != self._dev.home:
-            self._drain = True
+        """A call on `stream`, the current one. The caching allocator orders a
+        freed buffer's reuse after the stream it was allocated on and no other,
+        so a state that several streams used waits for all of them before its
+        buffers go (_close_driver), whichever is current then."""
+        if stream not in self._streams:
+            self._streams[stream] = torch.cuda.current_stream(self._dev.device)
+            if len(self._streams) > 1:
+                self._drain = True
 
     # ----------------------------------------------------------------- kernels
     def _timed(self, name):
@@ -756,8 +762,8 @@ class StreamCache:
         if nat is not None and self.position < self._fast_limit and not self._handle_dirty:
             pos = self.position
             stream = _hip.raw_stream(self._stream_index)
-            if stream != self._dev.home:
-                self._drain = True
+            if stream not in self._streams:
+                self._note_stream(stream)
             try:
                 r = nat(q, k, v, raw_q, raw_k, fusion_a, fusion_b, alpha, pos, stream)
             except TypeError:
@@ -894,7 +900,7 @@ class StreamCache:
         self._check_supported(q)
         if not self._replayable_next():
             raise RuntimeError("the next token seals or changes its route; decode it eagerly")
-        self._drain = True               # the caller's graph replays on any stream
+        self._drain = True               # replays: noted by _advance_replayed
         q, k, v, raw_q, raw_k = _hip.vector_operands(q, k, v, raw_q, raw_k)
         tok = _hip.tokens(q, k, v, raw_q, raw_k)
         fu = _hip.fusion(fusion_a, fusion_b, alpha, False, True, like=q)
@@ -912,6 +918,7 @@ class StreamCache:
         device-cursor step: driver cursor (tao_stream_advance), host cursor
         and the counters a driver call would have moved (a refresh turn
         among them ran its gated refresh on the device, keeping the route)."""
+        self._note_stream(self._dev.stream())
         _hip.check(_hip.lib().tao_stream_advance(self._handle, count))
         if not self._run_open:
             self._open_run()
@@ -1305,6 +1312,7 @@ class DecodeBatch:
         self._table = None
         self._key = None
         self._gens = None
+        self._stream = None          # of the last call, noted with every state
         self._info = (ctypes.c_int64 * (4 * len(self.states)))()
 
     def close(self):
@@ -1334,11 +1342,11 @@ class DecodeBatch:
             if dev.B != 1:
                 raise ValueError("batched decode takes one-request states (batch 1)")
             st._driver(dev)
-            st._drain = True              # the batch's calls do not note their stream
+            st._drain = True              # the batch's table refers to the drivers
         key = tuple((id(st), st._handle_serial) for st in self.states)
         gens = tuple(st._dev.generation for st in self.states)
         lib = _hip.lib()
-        stream = self.states[0]._dev.stream()
+        stream = self._stream = self.states[0]._dev.stream()
         if self._handle is None or key != self._key:
             self.close()
             nbytes = lib.tao_batch_table_bytes(len(self.states))
@@ -1395,9 +1403,14 @@ class DecodeBatch:
         out = torch.empty_like(q)
         out_s = (ctypes.c_int64 * 3)(*_hip.strides_bth(out))
         info = self._info
+        stream = self.states[0]._dev.stream()
+        if stream != self._stream:
+            for st in self.states:
+                st._note_stream(stream)
+            self._stream = stream
         _hip.check(_hip.lib().tao_batch_decode(
             self._handle, ctypes.byref(tok), ctypes.byref(fu), out.data_ptr(), out_s,
-            self.states[0]._dev.stream(), info))
+            stream, info))
         for r, st in enumerate(self.states):
             if not st._run_open:
                 st._open_run()

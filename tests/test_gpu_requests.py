@@ -41,23 +41,36 @@ def test_requests_in_flight_do_not_share_memory(device, side_stream):
         assert torch.equal(out, want[i % 3])
 
 
-def test_a_state_used_on_another_stream_is_drained(device):
-    """Buffers of the default stream, a decode on a side stream: closing the
-    driver waits for the side stream before the buffers are freed."""
+@pytest.mark.parametrize("inside", [True, False])
+@pytest.mark.parametrize("steps", [1, 3])
+def test_a_state_used_on_another_stream_is_drained(device, inside, steps):
+    """Buffers of the default stream, decodes on a side stream behind work
+    that takes its time: closing the driver waits for the side stream before
+    the buffers are freed, whichever stream is current where the state goes."""
     g = torch.Generator(device=device).manual_seed(10)
     fusion = [torch.randn(2, 64, 3, generator=g, device=device) * 0.02 for _ in range(2)]
-    xs = [torch.randn(1, 801, 2, 64, generator=g, device=device).to(torch.bfloat16)
+    xs = [torch.randn(1, 800 + steps, 2, 64, generator=g, device=device).to(torch.bfloat16)
           for _ in range(5)]
     _, state = _request([x[:, :800] for x in xs], fusion, TaoConfig(), 1)
     assert not state._drain
+    big = torch.randn(8192, 8192, generator=g, device=device)
+    big @ big                                      # the library's own first call
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
-    q, k, v, rq, rk = (x[:, 800:].contiguous() for x in xs)
+    cuts = [[x[:, i:i + 1].contiguous() for x in xs] for i in range(800, 800 + steps)]
     torch.cuda.synchronize()
     with torch.cuda.stream(side):
-        _, state = tao_attention_decode(q, k, v, raw_q=rq, raw_k=rk, fusion_a=fusion[0],
-                                        fusion_b=fusion[1], alpha=0.5, state=state,
-                                        position=state.get_pos())
-        assert state._drain
+        for _ in range(20):
+            busy = big @ big
+        for q, k, v, rq, rk in cuts:
+            _, state = tao_attention_decode(q, k, v, raw_q=rq, raw_k=rk, fusion_a=fusion[0],
+                                            fusion_b=fusion[1], alpha=0.5, state=state,
+                                            position=state.get_pos())
+        assert state._drain and not side.query()
+        if inside:
+            del state
+            assert side.query()
+    if not inside:
         del state
         assert side.query()
+    del busy
