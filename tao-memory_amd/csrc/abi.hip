@@ -1628,9 +1628,8 @@ TrainBwdLayout train_bwd_layout(const tao_state_dev* st, int64_t tokens, int fin
       l.pdsq = take(pvec);
       l.pdms = take(pvec);
       const int keep = st->local_keep, ft = st->fine_tokens, np = (int)pages;
-      const size_t fparts = (size_t)fines * tao::mix_splits(fines, (int)BH, (int)T, keep + ft);
-      const size_t pparts =
-          pages * tao::mix_splits(np, (int)BH, (int)T, keep + st->coarse_group * ft);
+      const size_t fparts = tao::mix_parts(fines, (int)BH, (int)T, keep + ft);
+      const size_t pparts = tao::mix_parts(np, (int)BH, (int)T, keep + st->coarse_group * ft);
       l.mix_part = take(std::max(fparts, pparts) * BH * (mat + (size_t)D * 4));
     }
   }

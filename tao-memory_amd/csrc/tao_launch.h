@@ -570,6 +570,11 @@ inline int mix_splits(int items, int bh, int T, int first_query) {
   const int n = want < 16 ? want : 16;
   return n < 1 ? 1 : n < chunks ? n : chunks;
 }
+// Partial sums of a head's items: none where one workgroup takes an item.
+inline size_t mix_parts(int items, int bh, int T, int first_query) {
+  const int splits = mix_splits(items, bh, T, first_query);
+  return splits > 1 ? (size_t)items * splits : 0;
+}
 constexpr int kMixMaxRank = 64;      // items one query reads
 constexpr int kMixMaxItems = 512;    // fine ids a query block can select
 hipError_t launch_mix_bwd(const MixBwdParams& p, int head_dim, hipStream_t s);

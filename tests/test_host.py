@@ -97,6 +97,25 @@ def test_workspace_size_and_error_convention():
         _hip.check(rc)
 
 
+def test_backward_workspace_holds_partial_sums_only_where_items_are_split():
+    """Feature writers, index-only, 29 fines: one head's items are dealt to
+    sixteen workgroups each, 64 heads' items go whole, so their workspace is 64
+    times one head's without its partial sums (but for the 256-byte rounding of
+    each array)."""
+    def need(heads):
+        st = _hip.StateDev()
+        st.batch, st.heads, st.head_dim = 1, heads, 128
+        st.local_keep, st.fine_tokens, st.coarse_group = 512, 256, 8
+        st.fine_cap, st.page_cap, st.sel_cap, st.chosen_cap = 32, 6, 12, 6
+        st.fine_writer = 1
+        pools = _hip.PrefillPools()
+        pools.pool_pcap = 4
+        return _hip.lib().tao_train_bwd_workspace_bytes(ctypes.byref(st), 8192, 29,
+                                                        ctypes.byref(pools))
+    parts = 16 * 29 * (128 * 128 + 128) * 4
+    assert 0 <= 64 * (need(1) - parts) - need(64) < 64 * 50 * 256
+
+
 def test_prompt_attention_and_step_stamps_argument_checks():
     """tao_prompt_attention refuses a call whose window reaches before the
     call (a continuing prefill needs the state's ring), too few tile words
