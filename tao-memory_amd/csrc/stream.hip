@@ -76,10 +76,6 @@ struct Stream {
   int64_t* seal_start = nullptr;   // device int64 (first word of the plan region)
 };
 
-// The value travels with the launch: nothing of the driver is read after the
-// call, which may be its last before it is closed.
-__global__ void store_word_kernel(int64_t* dst, int64_t value) { *dst = value; }
-
 int stream_fail(int code, const char* msg) {
   tao::set_error(msg);
   return code;
@@ -162,9 +158,8 @@ int post_step(Stream* s, const tao_tokens* tok, void* stream, int* sealed) {
   const int64_t limit = c.local_keep + c.fine_tokens;
   *sealed = 0;
   if (local_len_at(c, pos) + 1 == limit) {
-    hipLaunchKernelGGL(store_word_kernel, dim3(1), dim3(1), 0, (hipStream_t)stream,
-                       s->seal_start, pos + 1 - limit);
-    hipError_t e = hipGetLastError();
+    const hipError_t e = tao::launch_store_word(s->seal_start, pos + 1 - limit,
+                                                (hipStream_t)stream);
     if (e != hipSuccess) return stream_fail((int)e, "seal start");
     int rc = tao_write_fine(&s->st, tok, pos + 1, s->seal_start, (int32_t)fines, 1, stream);
     if (!rc) rc = tao_seal_epilogue(&s->st, (int32_t)fines,

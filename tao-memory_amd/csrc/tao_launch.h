@@ -303,6 +303,7 @@ struct WriterParams {
   int z_only;                    // write fine_z only (the caller owns the C slots)
 };
 hipError_t launch_writer(const WriterParams& p, int head_dim, hipStream_t s);
+hipError_t launch_store_word(int64_t* dst, int64_t value, hipStream_t s);
 
 // fine_mass (feature writers): a page's z is r(log) of its run's fp32 mass
 // total at the page's last fine (see FeatureDescParams) instead of
