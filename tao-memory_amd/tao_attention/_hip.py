@@ -272,6 +272,13 @@ def stream_ptr(device):
     return torch.cuda.current_stream(device).cuda_stream
 
 
+def stream_of(handle, device):
+    """The stream of a raw handle (0: the default stream)."""
+    if handle == 0:
+        return torch.cuda.default_stream(device)
+    return torch.cuda.ExternalStream(handle, device=device)
+
+
 def i64x3(values):
     return _I64x3(*[int(x) for x in values])
 

@@ -374,7 +374,7 @@ class StreamCache:
         # The regional graph serves the memo-backed index-only read only
         # (tao_stream.py:238-248). Replay mechanism: see HistoryRegionGraph.
         self._graph_mode = 0
-        self._streams = {}           # streams that calls ran on, by handle
+        self._streams = set()        # streams that calls ran on (handles)
         self._drain = False          # several of them, or steps in a caller's graph
         if (config.q1_history_region_graph and config.q1_page_normalization_memo
                 and config.coarse_index_only):
@@ -437,9 +437,8 @@ class StreamCache:
         captured steps or several streams, their work is waited for first."""
         if self._dev is not None and (self._drain or
                                       (self._graph_mode and self._handle is not None)):
-            current = torch.cuda.current_stream(self._dev.device)
-            for stream in {current, *self._streams.values()}:
-                stream.synchronize()
+            for stream in self._streams | {self._dev.stream()}:
+                _hip.stream_of(stream, self._dev.device).synchronize()
         if self._handle is not None:
             if self.history_region is not None:
                 self.history_region._stats()         # keep the final counters
@@ -498,9 +497,8 @@ class StreamCache:
         so a state that several streams used waits for all of them before its
         buffers go (_close_driver), whichever is current then."""
         if stream not in self._streams:
-            self._streams[stream] = torch.cuda.current_stream(self._dev.device)
-            if len(self._streams) > 1:
-                self._drain = True
+            self._streams.add(stream)
+            self._drain = self._drain or len(self._streams) > 1
 
     # ----------------------------------------------------------------- kernels
     def _timed(self, name):
