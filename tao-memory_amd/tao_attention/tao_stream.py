@@ -1311,10 +1311,17 @@ class DecodeBatch:
         self._key = None
         self._gens = None
         self._stream = None          # of the last call, noted with every state
+        self._streams = set()        # streams that used the table (handles)
         self._info = (ctypes.c_int64 * (4 * len(self.states)))()
 
     def close(self):
+        """Close the native batch. Its device table is freed in the order of
+        the stream that it was made on, so others that used it are waited for."""
         if self._handle is not None:
+            if len(self._streams) > 1:
+                for stream in self._streams:
+                    _hip.stream_of(stream, self._table.device).synchronize()
+            self._streams.clear()
             _hip.lib().tao_batch_close(self._handle)
             self._handle = None
 
@@ -1358,6 +1365,7 @@ class DecodeBatch:
         elif gens != self._gens:
             _hip.check(lib.tao_batch_sync(self._handle, stream))
             self._gens = gens
+        self._streams.add(stream)
         # What the next steps may skip re-checking (_bound): the operands'
         # geometry, each state's driver and buffers, and the last position
         # whose token its bank holds without growing.
@@ -1406,6 +1414,7 @@ class DecodeBatch:
             for st in self.states:
                 st._note_stream(stream)
             self._stream = stream
+            self._streams.add(stream)
         _hip.check(_hip.lib().tao_batch_decode(
             self._handle, ctypes.byref(tok), ctypes.byref(fu), out.data_ptr(), out_s,
             stream, info))

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from tao_attention import (TaoConfig, new_state, tao_attention_decode, tao_attention_prefill)
+from tao_attention.tao_stream import DecodeBatch
 
 pytestmark = pytest.mark.gpu
 
@@ -72,5 +73,38 @@ def test_a_state_used_on_another_stream_is_drained(device, inside, steps):
             assert side.query()
     if not inside:
         del state
+        assert side.query()
+    del busy
+
+
+@pytest.mark.parametrize("states_first", [True, False])
+def test_a_batch_used_on_another_stream_is_drained(device, states_first):
+    """A batch opened on the default stream and stepped on a side stream: its
+    table and its states' buffers go after the side stream's work."""
+    g = torch.Generator(device=device).manual_seed(11)
+    fusion = [torch.randn(2, 64, 3, generator=g, device=device) * 0.02 for _ in range(2)]
+    xs = [torch.randn(2, 802, 2, 64, generator=g, device=device).to(torch.bfloat16)
+          for _ in range(5)]
+    states = [_request([x[r:r + 1, :800].contiguous() for x in xs], fusion, TaoConfig(), 1)[1]
+              for r in range(2)]
+    batch = DecodeBatch(states)
+    first, second = ([x[:, i:i + 1].contiguous() for x in xs] for i in (800, 801))
+    batch.decode(*first, *fusion, 0.5)
+    big = torch.randn(8192, 8192, generator=g, device=device)
+    big @ big                                      # the library's own first call
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        for _ in range(20):
+            busy = big @ big
+        batch.decode(*second, *fusion, 0.5)
+        assert not side.query()
+    if states_first:
+        batch.states = []
+        del states                                 # each waits for the side stream
+        assert side.query()
+    else:
+        batch.close()                              # the table's own wait
         assert side.query()
     del busy
