@@ -437,8 +437,7 @@ class StreamCache:
         captured steps or several streams, their work is waited for first."""
         if self._dev is not None and (self._drain or
                                       (self._graph_mode and self._handle is not None)):
-            for stream in self._streams | {self._dev.stream()}:
-                _hip.stream_of(stream, self._dev.device).synchronize()
+            self._wait_streams()
         if self._handle is not None:
             if self.history_region is not None:
                 self.history_region._stats()         # keep the final counters
@@ -485,11 +484,20 @@ class StreamCache:
             self._dev = _DeviceState(self.config, b, h, d, q.device, cap, plan_words)
         elif not self._dev.matches(b, h, d, q.device):
             raise ValueError("batch/heads/width/device must stay fixed for a state")
-        elif self._dev.reserve(fines, schedule.fines_at(self.position, self.config)):
+        self._note_stream(self._dev.stream())
+        if fines > self._dev.fine_cap:
+            self._grow(self._dev.reserve, fines, schedule.fines_at(self.position, self.config))
+        return self._dev
+
+    def _grow(self, grow, *args):
+        """Let the device state grow by `grow`; the buffers that it replaces go
+        as a state's do (_note_stream)."""
+        old = dict(vars(self._dev)) if self._drain else None
+        if grow(*args):
+            if old is not None:
+                self._wait_streams()
             self._release_graph("capacity")
             self._handle_dirty = True
-        self._note_stream(self._dev.stream())
-        return self._dev
 
     def _note_stream(self, stream):
         """A call on `stream`, the current one. The caching allocator orders a
@@ -499,6 +507,10 @@ class StreamCache:
         if stream not in self._streams:
             self._streams.add(stream)
             self._drain = self._drain or len(self._streams) > 1
+
+    def _wait_streams(self):
+        for stream in self._streams | {self._dev.stream()}:
+            _hip.stream_of(stream, self._dev.device).synchronize()
 
     # ----------------------------------------------------------------- kernels
     def _timed(self, name):
@@ -568,9 +580,8 @@ class StreamCache:
     def _run_plan(self, dev, tok, fu, plan, info, local, out):
         plan_np = np.asarray(plan, dtype=np.int64)
         plan_arr = plan_np.ctypes.data_as(ctypes.POINTER(ctypes.c_int64))
-        if dev.ensure_plan(len(plan)):
-            self._release_graph("capacity")
-            self._handle_dirty = True
+        if len(plan) > dev.plan_words:
+            self._grow(dev.ensure_plan, len(plan))
         pools = _hip.PrefillPools()
         keep = []
         if info["epochs"] or info["turns"]:

@@ -108,3 +108,36 @@ def test_a_batch_used_on_another_stream_is_drained(device, states_first):
         batch.close()                              # the table's own wait
         assert side.query()
     del busy
+
+
+def test_growth_on_another_stream_waits_for_the_old_buffers(device):
+    """A prompt chunk on a side stream that outgrows a state's bank: the old
+    buffers are the default stream's, and are still read behind work that takes
+    its time. The outputs are those of one stream."""
+    g = torch.Generator(device=device).manual_seed(12)
+    fusion = [torch.randn(2, 64, 3, generator=g, device=device) * 0.02 for _ in range(2)]
+    xs = [torch.randn(1, 6000, 2, 64, generator=g, device=device).to(torch.bfloat16)
+          for _ in range(5)]
+    named = dict(fusion_a=fusion[0], fusion_b=fusion[1], alpha=0.5)
+    big = torch.randn(8192, 8192, generator=g, device=device)
+    big @ big                                      # the library's own first call
+    outs = []
+    for stream in (torch.cuda.current_stream(), torch.cuda.Stream()):
+        state = new_state(0, TaoConfig())
+        for lo, hi, at in ((0, 1500, torch.cuda.current_stream()), (1500, 6000, stream)):
+            q, k, v, rq, rk = (x[:, lo:hi].contiguous() for x in xs)
+            torch.cuda.synchronize()
+            with torch.cuda.stream(at):
+                if lo:
+                    for _ in range(20):
+                        busy = big @ big
+                before = torch.cuda.Event()
+                before.record()
+                out, state = tao_attention_prefill(q, k, v, raw_q=rq, raw_k=rk, state=state,
+                                                   position=state.get_pos(), **named)
+        if state._drain:
+            assert before.query()
+        torch.cuda.synchronize()
+        outs.append(out)
+    assert state._drain and torch.equal(*outs)
+    del busy
