@@ -5,11 +5,9 @@
 // state left by the previous chunk's seal (tao_stream.py:919-969); here every
 // seal epoch's page weights and pending segment weights are materialised in
 // pools at once (pages_kernel + epochs_kernel), routes for all refresh turns
-// run in one launch (route.hip, turn mode), and read_tiles_kernel performs
-// the selected read + fusion of all queries.
-//
-// read_groups_kernel: the selected read + fusion of every query, one
-// workgroup per 8 read tiles (route turns) of one head; see the kernel.
+// run in one launch (route.hip, turn mode), and read_stream_kernel performs
+// the selected read + fusion of all queries. The full-sequence read, whose
+// queries all route themselves, takes read_groups_kernel.
 #include "tao_launch.h"
 #include "tao_common.h"
 #include "tao_fusion.h"
@@ -134,13 +132,12 @@ struct GroupSmem {
     struct {
       uint32_t bits[kBitWords];
       int pre[kBitWords];
-      uint32_t wbits[kGroupWaves][kBitWords];   // PERQ: OR of each wave's bitmasks
+      uint32_t wbits[kGroupWaves][kBitWords];   // OR of each wave's bitmasks
     } setup;
     bf16_t c[2][D][D + 8];        // staged weighted C^T, rows padded by 16 bytes
   } u;
   bf16_t wr[2][D];                     // per buffer: the staged fine's weights r(pw * sw)
   float ez[2][D];                      // feature writers: exp(z) of the staged fine
-  int ids[kGroupWaves][kMaxM];
   int uni[kMaxUnion];
   uint32_t mask[kMaxUnion / 4];        // byte u: bit w set if wave w selected uni[u]
   int n_union;
@@ -185,9 +182,10 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
                        const bf16_t* tile_c, int lane, int b, int h, int q_first, int nq,
                        bool coarse_on);
 
-// Turn-group read: one 512-thread workgroup per (8 consecutive read tiles,
-// batch, head); wave w owns tile w (<= 32 queries sharing one route, its
-// own seal epoch and segment-weight source). The read of a fine is linear in
+// Per-query read (the full-sequence read, every query routed by itself; turn
+// routes take read_stream_kernel): one 512-thread workgroup per (8 consecutive
+// read tiles, batch, head); wave w owns tile w (<= 32 queries of one seal
+// epoch and segment-weight source). The read of a fine is linear in
 // its channel weights, num[q][e] = sum_d h_q[d] w[d] C^T[e][d] with
 // w = r(pw[page] * sw[fine]) shared by every tile of one seal epoch, so the
 // workgroup stages each fine's C^T already weighted (r(C^T * w), padded LDS,
@@ -203,23 +201,23 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
 // fp32 sums (selected_read.py:31, 48); here the product of the two weights
 // is rounded and folded into C, which moves the read within its bf16
 // tolerance. With the coarse value branch (COARSE), each e-tile of a tile
-// whose chunk has completed pages also runs 8 MFMAs of the wave's h against
+// whose chunk has completed pages also runs D / 16 MFMAs of the wave's h against
 // the folded coarse matrix of its page count (coarse.hip) before the fusion.
 //
-// PERQ (the full-sequence read, every query routed by itself): selections
-// are per-query bitmasks (route_queries_kernel). The union and the per-wave
-// masks come from the OR of the wave's bitmasks, and each A row is zeroed
-// unless its own query selected the fine, so a wave's 32 queries still share
-// every staged C^T and MFMA; the numerator and denominator of a query sum
+// Selections are per-query bitmasks (route_queries_kernel). The union and the
+// per-wave masks come from the OR of the wave's bitmasks, and each A row is
+// zeroed unless its own query selected the fine, so a wave's 32 queries still
+// share every staged C^T and MFMA; the numerator and denominator of a query sum
 // exactly its selected fines (selected_read.py:156-173).
 //
+// At D = 128 a CU holds one workgroup (about 230 registers; with the coarse branch
+// the epilogue's two tiles a wave make 138 KB of LDS).
 // PACKED (D = 64): within 128 registers, so that two workgroups share a CU. The
 // form with the coarse branch then spills 13 of them, which costs more than it
 // gives where a CU has one workgroup anyway (see launch_read_tiles).
-template <int D, bool COARSE, bool PERQ, bool FEAT, bool PACKED>
+template <int D, bool COARSE, bool FEAT, bool PACKED>
 __global__ __launch_bounds__(kGroupThreads, PACKED ? 4 : 2) void read_groups_kernel(ReadTilesParams p) {
   static_assert(!PACKED || (D == 64 && !FEAT), "only these fit");
-  static_assert(!FEAT || PERQ, "the group read's mixture serves per-query reads");
   constexpr int KK = D / 16, ET = D / 32, CPR = D / 8;   // k-steps, e-tiles, uint4 per row
   constexpr int CPT = D * CPR / kGroupThreads;           // C^T uint4 per thread
   static_assert(CPT == 1 || CPT == 4, "head width 64 or 128");
@@ -238,10 +236,10 @@ __global__ __launch_bounds__(kGroupThreads, PACKED ? 4 : 2) void read_groups_ker
   const int cc = tid % CPR;                              // this thread's column slice
 
   // This wave's tile.
-  int q_first = 0, nq = 0, slot = 0, M = 0, erel = 0, fine_on = 0, cpages = 0;
+  int q_first = 0, nq = 0, erel = 0, fine_on = 0, cpages = 0;
   if (w < nt) {
     const int64_t* desc = p.tiles + 8 * (t0 + w);
-    q_first = (int)desc[0]; nq = (int)desc[1]; slot = (int)desc[2]; M = (int)desc[3];
+    q_first = (int)desc[0]; nq = (int)desc[1];
     erel = (int)desc[4]; fine_on = (int)desc[6];
     cpages = (int)desc[7];
   }
@@ -293,12 +291,10 @@ __global__ __launch_bounds__(kGroupThreads, PACKED ? 4 : 2) void read_groups_ker
       hA[kk] = make_uint4(wv[0], wv[1], wv[2], wv[3]);
     }
   }
-  // PERQ: this lane's query bitmask (rows li >= nq select nothing).
+  // This lane's query bitmask (rows li >= nq select nothing).
   const uint32_t* qbits = nullptr;
-  if constexpr (PERQ) {
-    if (reads)
-      qbits = p.qsel + ((size_t)(b * p.T + q_first + min(li, nq - 1)) * p.H + h) * p.qsel_words;
-  }
+  if (reads)
+    qbits = p.qsel + ((size_t)(b * p.T + q_first + min(li, nq - 1)) * p.H + h) * p.qsel_words;
 
   // Feature writers: the query's mixture normaliser, the sum over its
   // selected fines (ascending id) of mass = sum_d h[d] exp(z[d]) in fp32,
@@ -367,31 +363,19 @@ __global__ __launch_bounds__(kGroupThreads, PACKED ? 4 : 2) void read_groups_ker
     // ---- union of the pass's selected sets (ascending fine id), per-wave masks
     for (int i = tid; i < kBitWords; i += kGroupThreads) sm.u.setup.bits[i] = 0;
     for (int i = tid; i < kMaxUnion / 4; i += kGroupThreads) sm.mask[i] = 0;
-    if constexpr (PERQ) {
-      for (int i = tid; i < kGroupWaves * kBitWords; i += kGroupThreads)
-        (&sm.u.setup.wbits[0][0])[i] = 0u;
-    } else if (in_pass) {
-      const int32_t* sel = p.sel_pool + ((size_t)slot * BH + bh) * p.sel_cap;
-      for (int m = lane; m < M; m += 64) sm.ids[w][m] = sel[m];
-    }
+    for (int i = tid; i < kGroupWaves * kBitWords; i += kGroupThreads)
+      (&sm.u.setup.wbits[0][0])[i] = 0u;
     __syncthreads();
-    if constexpr (PERQ) {
-      if (in_pass) {
-        const int words = (pass_epoch + 31) >> 5;
-        for (int i = 0; i < words; ++i) {
-          uint32_t v = (lane < 32 && li < nq) ? qbits[i] : 0u;
+    if (in_pass) {
+      const int words = (pass_epoch + 31) >> 5;
+      for (int i = 0; i < words; ++i) {
+        uint32_t v = (lane < 32 && li < nq) ? qbits[i] : 0u;
 #pragma unroll
-          for (int off = 1; off < 64; off <<= 1) v |= __shfl_xor(v, off, 64);
-          if (lane == 0) {
-            sm.u.setup.wbits[w][i] = v;
-            atomicOr(&sm.u.setup.bits[i], v);
-          }
+        for (int off = 1; off < 64; off <<= 1) v |= __shfl_xor(v, off, 64);
+        if (lane == 0) {
+          sm.u.setup.wbits[w][i] = v;
+          atomicOr(&sm.u.setup.bits[i], v);
         }
-      }
-    } else if (in_pass) {
-      for (int m = lane; m < M; m += 64) {
-        const int id = sm.ids[w][m];
-        atomicOr(&sm.u.setup.bits[id >> 5], 1u << (id & 31));
       }
     }
     __syncthreads();
@@ -421,24 +405,15 @@ __global__ __launch_bounds__(kGroupThreads, PACKED ? 4 : 2) void read_groups_ker
       while (bits) {
         const int bit = __ffs(bits) - 1;
         sm.uni[r] = i * 32 + bit;
-        if constexpr (PERQ) {
-          uint32_t byte = 0;
+        uint32_t byte = 0;
 #pragma unroll
-          for (int v = 0; v < kGroupWaves; ++v)
-            byte |= ((sm.u.setup.wbits[v][i] >> bit) & 1u) << v;
-          atomicOr(&sm.mask[r >> 2], byte << ((r & 3) * 8));
-        }
+        for (int v = 0; v < kGroupWaves; ++v)
+          byte |= ((sm.u.setup.wbits[v][i] >> bit) & 1u) << v;
+        atomicOr(&sm.mask[r >> 2], byte << ((r & 3) * 8));
         ++r;
         bits &= bits - 1;
       }
     }
-    if (!PERQ && in_pass)
-      for (int m = lane; m < M; m += 64) {
-        const int id = sm.ids[w][m];
-        const uint32_t word = sm.u.setup.bits[id >> 5];
-        const int rank = sm.u.setup.pre[id >> 5] + __popc(word & ((1u << (id & 31)) - 1u));
-        atomicOr(&sm.mask[rank >> 2], 1u << ((rank & 3) * 8 + w));
-      }
     __syncthreads();
     const int U = sm.n_union;
 
@@ -496,21 +471,18 @@ __global__ __launch_bounds__(kGroupThreads, PACKED ? 4 : 2) void read_groups_ker
     }                                                                    \
   } while (0)
 
-    // PERQ: the lane's bitmask word of the current fine (ids ascend).
+    // The lane's bitmask word of the current fine (ids ascend).
     int qword_at = -1;
     uint32_t qword = 0u;
     auto consume = [&](int u) __attribute__((always_inline)) {
       if (!active(u)) return;
       const int buf = u & 1;
-      uint32_t keep = 0xFFFFFFFFu;
-      if constexpr (PERQ) {
-        const int id = sm.uni[u];
-        if ((id >> 5) != qword_at) {
-          qword_at = id >> 5;
-          qword = li < nq ? qbits[qword_at] : 0u;
-        }
-        keep = ((qword >> (id & 31)) & 1u) ? 0xFFFFFFFFu : 0u;
+      const int id = sm.uni[u];
+      if ((id >> 5) != qword_at) {
+        qword_at = id >> 5;
+        qword = li < nq ? qbits[qword_at] : 0u;
       }
+      const uint32_t keep = ((qword >> (id & 31)) & 1u) ? 0xFFFFFFFFu : 0u;
       if constexpr (FEAT) {
         // coef = r(mix * h) with mix = mass / tot of this fine, rows of
         // queries that did not select it zero; no denominator.
@@ -545,7 +517,7 @@ __global__ __launch_bounds__(kGroupThreads, PACKED ? 4 : 2) void read_groups_ker
       for (int kk = 0; kk < KK; ++kk) {
         const int d0 = 16 * kk + 8 * hl;
         uint4 av = hA[kk];
-        if constexpr (PERQ) { av.x &= keep; av.y &= keep; av.z &= keep; av.w &= keep; }
+        av.x &= keep; av.y &= keep; av.z &= keep; av.w &= keep;
         const bf16x8 a = as_bf16x8(av);
 #pragma unroll
         for (int t = 0; t < ET; ++t) {
@@ -822,8 +794,9 @@ TAO_DEV void fuse_rows(const ReadTilesParams& p, const float (*fpar)[D * 3], con
 // workgroup, all of it in the same phase: 672 us at 16K (H32 D128), 588 now
 // (604 before the fusion's shorter arithmetic), of which about 145 are set-up,
 // softmax and fusion and about 210 the waits for a fine's rows, which one slot
-// ahead does not cover. Giving each XCD one or two heads at a time (their fines
-// then fit its L2) measured the same.
+// ahead does not cover. Giving each XCD one head at a time (its fines then fit
+// the L2) is within 1.5 % either way (16K: 988 us a request so, 980 as it is;
+// 7000 tokens in chunks, H8: 591 and 598).
 constexpr int kStreamWaves = 4;
 constexpr int kStreamThreads = 64 * kStreamWaves;
 constexpr int kStreamUnion = kStreamWaves * kMaxM;
@@ -1498,9 +1471,9 @@ hipError_t launch_read_tiles(const ReadTilesParams& p, int head_dim, hipStream_t
   const bool perq = p.qsel != nullptr;
   if (perq && (p.qsel_words < 1 || p.qsel_words > kBitWords)) return hipErrorInvalidValue;
 #define TAO_READ_LAUNCH(D_, C_, P_)                                                           \
-  hipLaunchKernelGGL((read_groups_kernel<D_, C_, true, false, P_>), grid, dim3(kGroupThreads), 0, s, p)
+  hipLaunchKernelGGL((read_groups_kernel<D_, C_, false, P_>), grid, dim3(kGroupThreads), 0, s, p)
 #define TAO_MIXTURE_LAUNCH(D_, C_)                                                            \
-  hipLaunchKernelGGL((read_groups_kernel<D_, C_, true, true, false>), grid, dim3(kGroupThreads), 0, s, p)
+  hipLaunchKernelGGL((read_groups_kernel<D_, C_, true, false>), grid, dim3(kGroupThreads), 0, s, p)
 #define TAO_STREAM_LAUNCH(D_, C_)                                                             \
   hipLaunchKernelGGL((read_stream_kernel<D_, C_, false>), sgrid, dim3(kStreamThreads), 0, s, p)
 #define TAO_FEATURE_LAUNCH(D_, C_)                                                            \
