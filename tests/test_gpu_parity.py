@@ -644,9 +644,9 @@ def test_full_sequence_read_short_and_training_shape():
     torch.testing.assert_close(out[:1, :768, :2].cpu().float(), first.float(), **TOL)
 
 
-def test_full_sequence_read_long_sequence_route_fallback():
-    """T16484 at D128: the tile rows exceed the LDS rows of the lane-per-pair
-    route, so the wave-per-query route runs. The read is causal, so the first
+def test_full_sequence_read_long_sequence():
+    """T16484 at D128: up to 62 visible fines, chosen pages below all pages, two
+    read tiles a routing workgroup. The read is causal, so the first
     2900 positions and the routes of tiles 3..11 must equal the oracle run on
     that prefix alone; every later query selects exactly M fines."""
     from tao_attention import TaoConfig, training
